@@ -17,6 +17,7 @@
 
 #include "eqd_internal.h"
 #include "eqd_precompute.h"
+#include "eqd_readback.h"
 
 using namespace eqd;
 
@@ -112,14 +113,6 @@ static inline uint16_t bf16_bits(float x)
     memcpy(&u, &x, 4);
     return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
 }
-static inline float bf16_value(uint16_t h)
-{
-    const uint32_t u = (uint32_t)h << 16;
-    float x;
-    memcpy(&x, &u, 4);
-    return x;
-}
-
 // comdampv, src/comdampv.f90:1-120 (region 14 compares y with xmax0 as the
 // reference does).  Returns d_x, d_y, d_z.
 static void pml_node_damping(const eqd_scalars &s, double x2, double y, double z, double d[3])
@@ -545,6 +538,7 @@ int eqd_create(const eqd_scalars *s, eqd_handle **out)
     if (s->precision != EQD_PREC_FP64 && s->precision != EQD_PREC_FP32) return EQD_EINVAL;
     eqd_handle *h = new eqd_handle();
     h->s = *s;
+    stage_retain();
     *out = h;
     return EQD_OK;
 }
@@ -1279,41 +1273,32 @@ extern "C" int eqd_wait(eqd_handle *h)
     return settle(h);
 }
 
+// a device array into host memory at dst, or into v
+static int d2h_to(eqd_handle *h, void *dst, const void *d, size_t bytes)
+{
+    HIPCHK(h, stage_copy(dst, d, bytes, h->stream));
+    return EQD_OK;
+}
+
 template <typename T>
 static int d2h(eqd_handle *h, std::vector<T> &v, const T *d, int64_t count)
 {
     v.resize(count);
-    if (count > 0) HIPCHK(h, hipMemcpy(v.data(), d, sizeof(T) * count, hipMemcpyDeviceToHost));
-    return 0;
+    return d2h_to(h, v.data(), d, sizeof(T) * count);
 }
 
-// Velocities (vel) or displacements of every node in blocked layout
-// (blk_at<3>) at the precision the device keeps: the FP64 arrays, or in the
-// FP32 bulk mode the FP32 values (displacement hi + lo) with the split nodes'
-// FP64 state from the fault's arrays.
-static int node_state(eqd_handle *h, bool vel, std::vector<double> &out)
+// Velocities (vel) or displacements of every node in the reference's layout
+// at the precision the device keeps: the FP64 arrays, or in the FP32 bulk mode
+// the FP32 values (displacement hi + lo) with the split nodes' FP64 state from
+// the fault's arrays.
+static int node_state(eqd_handle *h, bool vel, double *out)
 {
-    const int64_t nn = h->s.nn;
-    int rc;
-    if (!h->N.vel32) return d2h(h, out, vel ? h->N.vel : h->N.disp, blocked_count(nn, 3));
-    std::vector<float> a;
-    std::vector<uint16_t> b;
-    if ((rc = d2h(h, a, vel ? h->N.vel32 : h->N.dhi, blocked_count(nn, 3)))) return rc;
-    out.assign(a.begin(), a.end());
-    if (!vel) {
-        if ((rc = d2h(h, b, h->N.dlo, blocked_count(nn, 3)))) return rc;
-        for (size_t j = 0; j < out.size(); j++) out[j] = (double)a[j] + (double)bf16_value(b[j]);
-    }
-    const int64_t nf = h->F.nf, ld = h->F.ld;
-    if (nf > 0) {
-        std::vector<double> st;
-        if ((rc = d2h(h, st, vel ? h->F.sv : h->F.su, 6 * ld))) return rc;
-        const int32_t *nsmp = I32(h, EQD_NSMP);
-        for (int64_t i = 0; i < nf; i++)
-            for (int side = 0; side < 2; side++)
-                for (int k = 0; k < 3; k++)
-                    out[blocked_index(nsmp[i * 2 + side] - 1, k, 3)] = st[(side * 3 + k) * ld + i];
-    }
+    constexpr size_t row = 3 * sizeof(double);
+    HIPCHK(h, stage_out(out, row * (size_t)h->s.nn, row, h->stream,
+                        [h, vel](void *slot, size_t first, size_t count, hipStream_t s) {
+                            return launch_pack_nodes(h->N, h->F, vel, (int64_t)(first / row), (int64_t)(count / row),
+                                                     (double *)slot, s);
+                        }));
     return EQD_OK;
 }
 
@@ -1335,20 +1320,16 @@ int eqd_get(eqd_handle *h, int32_t field, void *host, int64_t count)
     int rc;
     switch (field) {
     case EQD_VELARR:
-    case EQD_DISPARR: {
-        std::vector<double> v;
-        if ((rc = node_state(h, field == EQD_VELARR, v))) return rc;
-        for (int64_t n = 0; n < nn; n++)
-            for (int k = 0; k < 3; k++) out[n * 3 + k] = v[blocked_index(n, k, 3)];
-        return EQD_OK;
-    }
+    case EQD_DISPARR:
+        return node_state(h, field == EQD_VELARR, out);
     case EQD_V1:
     case EQD_NODALFORCEARR: {
         // v1 of 3-component nodes is velArr; of PML nodes the 12 split velocities
         const bool isv = field == EQD_V1;
         std::vector<double> v, p;
         if (isv) {
-            if ((rc = node_state(h, true, v))) return rc;
+            v.resize(3 * nn);
+            if ((rc = node_state(h, true, v.data()))) return rc;
         } else if ((rc = d2h(h, v, h->N.acc, blocked_count(nn, 3)))) {
             return rc;
         }
@@ -1363,7 +1344,7 @@ int eqd_get(eqd_handle *h, int32_t field, void *host, int64_t count)
         for (int64_t i = 0; i < s.neq; i++) out[i] = orig.empty() ? 0.0 : orig[i];
         const int32_t *eqi = I32(h, EQD_EQNUMINDEXARR), *esl = I32(h, EQD_EQNUMSTARTINDEXLOC);
         for (int32_t n : h->node3_all)
-            for (int k = 0; k < 3; k++) out[eqi[esl[n] + k] - 1] = v[blocked_index(n, k, 3)];
+            for (int k = 0; k < 3; k++) out[eqi[esl[n] + k] - 1] = isv ? v[n * 3 + k] : v[blocked_index(n, k, 3)];
         const int64_t np = h->PN.n;
         for (int64_t q = 0; q < np; q++) {
             const int32_t n = h->pml_node_ids[q];
@@ -1372,25 +1353,20 @@ int eqd_get(eqd_handle *h, int32_t field, void *host, int64_t count)
         return EQD_OK;
     }
     case EQD_FRIC: {
-        std::vector<double> v;
-        const int64_t ld = h->F.ld;
-        if ((rc = d2h(h, v, h->F.fric, 100 * ld))) return rc;
-        for (int64_t i = 0; i < nf; i++)
-            for (int k = 0; k < 100; k++) out[i * 100 + k] = v[k * ld + i];
+        constexpr size_t row = 100 * sizeof(double);
+        HIPCHK(h, stage_out(out, row * (size_t)nf, row, h->stream,
+                            [h](void *slot, size_t first, size_t cnt, hipStream_t st) {
+                                return launch_pack_fric(h->F, (int64_t)(first / row), (int64_t)(cnt / row),
+                                                        (double *)slot, st);
+                            }));
         return EQD_OK;
     }
-    case EQD_FNFT: {
-        if (nf > 0) HIPCHK(h, hipMemcpy(out, h->F.fnft, sizeof(double) * nf, hipMemcpyDeviceToHost));
-        return EQD_OK;
-    }
-    case EQD_ONFAULTHIST: {
-        if (count > 0) HIPCHK(h, hipMemcpy(out, h->F.hist, sizeof(double) * count, hipMemcpyDeviceToHost));
-        return EQD_OK;
-    }
-    case EQD_OFFFAULTHIST: {
-        if (count > 0) HIPCHK(h, hipMemcpy(out, h->S.hist, sizeof(double) * count, hipMemcpyDeviceToHost));
-        return EQD_OK;
-    }
+    case EQD_FNFT:
+        return d2h_to(h, out, h->F.fnft, sizeof(double) * nf);
+    case EQD_ONFAULTHIST:
+        return d2h_to(h, out, h->F.hist, sizeof(double) * count);
+    case EQD_OFFFAULTHIST:
+        return d2h_to(h, out, h->S.hist, sizeof(double) * count);
     case EQD_STRESSARR: {
         const auto &orig = h->fd[EQD_STRESSARR];
         for (int64_t i = 0; i < s.size_stress; i++) out[i] = orig[i];
@@ -1765,6 +1741,7 @@ int eqd_destroy(eqd_handle *h)
     if (h->harvest) (void)hipFree(h->harvest);
     free_records(h);
     delete h;
+    stage_release();
     return EQD_OK;
 }
 

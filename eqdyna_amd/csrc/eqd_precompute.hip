@@ -17,6 +17,7 @@
 
 #include "../../include/eqdyna_amd.h"
 #include "eqd_precompute.h"
+#include "eqd_readback.h"
 
 namespace eqd {
 namespace {
@@ -160,6 +161,10 @@ extern "C" int eqd_precompute(const eqd_precompute_args *A, int32_t *bad_elem, d
             if (A->eqNumIndexArr[b + j] > neq) return EQD_EINVAL;
     }
     PCHK(hipSetDevice(A->device));
+    struct StageUser {
+        StageUser() { stage_retain(); }
+        ~StageUser() { stage_release(); }
+    } user;
     hipStream_t st;
     PCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     struct StreamGuard {
@@ -239,14 +244,13 @@ extern "C" int eqd_precompute(const eqd_precompute_args *A, int32_t *bad_elem, d
     node_mass_kernel<<<gn, 256, 0, st>>>(rowptr, ent, em, ndof, esl, eqi, nn, nm, fn);
     PCHK(hipGetLastError());
     PCHK(hipEventRecord(ev1, st));
-    auto d2h = [&](void *h, const void *d, size_t b) { return hipMemcpyAsync(h, d, b, hipMemcpyDeviceToHost, st); };
-    PCHK(d2h(A->eleshp, shp, sizeof(double) * 24 * ne));
-    PCHK(d2h(A->eledet, det, sizeof(double) * ne));
-    PCHK(d2h(A->elemass, em, sizeof(double) * 24 * ne));
-    PCHK(d2h(A->ss, ss, sizeof(double) * 6 * ne));
-    PCHK(d2h(A->phi, phi, sizeof(double) * 32 * ne));
-    PCHK(d2h(A->nodalMassArr, nm, sizeof(double) * neq));
-    PCHK(d2h(A->fnms, fn, sizeof(double) * nn));
+    PCHK(stage_copy(A->eleshp, shp, sizeof(double) * 24 * ne, st));
+    PCHK(stage_copy(A->eledet, det, sizeof(double) * ne, st));
+    PCHK(stage_copy(A->elemass, em, sizeof(double) * 24 * ne, st));
+    PCHK(stage_copy(A->ss, ss, sizeof(double) * 6 * ne, st));
+    PCHK(stage_copy(A->phi, phi, sizeof(double) * 32 * ne, st));
+    PCHK(stage_copy(A->nodalMassArr, nm, sizeof(double) * neq, st));
+    PCHK(stage_copy(A->fnms, fn, sizeof(double) * nn, st));
     PCHK(hipStreamSynchronize(st));
     if (device_ms) {
         float ms = 0.0f;

@@ -232,7 +232,7 @@ class Solver:
 
     def get(self, name: str) -> np.ndarray:
         fid, dt = FIELDS[name]
-        out = np.zeros(self._count(name), dtype="<" + dt)
+        out = np.empty(self._count(name), dtype="<" + dt)  # eqd_get writes every value
         self._check(self.L.eqd_get(self.h, fid, out.ctypes.data, out.size))
         return out
 
@@ -510,8 +510,9 @@ def precompute(bundle: Dict[str, np.ndarray], device: int = 0):
     eqi = np.ascontiguousarray(bundle["eqNumIndexArr"], dtype="<i4")
     nn, ne = ndof.size, et.size
     neq = int(np.asarray(bundle["nodalMassArr"]).size)
-    out = {"eleshp": np.zeros(24 * ne), "eledet": np.zeros(ne), "elemass": np.zeros(24 * ne), "ss": np.zeros(6 * ne),
-           "phi": np.zeros(32 * ne), "nodalMassArr": np.zeros(neq), "fnms": np.zeros(nn)}
+    # the element arrays are written in full, the nodal ones start from zero
+    out = {"eleshp": np.empty(24 * ne), "eledet": np.empty(ne), "elemass": np.empty(24 * ne), "ss": np.empty(6 * ne),
+           "phi": np.empty(32 * ne), "nodalMassArr": np.zeros(neq), "fnms": np.zeros(nn)}
     a = PrecomputeArgs(nn, ne, neq, eqi.size, coor.ctypes.data, ien.ctypes.data, et.ctypes.data, mat.ctypes.data,
                        ndof.ctypes.data, esl.ctypes.data, eqi.ctypes.data, out["eleshp"].ctypes.data,
                        out["eledet"].ctypes.data, out["elemass"].ctypes.data, out["ss"].ctypes.data,
