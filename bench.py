@@ -156,7 +156,7 @@ def kernel_bytes(bundle, sc, layout: dict, precision: str) -> dict:
     the full or the compact hourglass operators; or the geometry rows the
     FP32 mode rebuilds them from), connectivity, stresses and forces once per
     element, each node's state once per kernel that touches it, each
-    element-to-node force once.  Counts come from the mesh itself."""
+    element-to-node force that leaves its workgroup once.  Counts come from the mesh itself."""
     import numpy as np
     f32 = precision == "fp32"
     r = 4 if f32 else 8               # element operator / stress / force values
@@ -188,14 +188,19 @@ def kernel_bytes(bundle, sc, layout: dict, precision: str) -> dict:
     nodepml = (ndof == 12) & (occ_pml > 0)
     out = {}
     ns = 12 if q else 6
-    out["element"] = (nr * (32 + ops("regular") + 2 * ns * r + 24 * r + (1 if q else 0) + (24 if dp else 0)
+    # in tiles a force leaves the element kernel through a slot only where its
+    # node is not an inner node of the tile; an inner node's state is updated
+    inner, slots = layout.get("tile_inner_nodes", 0), layout.get("tile_slots", 0)
+    forces = slots * (3 * r + 2) if layout.get("tiles", 0) else nr * 24 * r
+    out["element"] = (nr * (32 + ops("regular") + 2 * ns * r + (1 if q else 0) + (24 if dp else 0)
                             + (24 * r if mass_term else 0))
-                      + int((occ_reg > 0).sum()) * 3 * (nv + nu_r))
+                      + forces + int((occ_reg > 0).sum()) * 3 * (nv + nu_r)
+                      + inner * (16 + mb + 3 * nv + 3 * (2 * nu_w - nu_r)))
     # PML element: a PML node takes 6 values of its slot, a 3-component node 3
     pml_slots = int(np.where(ndof[ien[pml]] == 12, 6, 3).sum()) if npl else 0
     out["element_pml"] = (npl * (32 + ops("pml") + 2 * 21 * r + 3 * r + 1 + 6 * r + (24 * r if mass_term else 0))
                           + pml_slots * r + int((occ_pml > 0).sum()) * 3 * (nv + nu_r))
-    n3, e3 = int(node3.sum()), int(occ[node3].sum())
+    n3, e3 = int(node3.sum()) - inner, int(occ[node3].sum()) - 8 * inner
     if layout.get("node3_slot_major", 0):
         # node id, mass, state; all 8 entry slots of the slot-major table; the forces
         out["node"] = n3 * (4 + mb + 3 * 2 * nv + 3 * 2 * nu_w + 8 * 4) + e3 * 3 * r

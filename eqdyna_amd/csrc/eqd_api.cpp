@@ -10,7 +10,6 @@
 #include <algorithm>
 #include <map>
 #include <string>
-#include <tuple>
 #include <type_traits>
 #include <unordered_map>
 #include <vector>
@@ -18,6 +17,7 @@
 #include "eqd_internal.h"
 #include "eqd_precompute.h"
 #include "eqd_readback.h"
+#include "eqd_tiles.h"
 
 using namespace eqd;
 
@@ -444,64 +444,6 @@ static int upload_operators(eqd_handle *h, E &X, int64_t n, bool no_classes, OpR
     return 0;
 }
 
-// Element order within a class: bricks of 4 (x) x 8 (z) x 32 (y) elements,
-// y fastest inside a brick and bricks in y, then z, then x order, so that the
-// elements that share a node run close together in time and the node's data
-// is still in L2 when its next element needs it.  Grid indices come from the
-// element centroids: x and z as ranks of the distinct centroid coordinates
-// (to the millimetre), y as the rank within each (x, z) column, which holds
-// for columns shifted by a rough fault surface.  Results do not depend on the
-// order: every node sums its elements in ascending reference id.  Selected by
-// EQD_ELEMENT_ORDER=1; measured no faster than the reference order on the
-// 50 m and rough-fault boxes (the element kernels' L2 misses are mostly their
-// compulsory streams), so the reference order is the default.
-static void brick_order(std::vector<int32_t> &ids, const double *coor, const int32_t *ien)
-{
-    const int64_t n = (int64_t)ids.size();
-    if (n == 0) return;
-    std::vector<int64_t> qx(n), qz(n);
-    std::vector<double> cy(n);
-    for (int64_t t = 0; t < n; t++) {
-        const int64_t e = ids[t];
-        double c[3] = {0.0, 0.0, 0.0};
-        for (int a = 0; a < 8; a++)
-            for (int k = 0; k < 3; k++) c[k] += coor[(int64_t)(ien[e * 8 + a] - 1) * 3 + k];
-        qx[t] = std::llround(c[0] / 8.0 * 1000.0);
-        qz[t] = std::llround(c[2] / 8.0 * 1000.0);
-        cy[t] = c[1] / 8.0;
-    }
-    auto ranks = [n](const std::vector<int64_t> &q) {
-        std::vector<int64_t> u(q);
-        std::sort(u.begin(), u.end());
-        u.erase(std::unique(u.begin(), u.end()), u.end());
-        std::vector<int32_t> r(n);
-        for (int64_t t = 0; t < n; t++) r[t] = (int32_t)(std::lower_bound(u.begin(), u.end(), q[t]) - u.begin());
-        return r;
-    };
-    const std::vector<int32_t> xi = ranks(qx), zi = ranks(qz);
-    std::vector<int64_t> ord(n);
-    for (int64_t t = 0; t < n; t++) ord[t] = t;
-    std::sort(ord.begin(), ord.end(), [&](int64_t a, int64_t b) {
-        if (xi[a] != xi[b]) return xi[a] < xi[b];
-        if (zi[a] != zi[b]) return zi[a] < zi[b];
-        if (cy[a] != cy[b]) return cy[a] < cy[b];
-        return ids[a] < ids[b];
-    });
-    std::vector<int32_t> yi(n);
-    for (int64_t k = 0; k < n; k++) {
-        const int64_t t = ord[k];
-        const bool same = k > 0 && xi[ord[k - 1]] == xi[t] && zi[ord[k - 1]] == zi[t];
-        yi[t] = same ? yi[ord[k - 1]] + 1 : 0;
-    }
-    auto key = [&](int64_t t) {
-        return std::make_tuple(xi[t] / 4, zi[t] / 8, yi[t] / 32, xi[t] % 4, zi[t] % 8, yi[t] % 32, ids[t]);
-    };
-    std::sort(ord.begin(), ord.end(), [&](int64_t a, int64_t b) { return key(a) < key(b); });
-    std::vector<int32_t> out(n);
-    for (int64_t k = 0; k < n; k++) out[k] = ids[ord[k]];
-    ids.swap(out);
-}
-
 template <typename T>
 static void keep_copy(eqd_handle *h, int f, std::map<int, std::vector<T>> &dst)
 {
@@ -717,13 +659,49 @@ int eqd_commit(eqd_handle *h)
         if (sci[e] < 0 || (int64_t)sci[e] + need > s.size_stress + (t == 2 ? 0 : 6))
             return fail(h, EQD_EINVAL, "element %lld: stress index out of range", (long long)e + 1);
     }
+    // element entries of every node (rows of the gather table)
+    std::vector<int32_t> degree(nn, 0);
+    for (int64_t i = 0; i < 8 * ne; i++) degree[ien[i] - 1]++;
+    // Regular elements in tiles whose inner nodes the element kernel updates
+    // itself (elem_regular_kernel), from kTileMinElems elements on;
+    // EQD_ELEMENT_ORDER=0 keeps the reference's order, 1 makes tiles of any
+    // mesh they fill well.  Split nodes belong to the fault kernel, and a
+    // station's node is read by the step start, which runs in the same launch.
+    TileSet tiles;
     {
         const char *o = std::getenv("EQD_ELEMENT_ORDER");
-        if (o && o[0] == '1') {
-            brick_order(h->reg_ids, coor, ien);
-            brick_order(h->pml_ids, coor, ien);
+        const bool want = o && (o[0] == '0' || o[0] == '1') ? o[0] == '1' : (int64_t)h->reg_ids.size() >= kTileMinElems;
+        if (want) {
+            std::vector<uint8_t> outer(is_split);
+            const int32_t *idh = s.noff > 0 ? I32(h, EQD_IDHIST) : nullptr;
+            for (int64_t i = 0; i < 6 * (int64_t)s.noff; i++)
+                if (idh[i * 3] >= 1 && idh[i * 3] <= nn) outer[idh[i * 3] - 1] = 1;
+            if (make_tiles(h->reg_ids, ien, nn, degree, outer, tiles)) {
+                h->n_tile = (int32_t)tiles.tile.size();
+                h->at.swap(tiles.at);
+                auto &f = h->node3_free;
+                f.erase(std::remove_if(f.begin(), f.end(), [&](int32_t n) { return tiles.inner[n] != 0; }), f.end());
+            }
         }
     }
+    // a node's place on the device, and per-node arrays (component-major, in
+    // the reference's order) in that order and in blocks
+    auto at = [&](int64_t n) -> int32_t { return h->at.empty() ? (int32_t)n : h->at[n]; };
+    auto in_place = [&](const std::vector<int32_t> &nodes) {
+        std::vector<int32_t> v(nodes.size());
+        for (size_t i = 0; i < v.size(); i++) v[i] = at(nodes[i]);
+        return v;
+    };
+    auto node_blocks = [&](auto zero, const auto &cm) {
+        using T = decltype(zero);
+        std::vector<T> b((size_t)blocked_count(nn, 3), zero);
+        for (int64_t n = 0; n < nn; n++)
+            for (int k = 0; k < 3; k++) b[blocked_index(at(n), k, 3)] = (T)cm[(size_t)k * nn + n];
+        return b;
+    };
+    std::vector<int32_t> n3free = in_place(h->node3_free), n3all = in_place(h->node3_all);
+    std::sort(n3free.begin(), n3free.end());
+    std::sort(n3all.begin(), n3all.end());
     const int64_t nr = (int64_t)h->reg_ids.size(), np = (int64_t)h->pml_ids.size();
     if (nr > (int64_t)kEntIdxMask || np > (int64_t)kEntIdxMask) return fail(h, EQD_EINVAL, "too many elements in one class");
     h->n_reg = (int32_t)nr;
@@ -750,7 +728,7 @@ int eqd_commit(eqd_handle *h)
 #pragma omp parallel for schedule(static) reduction(max : qbad)
         for (int64_t t = 0; t < nr; t++) {
             const int64_t e = h->reg_ids[t];
-            for (int a = 0; a < 8; a++) r_ien[a * nr + t] = ien[e * 8 + a] - 1;
+            for (int a = 0; a < 8; a++) r_ien[a * nr + t] = at(ien[e * 8 + a] - 1);
             for (int i = 0; i < 24; i++) {
                 r_shp[i * nr + t] = shp[e * 24 + i];
                 r_em[i * nr + t] = emass[e * 24 + i];
@@ -853,8 +831,22 @@ int eqd_commit(eqd_handle *h)
             R *p;
             if ((r2 = dupload(h, &p, to_blocks<R>(r_st, nr, nst)))) return r2;
             E.stress = p;
-            if ((r2 = dalloc(h, &p, (nr + 63) / 64 * 64 * kEfReg))) return r2;
+            // force slots: the tiles', or 8 per element
+            const int64_t slots = h->n_tile ? (int64_t)tiles.slot_src.size() : blocked_count(nr, 8);
+            h->n_slot = h->n_tile ? slots : 0;
+            if ((r2 = dalloc(h, &p, slots * 3))) return r2;
             E.ef = p;
+            if (h->n_tile) {
+                Tile *tp;
+                uint16_t *ep, *sp;
+                if ((r2 = dupload(h, &tp, tiles.tile)) || (r2 = dupload(h, &ep, tiles.node_ent)) ||
+                    (r2 = dupload(h, &sp, tiles.slot_src)))
+                    return r2;
+                E.tile = tp;
+                E.n_tile = h->n_tile;
+                E.tile_ent = (const uint4 *)ep;
+                E.tile_src = sp;
+            }
             E.porep = d_porep;
             E.pstrain = d_pstrain;
             E.qidx = d_q;
@@ -880,7 +872,7 @@ int eqd_commit(eqd_handle *h)
             double xc[3] = {0, 0, 0};
             for (int a = 0; a < 8; a++) {
                 const int32_t nd = ien[e * 8 + a] - 1;
-                p_ien[a * np + p] = nd;
+                p_ien[a * np + p] = at(nd);
                 if (ndof[nd] == 12) m |= (uint8_t)(1u << a);
                 for (int i = 0; i < 3; i++) xc[i] = xc[i] + coor[(int64_t)nd * 3 + i];
             }
@@ -971,22 +963,26 @@ int eqd_commit(eqd_handle *h)
         std::vector<int32_t> cls_index(ne);
         for (int64_t t = 0; t < nr; t++) cls_index[h->reg_ids[t]] = (int32_t)t;
         for (int64_t p = 0; p < np; p++) cls_index[h->pml_ids[p]] = (int32_t)p;
+        // (a tile's inner nodes have no row: the element kernel sums them)
+        auto inner = [&](int64_t n) { return h->n_tile && tiles.inner[n]; };
         std::vector<int32_t> rowptr(nn + 1, 0);
-        for (int64_t e = 0; e < ne; e++)
-            for (int a = 0; a < 8; a++) rowptr[ien[e * 8 + a]]++;  // node id is 1-based: counts land at [node]
-        for (int64_t n = 0; n < nn; n++) rowptr[n + 1] += rowptr[n];
+        for (int64_t n = 0; n < nn; n++) rowptr[at(n) + 1] = inner(n) ? 0 : degree[n];
+        for (int64_t i = 0; i < nn; i++) rowptr[i + 1] += rowptr[i];
         std::vector<int32_t> fillp(rowptr.begin(), rowptr.end() - 1);
         std::vector<uint32_t> ent(rowptr[nn]);
         for (int64_t e = 0; e < ne; e++) {
             const bool pml = etype[e] == 2;
+            const int64_t t = cls_index[e];
             for (int a = 0; a < 8; a++) {
                 const int32_t nd = ien[e * 8 + a] - 1;
-                ent[fillp[nd]++] = (pml ? kEntPml : 0u) | ((uint32_t)a << kEntLocalShift) | (uint32_t)cls_index[e];
+                if (inner(nd)) continue;
+                ent[fillp[at(nd)]++] = pml ? kEntPml | ((uint32_t)a << kEntLocalShift) | (uint32_t)t
+                                       : (h->n_tile ? tiles.slot_of[t * 8 + a] : (uint32_t)reg_slot(t, a));
             }
         }
         for (int64_t q = 0; q < npn; q++) {
             const int32_t n = h->pml_node_ids[q];
-            for (int j = rowptr[n]; j < rowptr[n + 1]; j++)
+            for (int j = rowptr[at(n)]; j < rowptr[at(n) + 1]; j++)
                 if (!(ent[j] & kEntPml)) return fail(h, EQD_EINVAL, "PML node %d touches a regular element", n + 1);
         }
         int rc;
@@ -1001,16 +997,16 @@ int eqd_commit(eqd_handle *h)
         // (EQD_NODE_ELL=0 keeps the CSR gather)
         const char *ell_env = std::getenv("EQD_NODE_ELL");
         bool ell_ok = !(ell_env && ell_env[0] == '0');
-        const int64_t n3 = (int64_t)h->node3_free.size();
+        const int64_t n3 = (int64_t)n3free.size();
         for (int64_t i = 0; i < n3 && ell_ok; i++) {
-            const int32_t n = h->node3_free[i];
+            const int32_t n = n3free[i];
             if (rowptr[n + 1] - rowptr[n] > kEll3) ell_ok = false;
         }
         h->d_ell3 = nullptr;
         if (ell_ok && n3 > 0) {
             std::vector<uint32_t> ell((size_t)blocked_count(n3, kEll3), kEntNone);
             for (int64_t i = 0; i < n3; i++) {
-                const int32_t n = h->node3_free[i];
+                const int32_t n = n3free[i];
                 for (int j = rowptr[n]; j < rowptr[n + 1]; j++) ell[blocked_index(i, j - rowptr[n], kEll3)] = ent[j];
             }
             if ((rc = dupload(h, &h->d_ell3, ell))) return rc;
@@ -1029,34 +1025,41 @@ int eqd_commit(eqd_handle *h)
                 hi[j] = (float)disp[j];
                 lo[j] = bf16_bits((float)(disp[j] - (double)hi[j]));
             }
-            for (int64_t n = 0; n < nn; n++) m32[n] = (float)mass[n];
+            for (int64_t n = 0; n < nn; n++) m32[at(n)] = (float)mass[n];
             float *f;
             uint16_t *l;
-            if ((rc = dupload(h, &f, to_blocks<float>(vel, nn, 3)))) return rc; h->N.vel32 = f;
-            if ((rc = dupload(h, &f, to_blocks<float>(hi, nn, 3)))) return rc; h->N.dhi = f;
-            if ((rc = dupload(h, &l, to_blocks<uint16_t>(lo, nn, 3)))) return rc; h->N.dlo = l;
+            if ((rc = dupload(h, &f, node_blocks(0.0f, vel)))) return rc; h->N.vel32 = f;
+            if ((rc = dupload(h, &f, node_blocks(0.0f, hi)))) return rc; h->N.dhi = f;
+            if ((rc = dupload(h, &l, node_blocks((uint16_t)0, lo)))) return rc; h->N.dlo = l;
             if ((rc = dupload(h, &f, m32))) return rc; h->N.mass32 = f;
             std::vector<int32_t> slot(nn, -1);
             for (int64_t i = 0; i < s.nf; i++)
-                for (int j = 0; j < 2; j++) slot[nsmp[i * 2 + j] - 1] = (int32_t)(2 * i + j);
+                for (int j = 0; j < 2; j++) slot[at(nsmp[i * 2 + j] - 1)] = (int32_t)(2 * i + j);
             int32_t *ps;
             if ((rc = dupload(h, &ps, slot))) return rc; h->N.pair_slot = ps;
         } else {
-            if ((rc = dupload(h, &d, to_blocks<double>(vel, nn, 3)))) return rc; h->N.vel = d;
-            if ((rc = dupload(h, &d, to_blocks<double>(disp, nn, 3)))) return rc; h->N.disp = d;
+            if ((rc = dupload(h, &d, node_blocks(0.0, vel)))) return rc; h->N.vel = d;
+            if ((rc = dupload(h, &d, node_blocks(0.0, disp)))) return rc; h->N.disp = d;
         }
-        if ((rc = dupload(h, &d, to_blocks<double>(acc, nn, 3)))) return rc; h->N.acc = d;
-        if ((rc = dupload(h, &d, mass))) return rc; h->N.mass = d;
+        if ((rc = dupload(h, &d, node_blocks(0.0, acc)))) return rc; h->N.acc = d;
+        std::vector<double> mass_at(nn);
+        for (int64_t n = 0; n < nn; n++) mass_at[at(n)] = mass[n];
+        if ((rc = dupload(h, &d, mass_at))) return rc; h->N.mass = d;
+        if (h->n_tile) {
+            int32_t *ip;
+            if ((rc = dupload(h, &ip, h->at))) return rc; h->N.at = ip;
+            if ((rc = dupload(h, &ip, tiles.ref))) return rc; h->N.ref = ip;
+        }
         unsigned long long *fl;
         if ((rc = dalloc(h, &fl, 1))) return rc;
         HIPCHK(h, hipMemset(fl, 0xFF, sizeof(unsigned long long)));
         h->N.nanflag = fl;
-        if ((rc = dupload(h, &h->d_node3_free, h->node3_free))) return rc;
-        if ((rc = dupload(h, &h->d_node3_all, h->node3_all))) return rc;
+        if ((rc = dupload(h, &h->d_node3_free, n3free))) return rc;
+        if ((rc = dupload(h, &h->d_node3_all, n3all))) return rc;
         PmlNodes &PN = h->PN;
         PN.n = npn;
         int32_t *pn;
-        if ((rc = dupload(h, &pn, h->pml_node_ids))) return rc; PN.node = pn;
+        if ((rc = dupload(h, &pn, in_place(h->pml_node_ids)))) return rc; PN.node = pn;
         if ((rc = dupload(h, &d, to_blocks<double>(pdamp, npn, 3)))) return rc; PN.damp = d;
         if (s.precision == EQD_PREC_FP32) {
             std::vector<float> d32(pdamp.begin(), pdamp.end());
@@ -1123,7 +1126,7 @@ int eqd_commit(eqd_handle *h)
             if ((rc = dupload(h, &d, sv))) return rc; F.sv = d;
             if ((rc = dupload(h, &d, su))) return rc; F.su = d;
         }
-        if ((rc = dupload(h, &pi, fn))) return rc; F.nsmp = pi;
+        if ((rc = dupload(h, &pi, in_place(fn)))) return rc; F.nsmp = pi;
         if ((rc = dupload(h, &pi, sta))) return rc; F.station = pi;
         if ((rc = dupload(h, &d, un))) return rc; F.un = d;
         if ((rc = dupload(h, &d, us))) return rc; F.us = d;
@@ -1186,6 +1189,7 @@ int eqd_commit(eqd_handle *h)
                 t[2 * S.nrow + i] = idh[i * 3 + 2];
                 if (t[i] < 0 || t[i] >= nn || t[S.nrow + i] < 0 || t[S.nrow + i] > 2)
                     return fail(h, EQD_EINVAL, "idhist row %d out of range", i + 1);
+                t[i] = at(t[i]);
             }
             int rc;
             int32_t *pi;
@@ -1344,7 +1348,7 @@ int eqd_get(eqd_handle *h, int32_t field, void *host, int64_t count)
         for (int64_t i = 0; i < s.neq; i++) out[i] = orig.empty() ? 0.0 : orig[i];
         const int32_t *eqi = I32(h, EQD_EQNUMINDEXARR), *esl = I32(h, EQD_EQNUMSTARTINDEXLOC);
         for (int32_t n : h->node3_all)
-            for (int k = 0; k < 3; k++) out[eqi[esl[n] + k] - 1] = isv ? v[n * 3 + k] : v[blocked_index(n, k, 3)];
+            for (int k = 0; k < 3; k++) out[eqi[esl[n] + k] - 1] = isv ? v[n * 3 + k] : v[blocked_index(h->at.empty() ? n : h->at[n], k, 3)];
         const int64_t np = h->PN.n;
         for (int64_t q = 0; q < np; q++) {
             const int32_t n = h->pml_node_ids[q];
@@ -1593,7 +1597,7 @@ int eqd_record(eqd_handle *h, const int32_t *node_ids, int32_t n_nodes, int32_t 
     h->version++;
     if (capacity == 0) return EQD_OK;
     std::vector<int32_t> ids(node_ids, node_ids + n_nodes);
-    for (int32_t &v : ids) v -= 1;
+    for (int32_t &v : ids) v = h->at.empty() ? v - 1 : h->at[v - 1];
     const size_t nv = sizeof(double) * 3 * (size_t)capacity * (size_t)std::max(n_nodes, 1);
     const size_t ns = sizeof(double) * (size_t)capacity * (size_t)std::max<int64_t>(h->F.nf, 1);
     RecStream &q = h->rq;
@@ -1720,6 +1724,9 @@ int eqd_layout_info(eqd_handle *h, const char *key, int64_t *value)
     else if (k == "phi_compact_pml") *value = h->phi_compact_pml;
     else if (k == "geom_ops_regular") *value = h->s.precision == EQD_PREC_FP32 ? h->E32.opb_geom : 0;
     else if (k == "geom_ops_pml") *value = h->s.precision == EQD_PREC_FP32 ? h->P32.opb_geom : 0;
+    else if (k == "tiles") *value = h->n_tile;
+    else if (k == "tile_inner_nodes") *value = (int64_t)h->node3_all.size() - 2 * h->F.nf - (int64_t)h->node3_free.size();
+    else if (k == "tile_slots") *value = h->n_slot;
     else if (k == "node3_slot_major") *value = h->d_ell3 ? 1 : 0;
     else return fail(h, EQD_EINVAL, "unknown layout key %s", key);
     return EQD_OK;

@@ -11,7 +11,9 @@
 //  * the element-force buffers hold, per element and local node, the force the
 //    element contributes to that node (for PML nodes in factored form); a
 //    node-to-element table (CSR, ascending element order) lets each node sum
-//    its contributions without atomics.
+//    its contributions without atomics.  On larger meshes the regular elements
+//    run in compact tiles, and a node whose elements all lie in one tile is
+//    summed and updated there (Tile): its forces never leave the workgroup.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -20,10 +22,12 @@
 
 namespace eqd {
 
-// CSR entry: bit 31 = PML element, bits 28..30 = local node a, bits 0..27 =
-// element index within its class.
+// CSR entry: bit 31 = PML element, with local node a in bits 28..30 and the
+// element's index within its class in bits 0..27; else a regular element's
+// force slot (reg_slot, or its tile's) in bits 0..30.
 constexpr uint32_t kEntPml = 0x80000000u;
 constexpr uint32_t kEntIdxMask = 0x0FFFFFFFu;
+constexpr uint32_t kEntSlotMask = 0x7FFFFFFFu;
 constexpr int kEntLocalShift = 28;
 constexpr uint32_t kEntNone = 0xFFFFFFFFu;  // an unused slot of the ELL gather table
 constexpr int kEll3 = 8;
@@ -61,6 +65,9 @@ struct NodeState {
     const float *mass32;   // [nn] the same rounded to FP32, read by the FP32 bulk mode's node kernels
     const int32_t *rowptr; // [nn+1]
     const uint32_t *ent;   // CSR entries
+    // where the elements run in tiles the nodes are stored tile by tile (TileSet):
+    // the reference's node n at at[n], ref its inverse; else null, in its order
+    const int32_t *at, *ref;
     unsigned long long *nanflag; // first NaN velocity: step << 32 | node + 1 (all ones: none)
 };
 
@@ -103,21 +110,22 @@ __host__ __device__ __forceinline__ int64_t blk_at(int64_t t, int s)
 // c4 FP64 PML element kernel 0.288 -> 0.252 ms, step 1.006 -> 0.966 ms; in
 // FP32 (8-byte pairs) the same layout measured no faster on c4 and 1.4 %
 // slower on the 64-scenario ensemble, so the FP32 mode keeps blk_at.
-// The regular elements' forces on their nodes, component c of local node a
-// of element t: FP64 keeps x and y of a node as a 16-byte pair (rows 2a,
-// 2a+1 of a 64-element block interleaved) and z in rows 16 + a, so a node's
-// force is one paired and one single access; FP32 keeps blk_at<24> slot
-// a*3+c.  Both fill 24 rows of 64 values per block.
+// The regular elements' forces on their nodes, component c of force slot s:
+// FP64 keeps x and y of a slot as a 16-byte pair and z apart, so a node's
+// force is one paired and one single access; FP32 keeps blk_at<3>.  Both fill
+// 3 rows of 64 values per 64 slots.
 template <typename R>
-__host__ __device__ __forceinline__ int64_t reg_ef_at(int64_t t, int a, int c)
+__host__ __device__ __forceinline__ int64_t slot_at(int64_t s, int c)
 {
     if constexpr (sizeof(R) == sizeof(double)) {
-        if (c < 2) return ((t >> 6) * 24 + 2 * a) * 64 + (t & 63) * 2 + c;
-        return ((t >> 6) * 24 + 16 + a) * 64 + (t & 63);
+        if (c < 2) return (s >> 6) * 192 + (s & 63) * 2 + c;
+        return (s >> 6) * 192 + 128 + (s & 63);
     } else {
-        return blk_at<24>(t, a * 3 + c);
+        return blk_at<3>(s, c);
     }
 }
+// slot of element t's force on local node a where the elements run in no tiles
+__host__ __device__ __forceinline__ int64_t reg_slot(int64_t t, int a) { return blk_at<8>(t, a); }
 
 template <typename R, int W>
 __host__ __device__ __forceinline__ int64_t pml_at(int64_t t, int s)
@@ -125,7 +133,7 @@ __host__ __device__ __forceinline__ int64_t pml_at(int64_t t, int s)
     if constexpr (sizeof(R) == sizeof(double)) return ((t >> 6) * W + (s & ~1)) * 64 + (t & 63) * 2 + (s & 1);
     else return blk_at<W>(t, s);
 }
-constexpr int kEfReg = 24, kEfPml = 48;
+constexpr int kEfPml = 48;
 
 // Where an element kernel finds its operators: class tables in global memory
 // or per-element rows with Phi; class tables staged in LDS; per-element rows
@@ -152,9 +160,25 @@ __host__ __device__ __forceinline__ R phi_compact(const R *c, int m, int a, R s0
     return r - h;
 }
 
+// One tile: elements [e0, e0 + ne) of the regular class, one workgroup.  Its
+// inner nodes, the ones that no element outside the tile touches, are nodes
+// [n0, n0 + nn) with 8 entries each at tile_ent + i0, and the forces on its
+// other nodes leave through slots [64 s0, 64 s0 + ns) of ef in the order of
+// tile_src.  An entry names a force staged in LDS: local node * kTileElems +
+// lane.
+constexpr int kTileElems = 256;
+constexpr uint16_t kTileNone = 0xFFFFu;
+struct Tile {
+    int32_t e0, ne, n0, nn, i0, s0, ns;
+};
+
 template <typename R>
 struct RegElems {
     int64_t n;
+    const Tile *tile;  // null when the elements run in no tiles
+    int32_t n_tile;
+    const uint4 *tile_ent;
+    const uint16_t *tile_src;
     const int32_t *ien;   // 8 per element (blk_at<8>), 0-based node ids
     R *stress;            // 6, or 12 with Q, per element (blk_at)
     const R *emass;       // 24 per element (blk_at<24>; inertia/gravity term only)
@@ -162,7 +186,7 @@ struct RegElems {
     double *pstrain;      // [n]      (plastic only)
     const uint8_t *qidx;  // [n]      (Q only) row of qtab
     const double *qtab;   // [16][6]  exp(-dt/tau), 1-exp(-dt/tau), 8*w_p, 8*w_s, c_p, c_s
-    R *ef;                // force on local node a, component c at slot a*3+c (blk_at<kEfReg>)
+    R *ef;                // forces on the nodes (slot_at)
     // Operators: with classes (optab set), elements whose operators are
     // bit-identical share one row of optab (kOpW values, at opc[t]) and of
     // phitab (32 values, at phic[t]); otherwise each element has its own
@@ -265,6 +289,8 @@ struct Clock {
     int32_t mode;     // 1 on the last step of a run: store F/m instead of the fused update
     int32_t run_end;  // the step at which the current run ends
     int32_t rec_lo;   // first record index the host can take in this run (Recorder)
+    int32_t done;     // the last step whose node kernels have begun: nt, but not written while the
+                      // element kernels run, which read it beside the step start that advances nt
 };
 
 // launch kinds of one step
@@ -299,7 +325,7 @@ struct Member {
     FaultState F;
     OffStations S;
     StepConsts C;
-    const int32_t *node3_free;  // 3-component nodes that are not split nodes
+    const int32_t *node3_free;  // 3-component nodes that are neither split nodes nor inner nodes of a tile
     int64_t n_node3_free;
     // the free nodes' gather entries slot-major by position in node3_free
     // (blk_at<kEll3>: entry k of free node i at slot k), unused slots

@@ -1,7 +1,7 @@
 // The step engine of libeqd: advances one scenario (a handle) or an ensemble
 // of scenarios.  One step is (src/driver.f90:9-34)
-//   step start (clock, stations) + regular elements -> records -> PML elements
-//     -> fault pairs | nodes (3-comp, PML)
+//   records -> step start (clock, stations) + regular elements with the inner
+//     nodes of their tiles -> PML elements -> fault pairs | other nodes (3-comp, PML)
 // with the step start in the first blocks of the regular-element launch and
 // the fault pairs on a second stream beside the node kernels.  Every
 // launch covers all scenarios that share its kernel variant: the kernels find
@@ -64,9 +64,10 @@ Member<R> make_member(const eqd_engine *e, const eqd_handle *h)
 int64_t count_of(const eqd_handle *h, int kind)
 {
     switch (kind) {
-    case kKElem: return h->n_reg;
+    case kKElem: return h->n_tile ? (int64_t)h->n_tile * kTileElems : h->n_reg;
     case kKPml: return h->n_pml;
-    case kKNode3: return (int64_t)h->node3_free.size();
+    // a scenario with tiles always has a block: it tells the next step's element kernel its step (Clock::done)
+    case kKNode3: return std::max<int64_t>((int64_t)h->node3_free.size(), h->n_tile ? 1 : 0);
     case kKNodePml: return h->PN.n;
     case kKFault: return h->F.nf;
     case kKStation: return 0;  // the step start: its own launch or blocks of the first element launch
@@ -106,7 +107,10 @@ int variant(const eqd_handle *h, int kind, size_t *lds)
     *lds = 0;
     if (kind == kKElem) {
         *lds = class_lds(elems<R>(h), sizeof(R));
-        return q | dp << 1 | hg << 2 | mass << 4 | ops_of(elems<R>(h), *lds) << 5;
+        const int ops = ops_of(elems<R>(h), *lds);
+        // the staged forces of a tile, behind the class tables
+        if (h->n_tile) *lds += 24 * kTileElems * sizeof(R);
+        return q | dp << 1 | hg << 2 | mass << 4 | ops << 5;
     }
     if (kind == kKPml) {
         *lds = class_lds(pmls<R>(h), sizeof(R));
@@ -151,8 +155,8 @@ int build(eqd_engine *e)
     for (int m = 0; m < n; m++) M[m] = make_member<R>(e, e->hs[m]);
     for (int kind = 0; kind < kKinds; kind++) {
         if (kind == kKClock) continue;
-        int block = e->tune.block[kind];
-        if (kind == kKStation) block = 64;
+        int tuned = e->tune.block[kind];
+        if (kind == kKStation) tuned = 64;
         std::map<int, Group> by;
         for (int m = 0; m < n; m++) {
             if (count_of(e->hs[m], kind) == 0) continue;
@@ -166,6 +170,11 @@ int build(eqd_engine *e)
         for (auto &kv : by) {
             Group g = kv.second;
             int64_t blocks = 0;
+            // a tile is one workgroup, whatever shape the scenarios without tiles would run in
+            int block = tuned;
+            if (kind == kKElem)
+                for (int m : g.members)
+                    if (e->hs[m]->n_tile) block = kTileElems;
             for (int m : g.members) {
                 M[m].blk0[kind] = (int32_t)blocks;
                 blocks += (count_of(e->hs[m], kind) + block - 1) / block;
@@ -258,6 +267,12 @@ int enqueue_step(eqd_engine *e)
 {
     const Member<R> *dM = (const Member<R> *)e->d_members;
     hipStream_t st = e->st;
+    {
+        // records come first: the element kernel updates the inner nodes of its tiles
+        const auto &gr = e->groups[kKRecord];
+        const Stamp p = take_timer(e, kKRecord, gr.size());
+        for (size_t i = 0; i < gr.size(); i++) HIPCHK(e, launch_record<R>(dM, gr[i].g, st, p.start(i), p.stop(i)));
+    }
     // The step start (clock advance and off-fault stations, one block per
     // scenario) rides in the first blocks of the first regular-element
     // launch, which needs no clock itself; a step without regular elements
@@ -275,13 +290,6 @@ int enqueue_step(eqd_engine *e)
             HIPCHK(e, launch_elem<R>(dM, g.g, g.sig & 1, (g.sig >> 1) & 1, (g.sig >> 2) & 3, (g.sig >> 4) & 1,
                                      (g.sig >> 5) & 3, i == 0 ? nstart : 0, st, p.start(i), p.stop(i)));
         }
-    }
-    {
-        // records read the advanced clock; the element kernels leave the node
-        // state they record untouched
-        const auto &gr = e->groups[kKRecord];
-        const Stamp p = take_timer(e, kKRecord, gr.size());
-        for (size_t i = 0; i < gr.size(); i++) HIPCHK(e, launch_record<R>(dM, gr[i].g, st, p.start(i), p.stop(i)));
     }
     {
         const auto &gs = e->groups[kKPml];
@@ -399,7 +407,7 @@ int launch(eqd_engine *e, int32_t nsteps, bool mirrors)
     for (size_t m = 0; m < e->hs.size(); m++) {
         eqd_handle *h = e->hs[m];
         if (mirrors && recording(e, h)) lo[m] = h->rq.drained;
-        const Clock c = {h->time, h->nt, 0, h->nt + nsteps, lo[m]};
+        const Clock c = {h->time, h->nt, 0, h->nt + nsteps, lo[m], h->nt};
         HIPCHK(e, hipMemcpy(h->d_clock, &c, sizeof(Clock), hipMemcpyHostToDevice));
     }
     for (auto &kv : e->timers) {

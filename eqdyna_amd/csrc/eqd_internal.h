@@ -139,6 +139,9 @@ struct eqd_handle {
     std::vector<int32_t> node3_all, node3_free, pml_node_ids;
     std::vector<int32_t> pml_node_index;       // node -> PML node index or -1
     int32_t n_reg = 0, n_pml = 0, nreg_stress = 6;
+    std::vector<int32_t> at;  // with tiles: a node's place on the device (NodeState::at), else empty
+    int32_t n_tile = 0;  // tiles of the regular elements (0: none)
+    int64_t n_slot = 0;  // and their force slots
     std::vector<int32_t> hyp_pairs;  // pairs (0-based) at the hypocentre, in pair order
     // device objects
     eqd::NodeState N{};

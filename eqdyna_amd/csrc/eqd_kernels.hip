@@ -34,7 +34,7 @@ __device__ __forceinline__ void store_nt(R *p, R v)
     __builtin_nontemporal_store(v, p);
 }
 
-// two values of a force slot or summed-stress row (pml_at, reg_ef_at) as one access in
+// two values of a force slot or summed-stress row (pml_at, slot_at) as one access in
 // FP64, as two in FP32
 template <typename R>
 struct Pair;
@@ -373,6 +373,56 @@ __device__ __forceinline__ void exact_store(const Member<R> &M, int node, int k,
     node_store<R>(M.N, node, k, v, u);
 }
 
+// First NaN velocity: the reference stops at the first node, in node order, of
+// the first step whose update gives a NaN (src/driver.f90:147-152).  The key
+// (step << 32 | node + 1) is lowered atomically, so the earliest step and then
+// the lowest node wins whatever thread or stream finds it first.
+__device__ __forceinline__ void flag_nan(const NodeState &N, int node, int step, double v0, double v1, double v2)
+{
+    if (v0 != v0 || v1 != v1 || v2 != v2) {
+        const unsigned long long key = ((unsigned long long)(uint32_t)step << 32) | (uint32_t)((N.ref ? N.ref[node] : node) + 1);
+        atomicMin(N.nanflag, key);
+    }
+}
+
+// mass, velocity and displacement of a 3-component node
+struct Node3 {
+    double m, v[3], u[3];
+};
+template <typename R>
+__device__ __forceinline__ void node3_load(const NodeState &N, int node, Node3 &S)
+{
+    S.m = node_mass<R>(N, node);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        S.v[k] = node_v<R>(N, node, k);
+        S.u[k] = node_u<R>(N, node, k);
+    }
+}
+
+// Assembled force F of a 3-component node to its new state: a = F/m and the
+// update of the next step, or (mode 1, the last step of a run) a = F/m stored
+// for the next run to apply.
+template <typename R>
+__device__ __forceinline__ void node3_update(const NodeState &N, int node, const Node3 &S, const double F[3], double dt,
+                                             int mode, int next_step)
+{
+    if (mode == 1) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) N.acc[blk_at<3>(node, k)] = F[k] / S.m;
+        return;
+    }
+    double vn[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const double a = F[k] / S.m;
+        const double v = S.v[k] + a * dt;
+        node_store<R>(N, node, k, v, S.u[k] + v * dt);
+        vn[k] = v;
+    }
+    flag_nan(N, node, next_step, vn[0], vn[1], vn[2]);
+}
+
 // ------------------------------------------------------------------------
 // Regular (type 1, 11, 12, 13) elements: calcElemKU + calcElemMass + hrglss
 // for one element per thread.
@@ -439,54 +489,35 @@ __device__ __forceinline__ void exact_store(const Member<R> &M, int node, int k,
 #define EQD_FAULT_WAVES 1
 #endif
 
-//
+template <typename R>
+using lds_ptr = __attribute__((address_space(3))) R *;
+
 // kOps: where the operators come from (kOpsRows, kOpsLds, kOpsCompact).  With
 // kOpsLds both class tables are staged in LDS (dynamic shared memory of
 // (n_opc * kOpW + n_phic * 32) values) at block start, so the operator reads
 // of the element loop are LDS reads; with kOpsCompact Phi is rebuilt per node
 // (phi_compact) from 16 values read once per element; with kOpsGeom all
 // operators are rebuilt from the element's corner coordinates (geo_ops).
+// stage: the tile's force buffer in LDS (component c of local node a of lane l
+// at (a*3+c)*kTileElems + l), or null to store the forces to their slots.
 template <typename R, bool kQ, bool kDP, int kHG, bool kMass, int kOps>
-__global__ void __launch_bounds__(256, (kOps == kOpsGeom && !kQ && !kDP && !kMass ? EQD_REG_GEO_WAVES : 1))
-    elem_regular_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem, int remap, int nstart)
+__device__ __forceinline__ void regular_element(const RegElems<R> &E, const NodeState &N, const StepConsts &C, int64_t t,
+                                                lds_ptr<R> tables, bool staged, lds_ptr<R> stage)
 {
-    // With nstart > 0 the launch carries the step start of scenarios
-    // 0 .. nstart-1 in its first blocks, rounded up to a multiple of 8 so
-    // that the element blocks keep their XCD assignment.
-    const int nskip = step_start_skip(nstart);
-    if ((int)blockIdx.x < nskip) {
-        if ((int)blockIdx.x < nstart) step_start_block<R>(Ms[blockIdx.x]);
-        return;
-    }
     constexpr bool kGeo = kOps == kOpsGeom;
     constexpr bool kLds = kOps == kOpsLds, kCmp = kOps == kOpsCompact || kGeo;
     constexpr int kW = kGeo ? kOpG : (kCmp ? kOpBc : kOpB);
     constexpr int kNst = kQ ? 12 : 6;  // stress values per element (with the Q memory variables)
-    extern __shared__ __attribute__((aligned(16))) unsigned char eqd_smem[];
-    typedef __attribute__((address_space(3))) R lds_R;
-    const unsigned gb = launch_block(remap, (unsigned)nskip);
-    const Member<R> &M = Ms[member_of(bmem, gb)];
-    const RegElems<R> E = M.E;
-    const NodeState N = M.N;
-    const StepConsts C = M.C;
-    const int64_t t = (int64_t)(gb - (unsigned)M.blk0[kKElem]) * blockDim.x + threadIdx.x;
     const R *op = nullptr, *pht = nullptr;
-    const lds_R *lrow = nullptr, *lphr = nullptr;
+    lds_ptr<R> lrow = nullptr, lphr = nullptr;
     if constexpr (kLds) {
-        lds_R *lop = (lds_R *)eqd_smem, *lph = lop + E.n_opc * kOpW;
-        for (int j = threadIdx.x; j < E.n_opc * kOpW; j += blockDim.x) lop[j] = E.optab[j];
-        for (int j = threadIdx.x; j < E.n_phic * 32; j += blockDim.x) lph[j] = E.phitab[j];
-        __syncthreads();
-        if (t >= E.n) return;
-        lrow = lop + (int64_t)E.opc[t] * kOpW;
-        lphr = lph + (int64_t)E.phic[t] * 32;
+        lrow = tables + (int64_t)E.opc[t] * kOpW;
+        lphr = tables + E.n_opc * kOpW + (int64_t)E.phic[t] * 32;
     } else {
-        if (t >= E.n) return;
         // operators: one class-table row, or the element's own arrays
         op = E.optab ? E.optab + (int64_t)E.opc[t] * kOpW : nullptr;
         pht = E.phitab ? E.phitab + (int64_t)E.phic[t] * 32 : nullptr;
     }
-    const int64_t n = E.n, nn = N.nn;
     constexpr bool kF32 = sizeof(R) != sizeof(double);
     GeoOps<R> geo;
     if constexpr (kGeo)
@@ -797,13 +828,126 @@ constexpr int kU2 = (kKeep || kGeo) ? 8 : EQD_ELEM_UNROLL;
                 f[i] = f[i] + fv;
             }
         }
-        store_pair_nt(E.ef + reg_ef_at<R>(t, a, 0), f[0], f[1]);
-        store_nt(E.ef + reg_ef_at<R>(t, a, 2), f[2]);
+        if (staged) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) stage[(a * 3 + k) * kTileElems + threadIdx.x] = f[k];
+        } else {
+            const int64_t slot = reg_slot(t, a);
+            store_pair_nt(E.ef + slot_at<R>(slot, 0), f[0], f[1]);
+            store_nt(E.ef + slot_at<R>(slot, 2), f[2]);
+        }
         if constexpr (!kLds && !kKeep) {
 #pragma unroll
             for (int k = 0; k < kNo; k++) opc_[k] = opn_[k];
         }
     }
+}
+
+// The end of a tile's workgroup, called when the thread's own forces are
+// staged: inner node tid is summed in ascending element order, as gather3 sums
+// it, and updated in place (nothing outside the workgroup reads it during this
+// launch, and the workgroup has read it); the forces on the other nodes leave
+// through the tile's slots in whole lines.  Everything that comes from memory
+// is asked for before the barrier, so that the workgroup waits for it once.
+template <typename R>
+__device__ __forceinline__ void finish_tile(const RegElems<R> &E, const NodeState &N, const Tile &T, lds_ptr<R> stage,
+                                            double dt, int mode, int next_step)
+{
+    const int tid = threadIdx.x, node = T.n0 + tid;
+    constexpr int kAhead = 4;  // of the slots of a thread (3.3 on a regular grid)
+    const int64_t s0 = (int64_t)T.s0 * 64 + tid;
+    uint4 q;
+    Node3 S;
+    unsigned src[kAhead];
+    if (tid < T.nn) {
+        q = E.tile_ent[T.i0 + tid];
+        node3_load<R>(N, node, S);
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; i++)
+        src[i] = tid + i * kTileElems < T.ns ? E.tile_src[s0 + i * kTileElems] : kTileNone;
+    __syncthreads();
+    auto send = [&](unsigned e, int64_t slot) {
+        if (e == kTileNone) return;
+        const unsigned at = (e / kTileElems) * 3 * kTileElems + e % kTileElems;
+        store_pair_nt(E.ef + slot_at<R>(slot, 0), stage[at], stage[at + kTileElems]);
+        store_nt(E.ef + slot_at<R>(slot, 2), stage[at + 2 * kTileElems]);
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; i++) send(src[i], s0 + i * kTileElems);
+    for (int p = tid + kAhead * kTileElems; p < T.ns; p += kTileElems) send(E.tile_src[s0 + p - tid], s0 + p - tid);
+    if (tid < T.nn) {
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        double F[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const unsigned e = (w[k >> 1] >> ((k & 1) * 16)) & 0xFFFFu;
+            if (e != kTileNone) {
+                const unsigned at = (e / kTileElems) * 3 * kTileElems + e % kTileElems;
+                F[0] = F[0] + (double)stage[at];
+                F[1] = F[1] + (double)stage[at + kTileElems];
+                F[2] = F[2] + (double)stage[at + 2 * kTileElems];
+            }
+        }
+        node3_update<R>(N, node, S, F, dt, mode, next_step);
+    }
+}
+
+// One workgroup: the step start of a scenario, or a tile of elements with its
+// inner nodes, or (no tiles) blockDim.x elements.
+//
+// In tiles the forces on inner nodes (58 % of the nodes, 8 forces each) stay in
+// LDS, and so does their read and the second read of the nodes' state by the
+// node kernel.  256 elements a tile: 24 staged values are 24.6 KB in FP32, four
+// workgroups a CU at the kernel's own four waves per SIMD, 49 KB in FP64, three;
+// larger tiles would leave a CU too few workgroups to cover each other's
+// barrier.  Nodes are stored tile by tile (TileSet): in the reference's order a
+// tile's rows of nodes were parts of many lines, fetched by every tile that
+// shared them (2.42 M elements, FP32: 957 MB fetched against 608, 265 against
+// 221 us), and loads asked for before the barrier took it to 212, FP64 with
+// stored rows (686,000 elements) 124 -> 111.  Element and node kernel of a
+// step together: 686,000 elements FP64 165 -> 138 us; FP32 geometry rows 249
+// -> 274 (bound by their arithmetic) while the fault kernel beside the smaller
+// node kernel ends 60 us earlier.
+template <typename R, bool kQ, bool kDP, int kHG, bool kMass, int kOps>
+__global__ void __launch_bounds__(256, (kOps == kOpsGeom && !kQ && !kDP && !kMass ? EQD_REG_GEO_WAVES : 1))
+    elem_regular_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem, int remap, int nstart)
+{
+    // With nstart > 0 the launch carries the step start of scenarios
+    // 0 .. nstart-1 in its first blocks, rounded up to a multiple of 8 so
+    // that the element blocks keep their XCD assignment.
+    const int nskip = step_start_skip(nstart);
+    if ((int)blockIdx.x < nskip) {
+        if ((int)blockIdx.x < nstart) step_start_block<R>(Ms[blockIdx.x]);
+        return;
+    }
+    extern __shared__ __attribute__((aligned(16))) unsigned char eqd_smem[];
+    const unsigned gb = launch_block(remap, (unsigned)nskip);
+    const Member<R> &M = Ms[member_of(bmem, gb)];
+    const RegElems<R> E = M.E;
+    const NodeState N = M.N;
+    const StepConsts C = M.C;
+    const unsigned b = gb - (unsigned)M.blk0[kKElem];
+    lds_ptr<R> tables = (lds_ptr<R>)eqd_smem, stage = tables;
+    if constexpr (kOps == kOpsLds) {
+        lds_ptr<R> lph = tables + E.n_opc * kOpW;
+        for (int j = threadIdx.x; j < E.n_opc * kOpW; j += blockDim.x) tables[j] = E.optab[j];
+        for (int j = threadIdx.x; j < E.n_phic * 32; j += blockDim.x) lph[j] = E.phitab[j];
+        __syncthreads();
+        stage = lph + E.n_phic * 32;
+    }
+    if (!E.tile) {
+        const int64_t t = (int64_t)b * blockDim.x + threadIdx.x;
+        if (t < E.n) regular_element<R, kQ, kDP, kHG, kMass, kOps>(E, N, C, t, tables, false, stage);
+        return;
+    }
+    const Tile T = E.tile[b];
+    // this step and whether it ends the run (the step start that advances the
+    // clock runs in this launch)
+    const int nt = M.clk->done + 1, mode = nt == M.clk->run_end ? 1 : 0;
+    if ((int)threadIdx.x < T.ne)
+        regular_element<R, kQ, kDP, kHG, kMass, kOps>(E, N, C, T.e0 + (int)threadIdx.x, tables, true, stage);
+    finish_tile<R>(E, N, T, stage, C.dt, mode, nt + 1);
 }
 
 // ------------------------------------------------------------------------
@@ -1188,8 +1332,8 @@ __device__ __forceinline__ void gather3(const NodeState &N, int node, const R *e
                     load_pair(efp + pml_at<R, kEfPml>(idx, a * 6), f[k][0], f[k][1]);
                     f[k][2] = efp[pml_at<R, kEfPml>(idx, a * 6 + 2)];
                 } else {
-                    load_pair(ef + reg_ef_at<R>(idx, a, 0), f[k][0], f[k][1]);
-                    f[k][2] = ef[reg_ef_at<R>(idx, a, 2)];
+                    load_pair(ef + slot_at<R>(e[k], 0), f[k][0], f[k][1]);
+                    f[k][2] = ef[slot_at<R>(e[k], 2)];
                 }
             }
         }
@@ -1224,8 +1368,8 @@ __device__ __forceinline__ void gather3_ell(const uint32_t *ell, int64_t i, cons
                 load_pair(efp + pml_at<R, kEfPml>(idx, a * 6), f[k][0], f[k][1]);
                 f[k][2] = efp[pml_at<R, kEfPml>(idx, a * 6 + 2)];
             } else {
-                load_pair(ef + reg_ef_at<R>(idx, a, 0), f[k][0], f[k][1]);
-                f[k][2] = ef[reg_ef_at<R>(idx, a, 2)];
+                load_pair(ef + slot_at<R>(e[k], 0), f[k][0], f[k][1]);
+                f[k][2] = ef[slot_at<R>(e[k], 2)];
             }
         }
     }
@@ -1239,21 +1383,8 @@ __device__ __forceinline__ void gather3_ell(const uint32_t *ell, int64_t i, cons
     }
 }
 
-// First NaN velocity: the reference stops at the first node, in node order, of
-// the first step whose update gives a NaN (src/driver.f90:147-152).  The key
-// (step << 32 | node + 1) is lowered atomically, so the earliest step and then
-// the lowest node wins whatever thread or stream finds it first.
-__device__ __forceinline__ void flag_nan(const NodeState &N, int node, int step, double v0, double v1, double v2)
-{
-    if (v0 != v0 || v1 != v1 || v2 != v2) {
-        const unsigned long long key = ((unsigned long long)(uint32_t)step << 32) | (uint32_t)(node + 1);
-        atomicMin(N.nanflag, key);
-    }
-}
-
-// Node kernel for 3-component nodes that are not split nodes.
-// mode 0: gather, a = F/m, then the update of the next step (fused);
-// mode 1: gather, store a = F/m (the last step of a run).
+// Node kernel for 3-component nodes that are neither split nodes nor inner
+// nodes of a tile: gather, then node3_update.
 template <typename R>
 __global__ void __launch_bounds__(256) node3_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem,
                                                     int remap)
@@ -1261,32 +1392,21 @@ __global__ void __launch_bounds__(256) node3_kernel(const Member<R> *__restrict_
     const unsigned gb = launch_block(remap);
     const Member<R> &M = Ms[member_of(bmem, gb)];
     const int64_t i = (int64_t)(gb - (unsigned)M.blk0[kKNode3]) * blockDim.x + threadIdx.x;
+    const Clock ck = *M.clk;
+    if (i == 0) M.clk->done = ck.nt;
     if (i >= M.n_node3_free) return;
     const NodeState N = M.N;
     const R *ef = M.E.ef, *efp = M.P.ef;
     const double dt = M.C.dt;
-    const Clock ck = *M.clk;
     const int mode = ck.mode, next_step = ck.nt + 1;
     const int node = M.node3_free[i];
     const int64_t nn = N.nn;
     double F[3];
     if (M.ell3) gather3_ell<R>(M.ell3, i, ef, efp, F);
     else gather3<R>(N, node, ef, efp, F);
-    const double m = node_mass<R>(N, node);
-    if (mode == 1) {
-#pragma unroll
-        for (int k = 0; k < 3; k++) N.acc[blk_at<3>(node, k)] = F[k] / m;
-        return;
-    }
-    double vn[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const double a = F[k] / m;
-        const double v = node_v<R>(N, node, k) + a * dt;
-        node_store<R>(N, node, k, v, node_u<R>(N, node, k) + v * dt);
-        vn[k] = v;
-    }
-    flag_nan(N, node, next_step, vn[0], vn[1], vn[2]);
+    Node3 S;
+    node3_load<R>(N, node, S);
+    node3_update<R>(N, node, S, F, dt, mode, next_step);
 }
 
 // 12-component (PML) nodes; the gather reads only PML element forces because
@@ -1970,7 +2090,7 @@ __global__ void __launch_bounds__(256) record_kernel(const Member<R> *__restrict
     const int64_t t = (int64_t)(gb - (unsigned)M.blk0[kKRecord]) * blockDim.x + threadIdx.x;
     const Recorder rc = *M.rec;
     if (t >= rc.n_nodes) return;
-    const int nt = M.clk->nt;
+    const int nt = M.clk->nt + 1;  // the step about to start
     if ((nt - 1) % rc.every != 0) return;
     const int32_t r = (nt - 1) / rc.every, lo = M.clk->rec_lo;
     if (r < lo || r - lo >= rc.capacity) return;
@@ -2009,21 +2129,21 @@ hipError_t launch_elem(const Member<R> *M, const LaunchGrid &g, int q, int dp, i
     // geometry rows exist in the FP32 bulk mode only
     if (ops == kOpsGeom && sizeof(R) != sizeof(float)) return hipErrorInvalidValue;
     constexpr int kGeoOr = sizeof(R) == sizeof(float) ? kOpsGeom : kOpsCompact;
-    // class tables in LDS (at most 16 KiB) or operators from memory
-    const size_t lds = ops == kOpsLds ? g.lds : 0;
+    // class tables (at most 16 KiB) and a tile's staged forces
+    const size_t lds = g.lds;
 #define EQD_LAUNCH(Q, DP, HG, MASS)                                                                               \
     do {                                                                                                          \
         if (ops == kOpsLds)                                                                                       \
             EQD_GO((elem_regular_kernel<R, Q, DP, HG, MASS, kOpsLds>), grid, g.block, lds, s, M, g.bmem, g.remap,  \
                    nstart);                                                                                       \
         else if (ops == kOpsGeom)                                                                                 \
-            EQD_GO((elem_regular_kernel<R, Q, DP, HG, MASS, kGeoOr>), grid, g.block, 0, s, M, g.bmem, g.remap,     \
+            EQD_GO((elem_regular_kernel<R, Q, DP, HG, MASS, kGeoOr>), grid, g.block, lds, s, M, g.bmem, g.remap,     \
                    nstart);                                                                                       \
         else if (ops == kOpsCompact)                                                                              \
-            EQD_GO((elem_regular_kernel<R, Q, DP, HG, MASS, kOpsCompact>), grid, g.block, 0, s, M, g.bmem,         \
+            EQD_GO((elem_regular_kernel<R, Q, DP, HG, MASS, kOpsCompact>), grid, g.block, lds, s, M, g.bmem,         \
                    g.remap, nstart);                                                                              \
         else                                                                                                      \
-            EQD_GO((elem_regular_kernel<R, Q, DP, HG, MASS, kOpsRows>), grid, g.block, 0, s, M, g.bmem, g.remap,   \
+            EQD_GO((elem_regular_kernel<R, Q, DP, HG, MASS, kOpsRows>), grid, g.block, lds, s, M, g.bmem, g.remap,   \
                    nstart);                                                                                       \
     } while (0)
 #define EQD_HG(Q, DP, MASS)                         \

@@ -30,7 +30,7 @@ __global__ void __launch_bounds__(256) pack_nodes_kernel(NodeState N, FaultState
 {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= 3 * count) return;
-    const int64_t node = first + j / 3;
+    const int64_t node = N.at ? N.at[first + j / 3] : first + j / 3;
     const int k = (int)(j % 3);
     const int64_t at = blk_at<3>(node, k);
     double x;

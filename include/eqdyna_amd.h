@@ -167,7 +167,10 @@ int64_t eqd_device_bytes(eqd_handle *h);
  * the coordinates, EQD_GEOM_OPS=0 in the environment keeps them stored);
  * "node3_slot_major": 1 when the 3-component nodes gather their element
  * forces from a slot-major table of 8 entries per node (every such node has
- * at most 8 elements; EQD_NODE_ELL=0 keeps the CSR table).
+ * at most 8 elements; EQD_NODE_ELL=0 keeps the CSR table); "tiles": the
+ * regular elements run in this many tiles whose "tile_inner_nodes" nodes the
+ * element kernel updates itself, the other forces leaving through
+ * "tile_slots" slots (0: no tiles; EQD_ELEMENT_ORDER).
  * Returns EQD_EINVAL for an unknown key. */
 int eqd_layout_info(eqd_handle *h, const char *key, int64_t *value);
 
