@@ -282,6 +282,161 @@ __device__ __forceinline__ void geo_ops(const R *opb, int64_t t, R lam, R mu, Ge
     }
 }
 
+// ------------------------------------------------------------------------
+// The same operators in modal form.  The eight signs of a trilinear element's
+// nodes split into a constant, three linear modes (ac) and the four hourglass
+// modes Gamma, mutually orthogonal, and every operator of the element kernels
+// is a few numbers in that basis:
+//   dN_a/dx_i = sum_l ac_al q c[l][i]      (c: cofactors of the Jacobian, q = 1 / (8 det))
+//   Phi_ma    = rs_m Gamma_ma - sum_l ac_al wr[m][l]
+// so gradients and hourglass amplitudes of a nodal field follow from its eight
+// modal sums (split8: 23 additions a component), and the eight nodal forces
+// from seven modal ones (join8): 1,260 vector instructions per regular element
+// instead of 2,300 node by node.  Fused multiply-adds allowed (each rounds once
+// where two operations round twice).
+//
+// Used by the regular elements of tiles, where the node-by-node form is bound
+// by its arithmetic (145 of 212 us for 2.42 M elements; this one takes 176 and
+// is bound by memory, 5.1 TB/s).  The PML elements are bound by memory in
+// either form (117 and 118 us for 1.04 M).  Error of velocity and displacement
+// against FP64, rough-fault boxes of 60,000 to 350,000 elements: 4.49e-7 and
+// 1.32e-7 node by node, 4.41e-7 and 1.29e-7 here; in boxes of a few thousand
+// elements, where neither form matters to the time, the displacement's was
+// larger here (2.1e-7 against 1.9e-7), so scenarios without tiles keep geo_ops.
+template <typename R>
+struct ModalOps {
+    R c[9], q, dq, det, ss[6], rs[4], wr[12];
+};
+
+// modal sums of eight nodal values: lin = sum_a ac_al f_a, hg = sum_a Gamma_ma f_a
+template <typename R>
+__device__ __forceinline__ void split8(const R f[8], R lin[3], R hg[4])
+{
+    R e[2], x[2], y[2], xy[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const R s0 = f[4 * h] + f[4 * h + 1], d0 = f[4 * h + 1] - f[4 * h];
+        const R s1 = f[4 * h + 3] + f[4 * h + 2], d1 = f[4 * h + 2] - f[4 * h + 3];
+        e[h] = s0 + s1;
+        y[h] = s1 - s0;
+        x[h] = d0 + d1;
+        xy[h] = d1 - d0;
+    }
+    lin[0] = x[0] + x[1];
+    lin[1] = y[0] + y[1];
+    lin[2] = e[1] - e[0];
+    hg[0] = y[1] - y[0];
+    hg[1] = x[1] - x[0];
+    hg[2] = xy[0] + xy[1];
+    hg[3] = xy[1] - xy[0];
+}
+
+// f_a = sum_l ac_al lin_l + sum_m Gamma_ma hg_m
+template <typename R>
+__device__ __forceinline__ void join8(const R lin[3], const R hg[4], R f[8])
+{
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const R z = h ? lin[2] : -lin[2];
+        const R x = h ? lin[0] + hg[1] : lin[0] - hg[1];
+        const R y = h ? lin[1] + hg[0] : lin[1] - hg[0];
+        const R q = h ? hg[2] + hg[3] : hg[2] - hg[3];
+        const R m = z - y, p = z + y, d = x - q, s = x + q;
+        f[4 * h] = m - d;
+        f[4 * h + 1] = m + d;
+        f[4 * h + 2] = p + s;
+        f[4 * h + 3] = p - s;
+    }
+}
+
+// from the coordinates of local nodes 1..7 relative to node 0, so the values
+// are rounded relative to the element's size
+template <typename R>
+__device__ __forceinline__ void modal_ops(const R *opb, int64_t t, R lam, R mu, ModalOps<R> &G)
+{
+#pragma clang fp contract(fast)
+    R a[3][3], b[4][3];  // a[l][j] = d x_j / d xi_l, b[m][j] = sum_b Gamma_mb x_bj
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        R x[8], lin[3], hg[4];
+        x[0] = 0;
+#pragma unroll
+        for (int k = 1; k < 8; k++) x[k] = opb_at<R, kOpG>(opb, t, (k - 1) * 3 + j);
+        split8<R>(x, lin, hg);
+#pragma unroll
+        for (int l = 0; l < 3; l++) a[l][j] = lin[l] * (R)0.125;
+#pragma unroll
+        for (int m = 0; m < 4; m++) b[m][j] = hg[m];
+    }
+    auto cross = [](const R u[3], const R v[3], R w[3]) {
+        w[0] = u[1] * v[2] - u[2] * v[1];
+        w[1] = u[2] * v[0] - u[0] * v[2];
+        w[2] = u[0] * v[1] - u[1] * v[0];
+    };
+    auto dot = [](const R u[3], const R v[3]) { return u[0] * v[0] + u[1] * v[1] + u[2] * v[2]; };
+    R c[3][3];  // c[l][i]: cofactors, d xi_l / d x_i times det
+    cross(a[1], a[2], c[0]);
+    cross(a[2], a[0], c[1]);
+    cross(a[0], a[1], c[2]);
+    G.det = dot(a[0], c[0]);
+    const R q = (R)0.125 / G.det;
+    G.q = q;
+    G.dq = __builtin_fmaf(-q, (R)8 * G.det, (R)1);
+#pragma unroll
+    for (int i = 0; i < 9; i++) G.c[i] = c[i / 3][i % 3];
+    // volume of the trilinear hexahedron (vlm, src/library.f90:60-93): the
+    // integral of the Jacobian determinant, whose even terms are these
+    R w0[3], w1[3], w2[3];
+    cross(b[2], b[1], w0);
+    cross(b[0], b[2], w1);
+    cross(b[1], b[0], w2);
+    const R vol = (R)8 * G.det + (dot(a[0], w0) + dot(a[1], w1) + dot(a[2], w2)) * (R)(1.0 / 24.0);
+    // SS = co X^T X with X the inverse Jacobian (calcSSPhi4Hrgls), X = 8 q c
+    const R ce = (R)16 * (mu * ((R)3 * lam + (R)2 * mu) / (lam + mu)) / (R)15;
+    const R cq = ce * vol / (R)0.75 * q * q, co = cq + (R)2 * G.dq * cq;
+    constexpr int si[6] = {0, 0, 0, 1, 1, 2}, sj[6] = {0, 1, 2, 1, 2, 2};
+#pragma unroll
+    for (int k = 0; k < 6; k++)
+        G.ss[k] = co * (G.c[si[k]] * G.c[sj[k]] + G.c[3 + si[k]] * G.c[3 + sj[k]] + G.c[6 + si[k]] * G.c[6 + sj[k]]);
+    // s_m, the rms over a of Gamma_ma - sum_l ac_al w_l, is sqrt(1 + |w|^2)
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        R w[3];
+#pragma unroll
+        for (int l = 0; l < 3; l++) w[l] = (b[m][0] * c[l][0] + b[m][1] * c[l][1] + b[m][2] * c[l][2]) * q;
+        G.rs[m] = (R)1 / sqrt((R)1 + dot(w, w));
+#pragma unroll
+        for (int l = 0; l < 3; l++) G.wr[3 * m + l] = w[l] * G.rs[m];
+    }
+}
+
+// The hourglass force modes of an element: with the amplitudes of ut,
+// pd_m = sum_a Phi_ma ut_a, and g_m = SS pd_m, the force -sum_m Phi_ma g_m on
+// node a is added to the linear modes lin[k][l] and put into hg[k][m].
+template <typename R>
+__device__ __forceinline__ void modal_hourglass(const ModalOps<R> &G, const R ul[3][3], const R uh[3][4], R lin[3][3],
+                                                R hg[3][4])
+{
+#pragma clang fp contract(fast)
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        R pd[3], g[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            pd[k] = G.rs[m] * uh[k][m] -
+                    (G.wr[3 * m] * ul[k][0] + G.wr[3 * m + 1] * ul[k][1] + G.wr[3 * m + 2] * ul[k][2]);
+        g[0] = G.ss[0] * pd[0] + G.ss[1] * pd[1] + G.ss[2] * pd[2];
+        g[1] = G.ss[1] * pd[0] + G.ss[3] * pd[1] + G.ss[4] * pd[2];
+        g[2] = G.ss[2] * pd[0] + G.ss[4] * pd[1] + G.ss[5] * pd[2];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            hg[k][m] = -(G.rs[m] * g[k]);
+#pragma unroll
+            for (int l = 0; l < 3; l++) lin[k][l] = lin[k][l] + G.wr[3 * m + l] * g[k];
+        }
+    }
+}
+
 // split velocity k of PML node q
 template <typename R>
 __device__ __forceinline__ double pml_v(const PmlNodes &P, int64_t q, int k)
@@ -498,6 +653,192 @@ using lds_ptr = __attribute__((address_space(3))) R *;
 // of the element loop are LDS reads; with kOpsCompact Phi is rebuilt per node
 // (phi_compact) from 16 values read once per element; with kOpsGeom all
 // operators are rebuilt from the element's corner coordinates (geo_ops).
+// Stress update of a regular element from its strain rate (and, with Q, its
+// strain): Hooke's law, the Q memory variables, the Drucker-Prager return
+// (src/calcElemKU.f90:36-167).  srt: the stress rate; stress: the new stress,
+// stored as well.
+template <typename R, bool kQ, bool kDP>
+__device__ __forceinline__ void regular_stress(const RegElems<R> &E, const StepConsts &C, int64_t t, R lam, R miu,
+                                               const R sr[6], const R strain[6], R srt[6], R stress[6])
+{
+    constexpr int kNst = kQ ? 12 : 6;  // stress values per element (with the Q memory variables)
+    const R cdiag = lam + (R)2 * miu;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        R acc = 0;
+#pragma unroll
+        for (int j = 0; j < 3; j++) acc = acc + (i == j ? cdiag : lam) * sr[j];
+        srt[i] = acc;
+    }
+#pragma unroll
+    for (int i = 3; i < 6; i++) srt[i] = miu * sr[i];
+
+    R strdev[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++) stress[i] = load_nt(E.stress + blk_at<kNst>(t, i));
+    if (!kQ) {
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            stress[i] = stress[i] + srt[i] * (R)C.dt;
+            strdev[i] = stress[i];
+        }
+    } else {
+        const double *q = E.qtab + 6 * E.qidx[t];
+        const R e1 = (R)q[0], e2 = (R)q[1], wkp = (R)q[2], wks = (R)q[3], cv = (R)q[4], cs = (R)q[5];
+        const R miuu = miu * cs;
+        const R Mu = (lam + (R)2 * miu) * cv;
+        const R vols = strain[0] + strain[1] + strain[2];
+        R anestr1[6], anestr[6];
+#pragma unroll
+        for (int i = 0; i < 6; i++) anestr1[i] = load_nt(E.stress + blk_at<kNst>(t, 6 + i));
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            anestr[i] = e1 * anestr1[i] + e2 * ((R)2 * miuu * strain[i] * wks + (Mu * wkp - (R)2 * miuu * wks) * vols);
+#pragma unroll
+        for (int i = 3; i < 6; i++) anestr[i] = e1 * anestr1[i] + e2 * (miuu * strain[i] * wks);
+#pragma unroll
+        for (int i = 0; i < 6; i++) store_nt(E.stress + blk_at<kNst>(t, 6 + i), anestr[i]);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            stress[i] = (R)2 * miuu * strain[i] + (Mu - (R)2 * miuu) * vols - (R)0.5 * (anestr[i] + anestr1[i]);
+#pragma unroll
+        for (int i = 3; i < 6; i++)
+            stress[i] = (R)2 * miuu * strain[i] / (R)2 - (R)0.5 * (anestr[i] + anestr1[i]);
+#pragma unroll
+        for (int i = 0; i < 6; i++) strdev[i] = stress[i];
+    }
+    if (kDP) {
+        // Drucker-Prager viscoplastic return, src/calcElemKU.f90:133-167
+        const R strmea = (stress[0] + stress[1] + stress[2]) / (R)3;
+#pragma unroll
+        for (int i = 0; i < 3; i++) strdev[i] = stress[i] - strmea;
+        R taomax = (R)0.5 * (sqr(strdev[0]) + sqr(strdev[1]) + sqr(strdev[2])) + sqr(strdev[3]) +
+                   sqr(strdev[4]) + sqr(strdev[5]);
+        taomax = sqrt(taomax);
+        R yield = (R)C.ccosphi - (R)C.sinphi * (strmea + (R)E.porep[t]);
+        if (yield < (R)0) yield = 0;
+        R pstrmag = 0;
+        if (taomax > yield) {
+            const R rjust = yield / taomax + ((R)1 - yield / taomax) * (R)C.exp_dt_tv;
+            R pstrinc[6];
+#pragma unroll
+            for (int i = 0; i < 6; i++) {
+                stress[i] = strdev[i] * rjust;
+                pstrinc[i] = (strdev[i] - stress[i]) / miu;
+                if (i < 3) stress[i] = stress[i] + strmea;
+            }
+            const R pstrmea = (pstrinc[0] + pstrinc[1] + pstrinc[2]) / (R)3;
+#pragma unroll
+            for (int i = 0; i < 6; i++) pstrinc[i] = pstrinc[i] - pstrmea;
+            R pm = (R)0.5 * (sqr(pstrinc[0]) + sqr(pstrinc[1]) + sqr(pstrinc[2])) + sqr(pstrinc[3]) +
+                   sqr(pstrinc[4]) + sqr(pstrinc[5]);
+            pstrmag = sqrt(pm);
+        }
+        E.pstrain[t] = E.pstrain[t] + (double)pstrmag;
+    }
+#pragma unroll
+    for (int i = 0; i < 6; i++) store_nt(E.stress + blk_at<kNst>(t, i), stress[i]);
+}
+
+// An element of a tile with its operators in modal form (kOpsGeom), otherwise
+// as regular_element.
+template <typename R, bool kQ, bool kDP, int kHG, bool kMass>
+__device__ __forceinline__ void regular_element_modal(const RegElems<R> &E, const NodeState &N, const StepConsts &C,
+                                                      int64_t t, lds_ptr<R> stage)
+{
+#pragma clang fp contract(fast)
+    int nds[8];
+#pragma unroll
+    for (int a = 0; a < 8; a++) nds[a] = load_nt(E.ien + blk_at<8>(t, a));
+    const R lam = opb_at<R, kOpG>(E.opb, t, kGeoMat), miu = opb_at<R, kOpG>(E.opb, t, kGeoMat + 1);
+    ModalOps<R> G;
+    modal_ops<R>(E.opb, t, lam, miu, G);
+    const R rdk = (R)C.rdampk;
+    // modal sums of velocity and displacement relative to the first node (the
+    // arithmetic then rounds relative to the deformation, not to the absolute
+    // motion): velocity gradient, strain with Q, and ut = u + rdampk v
+    R vl[3][3], ul[3][3], uh[3][4], vh[3][4];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        R f[8];
+#pragma unroll
+        for (int a = 0; a < 8; a++) f[a] = gather_v<R>(N, nds[a], k);
+#pragma unroll
+        for (int a = 7; a >= 0; a--) f[a] = f[a] - f[0];
+        split8<R>(f, vl[k], vh[k]);
+#pragma unroll
+        for (int a = 0; a < 8; a++) f[a] = gather_u<R>(N, nds[a], k);
+#pragma unroll
+        for (int a = 7; a >= 0; a--) f[a] = f[a] - f[0];
+        split8<R>(f, ul[k], uh[k]);
+    }
+    // gradient of component k along i
+    auto grad = [&](const R l[3][3], int k, int i) {
+        const R g = (G.c[i] * l[k][0] + G.c[3 + i] * l[k][1] + G.c[6 + i] * l[k][2]) * G.q;
+        return g + g * G.dq;  // q's rounding, the same in every element of a regular grid, would add up
+    };
+    auto strains = [&](const R l[3][3], R e[6]) {
+        e[0] = grad(l, 0, 0);
+        e[1] = grad(l, 1, 1);
+        e[2] = grad(l, 2, 2);
+        e[3] = grad(l, 1, 2) + grad(l, 2, 1);
+        e[4] = grad(l, 0, 2) + grad(l, 2, 0);
+        e[5] = grad(l, 0, 1) + grad(l, 1, 0);
+    };
+    R sr[6], strain[6], srt[6], stress[6];
+    strains(vl, sr);
+    if (kQ) strains(ul, strain);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+#pragma unroll
+        for (int l = 0; l < 3; l++) ul[k][l] = ul[k][l] + rdk * vl[k][l];
+#pragma unroll
+        for (int m = 0; m < 4; m++) uh[k][m] = uh[k][m] + rdk * vh[k][m];
+    }
+    regular_stress<R, kQ, kDP>(E, C, t, lam, miu, sr, strain, srt, stress);
+    // force modes: (-det*w) * B^T (sigma + rdampk*sigma_dot), - hourglass; det q = 1/8
+    const R temp = (R)-0.125 * (R)C.w;
+    R st[6], lin[3][3], hg[3][4];
+#pragma unroll
+    for (int i = 0; i < 6; i++) st[i] = temp * (stress[i] + rdk * srt[i]);
+    constexpr int sym[3][3] = {{0, 5, 4}, {5, 1, 3}, {4, 3, 2}};
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int l = 0; l < 3; l++)
+            lin[k][l] = G.c[3 * l] * st[sym[k][0]] + G.c[3 * l + 1] * st[sym[k][1]] + G.c[3 * l + 2] * st[sym[k][2]];
+    if (kHG == 1) {
+        // Kosloff-Frazier stiffness hourglass, src/hrglss.f90:20-55
+        modal_hourglass<R>(G, ul, uh, lin, hg);
+    } else {
+        // viscous hourglass, src/hrglss.f90:57-97
+        R coef = 0;
+        if (kHG == 2) {
+            const R vp = opb_at<R, kOpG>(E.opb, t, kGeoMat + 2), rho = opb_at<R, kOpG>(E.opb, t, kGeoMat + 3);
+            coef = (R)0.25 * (R)C.kapa_hg * rho * vp * (R)pow((double)G.det * C.w, 2.0 / 3.0);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int m = 0; m < 4; m++) hg[k][m] = kHG == 2 ? -(coef * vh[k][m]) : (R)0;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        R f[8];
+        join8<R>(lin[k], hg[k], f);
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            if (kMass) {
+                // absolute velocity here: the Rayleigh mass term is not translation invariant
+                R al = (R)(C.rdampm * node_v<R>(N, nds[a], k));
+                if (k == 2) al = al + (R)C.gterm;
+                f[a] = f[a] - al * E.emass[blk_at<24>(t, a * 3 + k)];
+            }
+            stage[(a * 3 + k) * kTileElems + threadIdx.x] = f[a];
+        }
+    }
+}
+
 // stage: the tile's force buffer in LDS (component c of local node a of lane l
 // at (a*3+c)*kTileElems + l), or null to store the forces to their slots.
 template <typename R, bool kQ, bool kDP, int kHG, bool kMass, int kOps>
@@ -507,7 +848,6 @@ __device__ __forceinline__ void regular_element(const RegElems<R> &E, const Node
     constexpr bool kGeo = kOps == kOpsGeom;
     constexpr bool kLds = kOps == kOpsLds, kCmp = kOps == kOpsCompact || kGeo;
     constexpr int kW = kGeo ? kOpG : (kCmp ? kOpBc : kOpB);
-    constexpr int kNst = kQ ? 12 : 6;  // stress values per element (with the Q memory variables)
     const R *op = nullptr, *pht = nullptr;
     lds_ptr<R> lrow = nullptr, lphr = nullptr;
     if constexpr (kLds) {
@@ -681,83 +1021,8 @@ constexpr int kU1 = (kKeep || kGeo) ? 8 : EQD_PREFETCH;
     }
     const R lam = OPK(kOpLam), miu = OPK(kOpMu);
     const R det = OPK(kOpDet);
-    const R cdiag = lam + (R)2 * miu;
-    R srt[6];
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        R acc = 0;
-#pragma unroll
-        for (int j = 0; j < 3; j++) acc = acc + (i == j ? cdiag : lam) * sr[j];
-        srt[i] = acc;
-    }
-#pragma unroll
-    for (int i = 3; i < 6; i++) srt[i] = miu * sr[i];
-
-    R stress[6], strdev[6];
-#pragma unroll
-    for (int i = 0; i < 6; i++) stress[i] = load_nt(E.stress + blk_at<kNst>(t, i));
-    if (!kQ) {
-#pragma unroll
-        for (int i = 0; i < 6; i++) {
-            stress[i] = stress[i] + srt[i] * (R)C.dt;
-            strdev[i] = stress[i];
-        }
-    } else {
-        const double *q = E.qtab + 6 * E.qidx[t];
-        const R e1 = (R)q[0], e2 = (R)q[1], wkp = (R)q[2], wks = (R)q[3], cv = (R)q[4], cs = (R)q[5];
-        const R miuu = miu * cs;
-        const R Mu = (lam + (R)2 * miu) * cv;
-        const R vols = strain[0] + strain[1] + strain[2];
-        R anestr1[6], anestr[6];
-#pragma unroll
-        for (int i = 0; i < 6; i++) anestr1[i] = load_nt(E.stress + blk_at<kNst>(t, 6 + i));
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-            anestr[i] = e1 * anestr1[i] + e2 * ((R)2 * miuu * strain[i] * wks + (Mu * wkp - (R)2 * miuu * wks) * vols);
-#pragma unroll
-        for (int i = 3; i < 6; i++) anestr[i] = e1 * anestr1[i] + e2 * (miuu * strain[i] * wks);
-#pragma unroll
-        for (int i = 0; i < 6; i++) store_nt(E.stress + blk_at<kNst>(t, 6 + i), anestr[i]);
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-            stress[i] = (R)2 * miuu * strain[i] + (Mu - (R)2 * miuu) * vols - (R)0.5 * (anestr[i] + anestr1[i]);
-#pragma unroll
-        for (int i = 3; i < 6; i++)
-            stress[i] = (R)2 * miuu * strain[i] / (R)2 - (R)0.5 * (anestr[i] + anestr1[i]);
-#pragma unroll
-        for (int i = 0; i < 6; i++) strdev[i] = stress[i];
-    }
-    if (kDP) {
-        // Drucker-Prager viscoplastic return, src/calcElemKU.f90:133-167
-        const R strmea = (stress[0] + stress[1] + stress[2]) / (R)3;
-#pragma unroll
-        for (int i = 0; i < 3; i++) strdev[i] = stress[i] - strmea;
-        R taomax = (R)0.5 * (sqr(strdev[0]) + sqr(strdev[1]) + sqr(strdev[2])) + sqr(strdev[3]) +
-                   sqr(strdev[4]) + sqr(strdev[5]);
-        taomax = sqrt(taomax);
-        R yield = (R)C.ccosphi - (R)C.sinphi * (strmea + (R)E.porep[t]);
-        if (yield < (R)0) yield = 0;
-        R pstrmag = 0;
-        if (taomax > yield) {
-            const R rjust = yield / taomax + ((R)1 - yield / taomax) * (R)C.exp_dt_tv;
-            R pstrinc[6];
-#pragma unroll
-            for (int i = 0; i < 6; i++) {
-                stress[i] = strdev[i] * rjust;
-                pstrinc[i] = (strdev[i] - stress[i]) / miu;
-                if (i < 3) stress[i] = stress[i] + strmea;
-            }
-            const R pstrmea = (pstrinc[0] + pstrinc[1] + pstrinc[2]) / (R)3;
-#pragma unroll
-            for (int i = 0; i < 6; i++) pstrinc[i] = pstrinc[i] - pstrmea;
-            R pm = (R)0.5 * (sqr(pstrinc[0]) + sqr(pstrinc[1]) + sqr(pstrinc[2])) + sqr(pstrinc[3]) +
-                   sqr(pstrinc[4]) + sqr(pstrinc[5]);
-            pstrmag = sqrt(pm);
-        }
-        E.pstrain[t] = E.pstrain[t] + (double)pstrmag;
-    }
-#pragma unroll
-    for (int i = 0; i < 6; i++) store_nt(E.stress + blk_at<kNst>(t, i), stress[i]);
+    R srt[6], stress[6];
+    regular_stress<R, kQ, kDP>(E, C, t, lam, miu, sr, strain, srt, stress);
 
     // f = -m*al (calcElemMass), + (-det*w) * B^T (sigma + rdampk*sigma_dot), - hourglass
     const R temp = -det * (R)C.w;
@@ -906,9 +1171,8 @@ __device__ __forceinline__ void finish_tile(const RegElems<R> &E, const NodeStat
 // shared them (2.42 M elements, FP32: 957 MB fetched against 608, 265 against
 // 221 us), and loads asked for before the barrier took it to 212, FP64 with
 // stored rows (686,000 elements) 124 -> 111.  Element and node kernel of a
-// step together: 686,000 elements FP64 165 -> 138 us; FP32 geometry rows 249
-// -> 274 (bound by their arithmetic) while the fault kernel beside the smaller
-// node kernel ends 60 us earlier.
+// step together: 686,000 elements FP64 165 -> 138 us, 2.42 M FP32 with
+// geometry rows 249 -> 235 (274 before their operators were in modal form).
 template <typename R, bool kQ, bool kDP, int kHG, bool kMass, int kOps>
 __global__ void __launch_bounds__(256, (kOps == kOpsGeom && !kQ && !kDP && !kMass ? EQD_REG_GEO_WAVES : 1))
     elem_regular_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem, int remap, int nstart)
@@ -938,15 +1202,19 @@ __global__ void __launch_bounds__(256, (kOps == kOpsGeom && !kQ && !kDP && !kMas
     }
     if (!E.tile) {
         const int64_t t = (int64_t)b * blockDim.x + threadIdx.x;
-        if (t < E.n) regular_element<R, kQ, kDP, kHG, kMass, kOps>(E, N, C, t, tables, false, stage);
+        if (t >= E.n) return;
+        regular_element<R, kQ, kDP, kHG, kMass, kOps>(E, N, C, t, tables, false, stage);
         return;
     }
     const Tile T = E.tile[b];
     // this step and whether it ends the run (the step start that advances the
     // clock runs in this launch)
     const int nt = M.clk->done + 1, mode = nt == M.clk->run_end ? 1 : 0;
-    if ((int)threadIdx.x < T.ne)
-        regular_element<R, kQ, kDP, kHG, kMass, kOps>(E, N, C, T.e0 + (int)threadIdx.x, tables, true, stage);
+    if ((int)threadIdx.x < T.ne) {
+        const int64_t t = T.e0 + (int)threadIdx.x;
+        if constexpr (kOps == kOpsGeom) regular_element_modal<R, kQ, kDP, kHG, kMass>(E, N, C, t, stage);
+        else regular_element<R, kQ, kDP, kHG, kMass, kOps>(E, N, C, t, tables, true, stage);
+    }
     finish_tile<R>(E, N, T, stage, C.dt, mode, nt + 1);
 }
 

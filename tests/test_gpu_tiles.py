@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from eqdyna_amd.solver import Ensemble, Solver
-from fixtures import load_golden
+from fixtures import channel_errors, channels, load_golden
 from test_gpu_engine import assert_same, outputs
 
 
@@ -33,6 +33,7 @@ def test_tiles_match_reference_order(name, precision, monkeypatch):
     res = []
     for tiles, classes in ((False, "0"), (True, "0"), (False, "1"), (True, "1")):
         monkeypatch.setenv("EQD_NO_OPERATOR_CLASSES", classes)
+        monkeypatch.setenv("EQD_GEOM_OPS", "0")  # operators rebuilt in the kernels: test_modal_operators
         print(f"case {name} {precision} tiles {tiles} per-element operators {classes}", flush=True)
         s, bundle, sc = solver(name, precision, tiles, monkeypatch)
         n = int(sc["nstep"])
@@ -46,6 +47,30 @@ def test_tiles_match_reference_order(name, precision, monkeypatch):
         s.close()
     assert_same(res[1], res[0], f"{name} {precision} tiles")
     assert_same(res[3], res[2], f"{name} {precision} tiles, per-element operators")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["box_rough", "box_q", "box_hg2", "box_plastic", "box_tw"])
+def test_modal_operators(name, monkeypatch):
+    # FP32, operators rebuilt from corner coordinates: tiles form them per mode
+    # (split8, join8), the reference's order node by node.  The two round
+    # differently; both have FP32's bars against the FP64 run: rupture times
+    # within half a step, and every channel within 1e-4 of the other (about a
+    # thousand roundings of 6e-8 that add up over the run)
+    monkeypatch.setenv("EQD_NO_OPERATOR_CLASSES", "1")
+    out = {}
+    for tiles in (False, True):
+        print(f"case {name} tiles {tiles}", flush=True)
+        s, bundle, sc = solver(name, "fp32", tiles, monkeypatch)
+        assert s.layout_info()["geom_ops_regular"] == 1
+        s.run(int(sc["nstep"]))
+        out[tiles] = s.outputs()
+        s.close()
+    d = channel_errors(channels(out[True]), channels(out[False]))
+    worst = max(d, key=d.get)
+    print(f"[{name}] modal against node by node: worst channel {worst} {d[worst]:.2e}", flush=True)
+    assert d[worst] <= 1e-4
+    assert np.max(np.abs(out[True]["fnft"] - out[False]["fnft"])) <= 0.5 * float(sc["dt"])
 
 
 @pytest.mark.gpu
