@@ -197,18 +197,23 @@ def kernel_bytes(bundle, sc, layout: dict, precision: str) -> dict:
                       + forces + int((occ_reg > 0).sum()) * 3 * (nv + nu_r)
                       + inner * (16 + mb + 3 * nv + 3 * (2 * nu_w - nu_r)))
     # PML element: a PML node takes 6 values of its slot, a 3-component node 3
+    pinner, pslots = layout.get("tile_inner_nodes_pml", 0), layout.get("tile_slots_pml", 0)
     pml_slots = int(np.where(ndof[ien[pml]] == 12, 6, 3).sum()) if npl else 0
+    pml_forces = pslots * (6 * r + 2) if layout.get("tiles_pml", 0) else pml_slots * r
+    pml_state = 4 + mb + 3 * mb + 12 * 2 * nv  # node id, mass, damping, split velocities
     out["element_pml"] = (npl * (32 + ops("pml") + 2 * 21 * r + 3 * r + 1 + 6 * r + (24 * r if mass_term else 0))
-                          + pml_slots * r + int((occ_pml > 0).sum()) * 3 * (nv + nu_r))
-    n3, e3 = int(node3.sum()) - inner, int(occ[node3].sum()) - 8 * inner
+                          + pml_forces + int((occ_pml > 0).sum()) * 3 * (nv + nu_r)
+                          + pinner * (12 + pml_state + 3 * nv + 3 * (2 * nu_w - nu_r)))
+    # (an inner node's entries are the ones without a slot)
+    n3, e3 = int(node3.sum()) - inner, int(occ[node3].sum()) - (8 * nr - slots if inner else 0)
     if layout.get("node3_slot_major", 0):
         # node id, mass, state; all 8 entry slots of the slot-major table; the forces
         out["node"] = n3 * (4 + mb + 3 * 2 * nv + 3 * 2 * nu_w + 8 * 4) + e3 * 3 * r
     else:
         out["node"] = n3 * (4 + 4 + mb + 3 * 2 * nv + 3 * 2 * nu_w) + e3 * (4 + 3 * r)
-    npn, ep = int(nodepml.sum()), int(occ[nodepml].sum())
-    out["node_pml"] = (npn * (4 + 4 + mb + 3 * mb + 12 * 2 * nv + 3 * 2 * nv + 3 * 2 * nu_w)
-                       + ep * (4 + 6 * r) + npl * 6 * r)
+    npn, ep = int(nodepml.sum()) - pinner, int(occ[nodepml].sum()) - (8 * npl - pslots if pinner else 0)
+    out["node_pml"] = (npn * (4 + pml_state + 3 * 2 * nv + 3 * 2 * nu_w)
+                       + ep * (4 + 6 * r + (4 if layout.get("tiles_pml", 0) else 0)) + npl * 6 * r)
     return {k: int(v) for k, v in out.items()}
 
 

@@ -444,6 +444,24 @@ static int upload_operators(eqd_handle *h, E &X, int64_t n, bool no_classes, OpR
     return 0;
 }
 
+// a class's tiles on the device (none: X.tile stays null)
+template <typename E>
+static int upload_tiles(eqd_handle *h, E &X, const TileSet &T)
+{
+    X.tile = nullptr;
+    X.n_tile = (int32_t)T.tile.size();
+    if (T.tile.empty()) return 0;
+    Tile *t;
+    uint16_t *ent, *src;
+    int rc;
+    if ((rc = dupload(h, &t, T.tile)) || (rc = dupload(h, &ent, T.node_ent)) || (rc = dupload(h, &src, T.slot_src)))
+        return rc;
+    X.tile = t;
+    X.tile_ent = (const uint4 *)ent;
+    X.tile_src = src;
+    return 0;
+}
+
 template <typename T>
 static void keep_copy(eqd_handle *h, int f, std::map<int, std::vector<T>> &dst)
 {
@@ -662,27 +680,53 @@ int eqd_commit(eqd_handle *h)
     // element entries of every node (rows of the gather table)
     std::vector<int32_t> degree(nn, 0);
     for (int64_t i = 0; i < 8 * ne; i++) degree[ien[i] - 1]++;
-    // Regular elements in tiles whose inner nodes the element kernel updates
-    // itself (elem_regular_kernel), from kTileMinElems elements on;
+    // Elements in tiles whose inner nodes the element kernels update themselves,
+    // from kTileMinElems (kTileMinPml) elements of a class on;
     // EQD_ELEMENT_ORDER=0 keeps the reference's order, 1 makes tiles of any
-    // mesh they fill well.  Split nodes belong to the fault kernel, and a
-    // station's node is read by the step start, which runs in the same launch.
-    TileSet tiles;
+    // mesh.  Split nodes belong to the fault kernel, fixed nodes to none, and a
+    // station's node is read by the step start, which runs beside the regular
+    // elements.
+    TileSet tiles[2];
+    NodeOrder order;
     {
         const char *o = std::getenv("EQD_ELEMENT_ORDER");
-        const bool want = o && (o[0] == '0' || o[0] == '1') ? o[0] == '1' : (int64_t)h->reg_ids.size() >= kTileMinElems;
-        if (want) {
-            std::vector<uint8_t> outer(is_split);
-            const int32_t *idh = s.noff > 0 ? I32(h, EQD_IDHIST) : nullptr;
-            for (int64_t i = 0; i < 6 * (int64_t)s.noff; i++)
-                if (idh[i * 3] >= 1 && idh[i * 3] <= nn) outer[idh[i * 3] - 1] = 1;
-            if (make_tiles(h->reg_ids, ien, nn, degree, outer, tiles)) {
-                h->n_tile = (int32_t)tiles.tile.size();
-                h->at.swap(tiles.at);
-                auto &f = h->node3_free;
-                f.erase(std::remove_if(f.begin(), f.end(), [&](int32_t n) { return tiles.inner[n] != 0; }), f.end());
-            }
+        const bool never = o && o[0] == '0', always = o && o[0] == '1';
+        const bool want[2] = {!never && (always || (int64_t)h->reg_ids.size() >= kTileMinElems),
+                              !never && (always || (int64_t)h->pml_ids.size() >= kTileMinPml)};
+        std::vector<uint8_t> kind(nn, 0);
+        for (int32_t n : h->node3_free) kind[n] = 1;
+        for (int32_t n : h->pml_node_ids) kind[n] = 2;
+        const int32_t *idh = s.noff > 0 ? I32(h, EQD_IDHIST) : nullptr;
+        for (int64_t i = 0; i < 6 * (int64_t)s.noff; i++)
+            if (idh[i * 3] >= 1 && idh[i * 3] <= nn) kind[idh[i * 3] - 1] = 0;
+        std::vector<int32_t> *const ids[2] = {&h->reg_ids, &h->pml_ids};
+        if (make_tiles(ids, want, ien, ne, nn, degree, kind, always ? 0.0 : kTileMinFill, tiles, order)) {
+            h->n_tile = (int32_t)tiles[0].tile.size();
+            h->n_ptile = (int32_t)tiles[1].tile.size();
+            h->at.swap(order.at);
+            auto &f = h->node3_free;
+            f.erase(std::remove_if(f.begin(), f.end(), [&](int32_t n) { return order.inner[n] != 0; }), f.end());
         }
+    }
+    // PML nodes in device order, the tiles' inner ones last
+    h->PN.n_outer = npn - tiles[1].n_inner;
+    if (!h->at.empty() && npn > 0) {
+        std::vector<int32_t> q;
+        q.reserve(npn);
+        for (int in = 0; in < 2; in++)
+            for (int32_t n : order.ref)
+                if (h->pml_node_index[n] >= 0 && order.inner[n] == in) q.push_back(h->pml_node_index[n]);
+        auto &id = h->pml_node_ids;
+        auto take = [&](auto &v, int w) {  // component-major
+            auto old = v;
+            for (int k = 0; k < w; k++)
+                for (int64_t i = 0; i < npn; i++) v[k * npn + i] = old[k * npn + q[i]];
+        };
+        take(id, 1);
+        take(pv12, 12);
+        take(pacc, 12);
+        take(pdamp, 3);
+        for (int64_t i = 0; i < npn; i++) h->pml_node_index[id[i]] = (int32_t)i;
     }
     // a node's place on the device, and per-node arrays (component-major, in
     // the reference's order) in that order and in blocks
@@ -703,7 +747,7 @@ int eqd_commit(eqd_handle *h)
     std::sort(n3free.begin(), n3free.end());
     std::sort(n3all.begin(), n3all.end());
     const int64_t nr = (int64_t)h->reg_ids.size(), np = (int64_t)h->pml_ids.size();
-    if (nr > (int64_t)kEntIdxMask || np > (int64_t)kEntIdxMask) return fail(h, EQD_EINVAL, "too many elements in one class");
+    if (8 * (nr + 64) >= (int64_t)kEntSlotMask || 8 * (np + 64) >= (int64_t)kEntSlotMask) return fail(h, EQD_EINVAL, "too many elements in one class");
     h->n_reg = (int32_t)nr;
     h->n_pml = (int32_t)np;
     const bool fp32 = s.precision == EQD_PREC_FP32;
@@ -831,22 +875,10 @@ int eqd_commit(eqd_handle *h)
             R *p;
             if ((r2 = dupload(h, &p, to_blocks<R>(r_st, nr, nst)))) return r2;
             E.stress = p;
-            // force slots: the tiles', or 8 per element
-            const int64_t slots = h->n_tile ? (int64_t)tiles.slot_src.size() : blocked_count(nr, 8);
-            h->n_slot = h->n_tile ? slots : 0;
-            if ((r2 = dalloc(h, &p, slots * 3))) return r2;
+            h->n_slot = h->n_tile ? (int64_t)tiles[0].slot_src.size() : 0;
+            if ((r2 = dalloc(h, &p, 3 * (h->n_tile ? h->n_slot : blocked_count(nr, 8))))) return r2;
             E.ef = p;
-            if (h->n_tile) {
-                Tile *tp;
-                uint16_t *ep, *sp;
-                if ((r2 = dupload(h, &tp, tiles.tile)) || (r2 = dupload(h, &ep, tiles.node_ent)) ||
-                    (r2 = dupload(h, &sp, tiles.slot_src)))
-                    return r2;
-                E.tile = tp;
-                E.n_tile = h->n_tile;
-                E.tile_ent = (const uint4 *)ep;
-                E.tile_src = sp;
-            }
+            if ((r2 = upload_tiles(h, E, tiles[0]))) return r2;
             E.porep = d_porep;
             E.pstrain = d_pstrain;
             E.qidx = d_q;
@@ -945,8 +977,13 @@ int eqd_commit(eqd_handle *h)
             R *q;
             if ((r2 = dupload(h, &q, to_blocks<R>(p_st, np, 21)))) return r2;
             P.stress = q;
-            if ((r2 = dalloc(h, &q, blocked_count(np, kEfPml)))) return r2;
+            h->n_pslot = h->n_ptile ? (int64_t)tiles[1].slot_src.size() : 0;
+            const int64_t slots = h->n_ptile ? h->n_pslot : blocked_count(np, 8);
+            if ((r2 = dalloc(h, &q, 3 * slots))) return r2;
             P.ef = q;
+            if ((r2 = dalloc(h, &q, 3 * slots))) return r2;
+            P.ef2 = q;
+            if ((r2 = upload_tiles(h, P, tiles[1]))) return r2;
             if ((r2 = dalloc(h, &q, blocked_count(np, 6)))) return r2;
             P.ssum = q;
             return 0;
@@ -964,20 +1001,23 @@ int eqd_commit(eqd_handle *h)
         for (int64_t t = 0; t < nr; t++) cls_index[h->reg_ids[t]] = (int32_t)t;
         for (int64_t p = 0; p < np; p++) cls_index[h->pml_ids[p]] = (int32_t)p;
         // (a tile's inner nodes have no row: the element kernel sums them)
-        auto inner = [&](int64_t n) { return h->n_tile && tiles.inner[n]; };
+        auto inner = [&](int64_t n) { return !h->at.empty() && order.inner[n]; };
         std::vector<int32_t> rowptr(nn + 1, 0);
         for (int64_t n = 0; n < nn; n++) rowptr[at(n) + 1] = inner(n) ? 0 : degree[n];
         for (int64_t i = 0; i < nn; i++) rowptr[i + 1] += rowptr[i];
         std::vector<int32_t> fillp(rowptr.begin(), rowptr.end() - 1);
         std::vector<uint32_t> ent(rowptr[nn]);
+        std::vector<int32_t> ent_el(h->n_ptile ? rowptr[nn] : 0);
         for (int64_t e = 0; e < ne; e++) {
             const bool pml = etype[e] == 2;
             const int64_t t = cls_index[e];
+            const TileSet &T = tiles[pml ? 1 : 0];
             for (int a = 0; a < 8; a++) {
                 const int32_t nd = ien[e * 8 + a] - 1;
                 if (inner(nd)) continue;
-                ent[fillp[at(nd)]++] = pml ? kEntPml | ((uint32_t)a << kEntLocalShift) | (uint32_t)t
-                                       : (h->n_tile ? tiles.slot_of[t * 8 + a] : (uint32_t)reg_slot(t, a));
+                const int32_t j = fillp[at(nd)]++;
+                ent[j] = (pml ? kEntPml : 0u) | (T.tile.empty() ? (uint32_t)elem_slot(t, a) : T.slot_of[t * 8 + a]);
+                if (h->n_ptile) ent_el[j] = (int32_t)t;
             }
         }
         for (int64_t q = 0; q < npn; q++) {
@@ -992,6 +1032,9 @@ int eqd_commit(eqd_handle *h)
         if ((rc = dupload(h, &d_ent, ent))) return rc;
         h->N.rowptr = d_rp;
         h->N.ent = d_ent;
+        int32_t *d_el;
+        if ((rc = dupload(h, &d_el, ent_el))) return rc;
+        h->N.ent_el = d_el;
         // the free 3-component nodes' entries again, slot-major by position,
         // so that a wavefront's load of slot k reads consecutive words
         // (EQD_NODE_ELL=0 keeps the CSR gather)
@@ -1045,10 +1088,10 @@ int eqd_commit(eqd_handle *h)
         std::vector<double> mass_at(nn);
         for (int64_t n = 0; n < nn; n++) mass_at[at(n)] = mass[n];
         if ((rc = dupload(h, &d, mass_at))) return rc; h->N.mass = d;
-        if (h->n_tile) {
+        if (!h->at.empty()) {
             int32_t *ip;
             if ((rc = dupload(h, &ip, h->at))) return rc; h->N.at = ip;
-            if ((rc = dupload(h, &ip, tiles.ref))) return rc; h->N.ref = ip;
+            if ((rc = dupload(h, &ip, order.ref))) return rc; h->N.ref = ip;
         }
         unsigned long long *fl;
         if ((rc = dalloc(h, &fl, 1))) return rc;
@@ -1727,6 +1770,9 @@ int eqd_layout_info(eqd_handle *h, const char *key, int64_t *value)
     else if (k == "tiles") *value = h->n_tile;
     else if (k == "tile_inner_nodes") *value = (int64_t)h->node3_all.size() - 2 * h->F.nf - (int64_t)h->node3_free.size();
     else if (k == "tile_slots") *value = h->n_slot;
+    else if (k == "tiles_pml") *value = h->n_ptile;
+    else if (k == "tile_inner_nodes_pml") *value = h->PN.n - h->PN.n_outer;
+    else if (k == "tile_slots_pml") *value = h->n_pslot;
     else if (k == "node3_slot_major") *value = h->d_ell3 ? 1 : 0;
     else return fail(h, EQD_EINVAL, "unknown layout key %s", key);
     return EQD_OK;

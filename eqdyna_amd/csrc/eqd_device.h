@@ -22,13 +22,10 @@
 
 namespace eqd {
 
-// CSR entry: bit 31 = PML element, with local node a in bits 28..30 and the
-// element's index within its class in bits 0..27; else a regular element's
-// force slot (reg_slot, or its tile's) in bits 0..30.
+// CSR entry: bit 31 = PML element, bits 0..30 = the slot of the element's force
+// on the node in its class (elem_slot, or its tile's).
 constexpr uint32_t kEntPml = 0x80000000u;
-constexpr uint32_t kEntIdxMask = 0x0FFFFFFFu;
 constexpr uint32_t kEntSlotMask = 0x7FFFFFFFu;
-constexpr int kEntLocalShift = 28;
 constexpr uint32_t kEntNone = 0xFFFFFFFFu;  // an unused slot of the ELL gather table
 constexpr int kEll3 = 8;
 // values recorded per step for a hypocentre pair (showSourceDynamics,
@@ -65,6 +62,7 @@ struct NodeState {
     const float *mass32;   // [nn] the same rounded to FP32, read by the FP32 bulk mode's node kernels
     const int32_t *rowptr; // [nn+1]
     const uint32_t *ent;   // CSR entries
+    const int32_t *ent_el; // and each entry's element in its class, where the PML elements run in tiles (else null)
     // where the elements run in tiles the nodes are stored tile by tile (TileSet):
     // the reference's node n at at[n], ref its inverse; else null, in its order
     const int32_t *at, *ref;
@@ -103,14 +101,14 @@ __host__ __device__ __forceinline__ int64_t blk_at(int64_t t, int s)
     return ((t >> 6) * W + s) * 64 + (t & 63);
 }
 
-// The FP64 PML elements' node slots and summed stresses are read in pairs:
+// The FP64 PML elements' summed stresses are read in pairs:
 // values 2j and 2j+1 of item t sit side by side, so one lane loads or stores
 // both at once (16 bytes) and a wavefront's access to a pair is one
 // contiguous run of 128 values (W even; the same footprint as blk_at<W>).
 // c4 FP64 PML element kernel 0.288 -> 0.252 ms, step 1.006 -> 0.966 ms; in
 // FP32 (8-byte pairs) the same layout measured no faster on c4 and 1.4 %
 // slower on the 64-scenario ensemble, so the FP32 mode keeps blk_at.
-// The regular elements' forces on their nodes, component c of force slot s:
+// The elements' forces on their nodes, component c of force slot s:
 // FP64 keeps x and y of a slot as a 16-byte pair and z apart, so a node's
 // force is one paired and one single access; FP32 keeps blk_at<3>.  Both fill
 // 3 rows of 64 values per 64 slots.
@@ -124,8 +122,10 @@ __host__ __device__ __forceinline__ int64_t slot_at(int64_t s, int c)
         return blk_at<3>(s, c);
     }
 }
-// slot of element t's force on local node a where the elements run in no tiles
-__host__ __device__ __forceinline__ int64_t reg_slot(int64_t t, int a) { return blk_at<8>(t, a); }
+// slot of element t's force on local node a where its class runs in no tiles, and
+// the element of such a slot
+__host__ __device__ __forceinline__ int64_t elem_slot(int64_t t, int a) { return blk_at<8>(t, a); }
+__host__ __device__ __forceinline__ int64_t slot_elem(int64_t s) { return (s >> 9) * 64 + (s & 63); }
 
 template <typename R, int W>
 __host__ __device__ __forceinline__ int64_t pml_at(int64_t t, int s)
@@ -133,7 +133,6 @@ __host__ __device__ __forceinline__ int64_t pml_at(int64_t t, int s)
     if constexpr (sizeof(R) == sizeof(double)) return ((t >> 6) * W + (s & ~1)) * 64 + (t & 63) * 2 + (s & 1);
     else return blk_at<W>(t, s);
 }
-constexpr int kEfPml = 48;
 
 // Where an element kernel finds its operators: class tables in global memory
 // or per-element rows with Phi; class tables staged in LDS; per-element rows
@@ -160,7 +159,7 @@ __host__ __device__ __forceinline__ R phi_compact(const R *c, int m, int a, R s0
     return r - h;
 }
 
-// One tile: elements [e0, e0 + ne) of the regular class, one workgroup.  Its
+// One tile: elements [e0, e0 + ne) of a class, one workgroup.  Its
 // inner nodes, the ones that no element outside the tile touches, are nodes
 // [n0, n0 + nn) with 8 entries each at tile_ent + i0, and the forces on its
 // other nodes leave through slots [64 s0, 64 s0 + ns) of ef in the order of
@@ -168,6 +167,8 @@ __host__ __device__ __forceinline__ R phi_compact(const R *c, int m, int a, R s0
 // lane.
 constexpr int kTileElems = 256;
 constexpr uint16_t kTileNone = 0xFFFFu;
+// values a PML element stages at a time: 3 per local node and its 6 summed stresses
+constexpr int kPmlStage = 30;
 struct Tile {
     int32_t e0, ne, n0, nn, i0, s0, ns;
 };
@@ -210,10 +211,13 @@ struct PmlElems {
     const R *emass;        // 24 per element (blk_at<24>)
     const R *damp;         // 3 per element (blk_at<3>): element-centre damping d_x, d_y, d_z
     const uint8_t *mask12; // [n] bit a: local node a carries 12 components
-    R *ef;                 // 6 slots per local node a (blk_at<kEfPml>, slot a*6+k): a 3-component
-                           // node's force at k = 0..2; a 12-component node's det*w*dN_a/dx at
-                           // k = 0..2 (its 9 split forces follow from ssum) and force
-                           // components 10-12 at k = 3..5
+    const Tile *tile;      // as in RegElems
+    int32_t n_tile;
+    const uint4 *tile_ent;
+    const uint16_t *tile_src;
+    R *ef, *ef2;           // forces on the nodes (slot_at): a 3-component node's force in ef; a
+                           // 12-component node's det*w*dN_a/dx in ef (its 9 split forces follow
+                           // from ssum) and force components 10-12 in ef2
     R *ssum;               // 6 per element (blk_at<6>): summed stresses xx, yy, zz, xy, xz, yz
     // operators as in RegElems
     const uint32_t *opc;
@@ -228,6 +232,7 @@ struct PmlElems {
 
 struct PmlNodes {
     int64_t n;
+    int64_t n_outer;      // the first n_outer are no inner nodes of a tile; these follow tile by tile
     const int32_t *node;  // [n]
     const double *damp;   // 3 per node (blk_at<3>): d_x, d_y, d_z at the node
     const float *damp32;  // the same rounded to FP32, read by the FP32 bulk mode

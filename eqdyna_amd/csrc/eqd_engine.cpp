@@ -65,10 +65,10 @@ int64_t count_of(const eqd_handle *h, int kind)
 {
     switch (kind) {
     case kKElem: return h->n_tile ? (int64_t)h->n_tile * kTileElems : h->n_reg;
-    case kKPml: return h->n_pml;
+    case kKPml: return h->n_ptile ? (int64_t)h->n_ptile * kTileElems : h->n_pml;
     // a scenario with tiles always has a block: it tells the next step's element kernel its step (Clock::done)
     case kKNode3: return std::max<int64_t>((int64_t)h->node3_free.size(), h->n_tile ? 1 : 0);
-    case kKNodePml: return h->PN.n;
+    case kKNodePml: return h->PN.n_outer;
     case kKFault: return h->F.nf;
     case kKStation: return 0;  // the step start: its own launch or blocks of the first element launch
     case kKPend3: return (int64_t)h->node3_all.size();
@@ -114,7 +114,9 @@ int variant(const eqd_handle *h, int kind, size_t *lds)
     }
     if (kind == kKPml) {
         *lds = class_lds(pmls<R>(h), sizeof(R));
-        return hg | mass << 2 | ops_of(pmls<R>(h), *lds) << 3;
+        const int ops = ops_of(pmls<R>(h), *lds);
+        if (h->n_ptile) *lds += kPmlStage * kTileElems * sizeof(R);
+        return hg | mass << 2 | ops << 3 | (h->n_ptile ? 1 : 0) << 5;
     }
     if (kind == kKFault) return h->learn ? 1 : 0;
     return 0;
@@ -172,9 +174,9 @@ int build(eqd_engine *e)
             int64_t blocks = 0;
             // a tile is one workgroup, whatever shape the scenarios without tiles would run in
             int block = tuned;
-            if (kind == kKElem)
+            if (kind == kKElem || kind == kKPml)
                 for (int m : g.members)
-                    if (e->hs[m]->n_tile) block = kTileElems;
+                    if (kind == kKElem ? e->hs[m]->n_tile : e->hs[m]->n_ptile) block = kTileElems;
             for (int m : g.members) {
                 M[m].blk0[kind] = (int32_t)blocks;
                 blocks += (count_of(e->hs[m], kind) + block - 1) / block;
@@ -296,7 +298,7 @@ int enqueue_step(eqd_engine *e)
         const Stamp p = take_timer(e, kKPml, gs.size());
         for (size_t i = 0; i < gs.size(); i++) {
             const Group &g = gs[i];
-            HIPCHK(e, launch_pml<R>(dM, g.g, g.sig & 3, (g.sig >> 2) & 1, (g.sig >> 3) & 3, st, p.start(i),
+            HIPCHK(e, launch_pml<R>(dM, g.g, g.sig & 3, (g.sig >> 2) & 1, (g.sig >> 3) & 3, g.sig >> 5, st, p.start(i),
                                     p.stop(i)));
         }
     }

@@ -19,7 +19,7 @@ template <typename R>
 hipError_t launch_elem(const Member<R> *, const LaunchGrid &, int q, int dp, int hg, int mass, int ops, int nstart,
                        hipStream_t, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
 template <typename R>
-hipError_t launch_pml(const Member<R> *, const LaunchGrid &, int hg, int mass, int ops, hipStream_t,
+hipError_t launch_pml(const Member<R> *, const LaunchGrid &, int hg, int mass, int ops, int tiled, hipStream_t,
                       hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
 template <typename R>
 hipError_t launch_node3(const Member<R> *, const LaunchGrid &, hipStream_t, hipEvent_t t0 = nullptr,
@@ -142,6 +142,8 @@ struct eqd_handle {
     std::vector<int32_t> at;  // with tiles: a node's place on the device (NodeState::at), else empty
     int32_t n_tile = 0;  // tiles of the regular elements (0: none)
     int64_t n_slot = 0;  // and their force slots
+    int32_t n_ptile = 0;  // the same of the PML elements
+    int64_t n_pslot = 0;
     std::vector<int32_t> hyp_pairs;  // pairs (0-based) at the hypocentre, in pair order
     // device objects
     eqd::NodeState N{};

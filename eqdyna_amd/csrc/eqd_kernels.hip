@@ -80,6 +80,20 @@ __device__ __forceinline__ void load_pair(const R *p, R &a, R &b)
     }
 }
 
+// the three values of a force slot
+template <typename R>
+__device__ __forceinline__ void store3_nt(R *ef, int64_t slot, R x, R y, R z)
+{
+    store_pair_nt(ef + slot_at<R>(slot, 0), x, y);
+    store_nt(ef + slot_at<R>(slot, 2), z);
+}
+template <typename R>
+__device__ __forceinline__ void load3(const R *ef, int64_t slot, R &x, R &y, R &z)
+{
+    load_pair(ef + slot_at<R>(slot, 0), x, y);
+    z = ef[slot_at<R>(slot, 2)];
+}
+
 // The element kernels' other once-per-step streams (IEN, stresses, operator
 // rows) are loaded non-temporal for the same reason: c4 FP32 step 0.688 ->
 // 0.664 ms, FP64 3.2 % faster, c2 FP32 1.1 %.
@@ -295,10 +309,9 @@ __device__ __forceinline__ void geo_ops(const R *opb, int64_t t, R lam, R mu, Ge
 // instead of 2,300 node by node.  Fused multiply-adds allowed (each rounds once
 // where two operations round twice).
 //
-// Used by the regular elements of tiles, where the node-by-node form is bound
-// by its arithmetic (145 of 212 us for 2.42 M elements; this one takes 176 and
-// is bound by memory, 5.1 TB/s).  The PML elements are bound by memory in
-// either form (117 and 118 us for 1.04 M).  Error of velocity and displacement
+// Used by the elements of tiles, where the node-by-node form is bound by its
+// arithmetic (regular: 145 of 212 us for 2.42 M elements; this one takes 176 and
+// is bound by memory, 5.1 TB/s; PML: 147 and 130 us for 1.04 M).  Error of velocity and displacement
 // against FP64, rough-fault boxes of 60,000 to 350,000 elements: 4.49e-7 and
 // 1.32e-7 node by node, 4.41e-7 and 1.29e-7 here; in boxes of a few thousand
 // elements, where neither form matters to the time, the displacement's was
@@ -349,10 +362,25 @@ __device__ __forceinline__ void join8(const R lin[3], const R hg[4], R f[8])
     }
 }
 
+// f_a = sum_l ac_al l_l
+template <typename R>
+__device__ __forceinline__ void join3(R l0, R l1, R l2, R f[8])
+{
+    const R p = l0 + l1, m = l0 - l1;
+    f[0] = -p - l2;
+    f[1] = m - l2;
+    f[2] = p - l2;
+    f[3] = -m - l2;
+    f[4] = l2 - p;
+    f[5] = m + l2;
+    f[6] = p + l2;
+    f[7] = l2 - m;
+}
+
 // from the coordinates of local nodes 1..7 relative to node 0, so the values
 // are rounded relative to the element's size
 template <typename R>
-__device__ __forceinline__ void modal_ops(const R *opb, int64_t t, R lam, R mu, ModalOps<R> &G)
+__device__ __forceinline__ void modal_ops(const R xc[21], R lam, R mu, ModalOps<R> &G)
 {
 #pragma clang fp contract(fast)
     R a[3][3], b[4][3];  // a[l][j] = d x_j / d xi_l, b[m][j] = sum_b Gamma_mb x_bj
@@ -361,7 +389,7 @@ __device__ __forceinline__ void modal_ops(const R *opb, int64_t t, R lam, R mu, 
         R x[8], lin[3], hg[4];
         x[0] = 0;
 #pragma unroll
-        for (int k = 1; k < 8; k++) x[k] = opb_at<R, kOpG>(opb, t, (k - 1) * 3 + j);
+        for (int k = 1; k < 8; k++) x[k] = xc[(k - 1) * 3 + j];
         split8<R>(x, lin, hg);
 #pragma unroll
         for (int l = 0; l < 3; l++) a[l][j] = lin[l] * (R)0.125;
@@ -750,9 +778,12 @@ __device__ __forceinline__ void regular_element_modal(const RegElems<R> &E, cons
     int nds[8];
 #pragma unroll
     for (int a = 0; a < 8; a++) nds[a] = load_nt(E.ien + blk_at<8>(t, a));
-    const R lam = opb_at<R, kOpG>(E.opb, t, kGeoMat), miu = opb_at<R, kOpG>(E.opb, t, kGeoMat + 1);
+    R xc[kGeoMat + 2];
+#pragma unroll
+    for (int i = 0; i < kGeoMat + 2; i++) xc[i] = opb_at<R, kOpG>(E.opb, t, i);
+    const R lam = xc[kGeoMat], miu = xc[kGeoMat + 1];
     ModalOps<R> G;
-    modal_ops<R>(E.opb, t, lam, miu, G);
+    modal_ops<R>(xc, lam, miu, G);
     const R rdk = (R)C.rdampk;
     // modal sums of velocity and displacement relative to the first node (the
     // arithmetic then rounds relative to the deformation, not to the absolute
@@ -1097,9 +1128,7 @@ constexpr int kU2 = (kKeep || kGeo) ? 8 : EQD_ELEM_UNROLL;
 #pragma unroll
             for (int k = 0; k < 3; k++) stage[(a * 3 + k) * kTileElems + threadIdx.x] = f[k];
         } else {
-            const int64_t slot = reg_slot(t, a);
-            store_pair_nt(E.ef + slot_at<R>(slot, 0), f[0], f[1]);
-            store_nt(E.ef + slot_at<R>(slot, 2), f[2]);
+            store3_nt(E.ef, elem_slot(t, a), f[0], f[1], f[2]);
         }
         if constexpr (!kLds && !kKeep) {
 #pragma unroll
@@ -1135,8 +1164,7 @@ __device__ __forceinline__ void finish_tile(const RegElems<R> &E, const NodeStat
     auto send = [&](unsigned e, int64_t slot) {
         if (e == kTileNone) return;
         const unsigned at = (e / kTileElems) * 3 * kTileElems + e % kTileElems;
-        store_pair_nt(E.ef + slot_at<R>(slot, 0), stage[at], stage[at + kTileElems]);
-        store_nt(E.ef + slot_at<R>(slot, 2), stage[at + 2 * kTileElems]);
+        store3_nt<R>(E.ef, slot, stage[at], stage[at + kTileElems], stage[at + 2 * kTileElems]);
     };
 #pragma unroll
     for (int i = 0; i < kAhead; i++) send(src[i], s0 + i * kTileElems);
@@ -1218,6 +1246,54 @@ __global__ void __launch_bounds__(256, (kOps == kOpsGeom && !kQ && !kDP && !kMas
     finish_tile<R>(E, N, T, stage, C.dt, mode, nt + 1);
 }
 
+// mass, damping, split velocities and displacement of a 12-component node
+struct NodePml {
+    double m, d[3], v[12], u[3];
+};
+template <typename R>
+__device__ __forceinline__ void node_pml_load(const NodeState &N, const PmlNodes &P, int64_t q, int node, NodePml &S)
+{
+    S.m = node_mass<R>(N, node);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        S.d[k] = pml_damp<R>(P, q, k);
+        S.u[k] = node_u<R>(N, node, k);
+    }
+#pragma unroll
+    for (int k = 0; k < 12; k++) S.v[k] = pml_v<R>(P, q, k);
+}
+
+// Assembled force F of a 12-component node to its new state (node3_update's
+// modes); src/driver.f90:107-141 for the damped split update.
+template <typename R>
+__device__ __forceinline__ void node_pml_update(const NodeState &N, const PmlNodes &P, int64_t q, int node,
+                                                const NodePml &S, const double F[12], double dt, int mode,
+                                                int next_step)
+{
+    if (mode == 1) {
+#pragma unroll
+        for (int k = 0; k < 12; k++) P.acc[blk_at<12>(q, k)] = F[k] / S.m;
+        return;
+    }
+    double v[12];
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const double dv = S.d[k % 3];
+        v[k] = (F[k] / S.m + S.v[k] * (1.0 / dt - dv / 2.0)) / (1.0 / dt + dv / 2.0);
+    }
+#pragma unroll
+    for (int k = 9; k < 12; k++) v[k] = S.v[k] + F[k] / S.m * dt;
+#pragma unroll
+    for (int k = 0; k < 12; k++) pml_store<R>(P, q, k, v[k]);
+    double vel[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        vel[k] = v[3 * k] + v[3 * k + 1] + v[3 * k + 2] + v[9 + k];
+        node_store<R>(N, node, k, vel[k], S.u[k] + vel[k] * dt);
+    }
+    flag_nan(N, node, next_step, vel[0], vel[1], vel[2]);
+}
+
 // ------------------------------------------------------------------------
 // PML elements: calcPMLElemKU + calcElemMass + hrglss, one element per thread.
 //   src/assembleGlobalKU.f90:36-64, 70-346; src/hrglss.f90
@@ -1228,38 +1304,25 @@ __global__ void __launch_bounds__(256, (kOps == kOpsGeom && !kQ && !kDP && !kMas
 // At least 3 waves per SIMD in FP64 (4 in FP32): caps the FP64 per-element
 // variant at 168 VGPRs without spills (it would take 176, leaving 2 waves);
 // measured 0.324 -> 0.307 ms on the rough-fault box.
-template <typename R, int kHG, bool kMass, int kOps>
-__global__ void __launch_bounds__(256, (sizeof(R) == 8 ? 3 : (kOps == kOpsGeom ? EQD_PML_GEO_WAVES : 4)))
-    elem_pml_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem, int remap)
+// kTile: the forces are staged in LDS (component c of local node a of lane l at
+// (a*3+c)*kTileElems + l, the six summed stresses behind them) and components
+// 10-12 of the nodes returned in d, to be staged once the others are used.
+template <typename R, int kHG, bool kMass, int kOps, bool kTile>
+__device__ __forceinline__ void pml_element(const PmlElems<R> &E, const NodeState &N, const StepConsts &C, int64_t p,
+                                            lds_ptr<R> tables, lds_ptr<R> stage, R d[kTile ? 24 : 1])
 {
     constexpr bool kGeo = kOps == kOpsGeom;
     constexpr bool kLds = kOps == kOpsLds, kCmp = kOps == kOpsCompact || kGeo;
     constexpr int kW = kGeo ? kOpG : (kCmp ? kOpBc : kOpB);
-    extern __shared__ __attribute__((aligned(16))) unsigned char eqd_smem[];
-    typedef __attribute__((address_space(3))) R lds_R;
-    const unsigned gb = launch_block(remap);
-    const Member<R> &M = Ms[member_of(bmem, gb)];
-    const PmlElems<R> E = M.P;
-    const NodeState N = M.N;
-    const StepConsts C = M.C;
-    const int64_t p = (int64_t)(gb - (unsigned)M.blk0[kKPml]) * blockDim.x + threadIdx.x;
     const R *op = nullptr, *pht = nullptr;
-    const lds_R *lrow = nullptr, *lphr = nullptr;
+    lds_ptr<R> lrow = nullptr, lphr = nullptr;
     if constexpr (kLds) {
-        // class tables staged in LDS, as in elem_regular_kernel
-        lds_R *lop = (lds_R *)eqd_smem, *lph = lop + E.n_opc * kOpW;
-        for (int j = threadIdx.x; j < E.n_opc * kOpW; j += blockDim.x) lop[j] = E.optab[j];
-        for (int j = threadIdx.x; j < E.n_phic * 32; j += blockDim.x) lph[j] = E.phitab[j];
-        __syncthreads();
-        if (p >= E.n) return;
-        lrow = lop + (int64_t)E.opc[p] * kOpW;
-        lphr = lph + (int64_t)E.phic[p] * 32;
+        lrow = tables + (int64_t)E.opc[p] * kOpW;
+        lphr = tables + E.n_opc * kOpW + (int64_t)E.phic[p] * 32;
     } else {
-        if (p >= E.n) return;
         op = E.optab ? E.optab + (int64_t)E.opc[p] * kOpW : nullptr;
         pht = E.phitab ? E.phitab + (int64_t)E.phic[p] * 32 : nullptr;
     }
-    const int64_t n = E.n, nn = N.nn;
     constexpr bool kF64 = sizeof(R) == sizeof(double);
     GeoOps<R> geo;
     if constexpr (kGeo)
@@ -1300,6 +1363,17 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 8 ? 3 : (kOps == kOpsGeom ?
     int nds[8];
 #pragma unroll
     for (int a = 0; a < 8; a++) nds[a] = load_nt(E.ien + blk_at<8>(p, a));
+    // in tiles, whose waves wait together and few of which share a SIMD, the
+    // stresses are asked for ahead too
+    R old[kTile ? 21 : 1];
+    if constexpr (kTile) {
+#pragma unroll
+        for (int i = 0; i < 21; i++) old[i] = load_nt(E.stress + blk_at<21>(p, i));
+    }
+    auto old_stress = [&](int i) -> R {
+        if constexpr (kTile) return old[i];
+        else return load_nt(E.stress + blk_at<21>(p, i));
+    };
     constexpr int P = EQD_PREFETCH;
     R vq[P][3], uq[P][3];
 #pragma unroll
@@ -1343,8 +1417,7 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 8 ? 3 : (kOps == kOpsGeom ?
     constexpr bool kKeep = !kLds && !kGeo && (EQD_KEEP_OPS_PML == 2 || (EQD_KEEP_OPS_PML == 1 && sizeof(R) == sizeof(float)));
     constexpr bool kStage = !kLds && !kKeep && !kGeo && EQD_STAGE_SHP_PML;
     constexpr int kNk = kCmp ? 3 : kNo;
-    lds_R *stage = (lds_R *)eqd_smem;
-    const unsigned bd = blockDim.x, tx = threadIdx.x;
+    const unsigned bd = kTile ? kTileElems : blockDim.x, tx = threadIdx.x;
     // the force pass's operator values: dN/dx from the stage, Phi from memory
     // (or rebuilt from the compact operators)
     auto load_op2 = [&](int a, R o[kNo]) {
@@ -1459,7 +1532,7 @@ constexpr int kU1 = (kKeep || kGeo) ? 8 : EQD_PREFETCH;
 #pragma unroll
     for (int c = 0; c < 15; c++) {
         const R dd = dir[c] == 0 ? d0 : (dir[c] == 1 ? d1 : d2);
-        R sc = load_nt(E.stress + blk_at<21>(p, c));
+        R sc = old_stress(c);
         sc = coef[c] * grad[c] + ((R)1 / dt - dd / (R)2) * sc;
         sc = sc / ((R)1 / dt + dd / (R)2);
         sv[c] = sc;
@@ -1475,9 +1548,14 @@ constexpr int kU1 = (kKeep || kGeo) ? 8 : EQD_PREFETCH;
     store_pair(E.ssum + pml_at<R, 6>(p, 0), sxx, syy);
     store_pair(E.ssum + pml_at<R, 6>(p, 2), szz, sxy);
     store_pair(E.ssum + pml_at<R, 6>(p, 4), sxz, syz);
+    if constexpr (kTile) {
+        const R sum[6] = {sxx, syy, szz, sxy, sxz, syz};
+#pragma unroll
+        for (int c = 0; c < 6; c++) stage[(24 + c) * kTileElems + tx] = sum[c];
+    }
     R s0[6];
 #pragma unroll
-    for (int k = 0; k < 6; k++) s0[k] = load_nt(E.stress + blk_at<21>(p, 15 + k)) + (R)C.rdampk * srt[k];
+    for (int k = 0; k < 6; k++) s0[k] = old_stress(15 + k) + (R)C.rdampk * srt[k];
     const R dw = det * (R)C.w;
     const unsigned mask = E.mask12[p];
     R g[4][3];
@@ -1498,7 +1576,7 @@ constexpr int kU1 = (kKeep || kGeo) ? 8 : EQD_PREFETCH;
     }
 
     if constexpr (!kLds && !kKeep) load_op2(0, opc_);
-constexpr int kU2 = (kKeep || kGeo) ? 8 : EQD_ELEM_UNROLL;
+constexpr int kU2 = (kKeep || kGeo || kTile) ? 8 : EQD_ELEM_UNROLL;
 #pragma unroll kU2
     for (int a = 0; a < 8; a++) {
         if constexpr (kLds) {
@@ -1556,23 +1634,324 @@ constexpr int kU2 = (kKeep || kGeo) ? 8 : EQD_ELEM_UNROLL;
         f[9] = f[9] - dw * (g1 * s0[0] + g3 * s0[4] + g2 * s0[5]);
         f[10] = f[10] - dw * (g2 * s0[1] + g3 * s0[3] + g1 * s0[5]);
         f[11] = f[11] - dw * (g3 * s0[2] + g2 * s0[3] + g1 * s0[4]);
+        R o[3];
         if (mask & (1u << a)) {
             // a PML node: its 9 split components are (0 - (dw g_i) s_j) with
             // the summed stresses stored above, so the node kernel forms them
             // from dw g (3 values) bit for bit; 10-12 are stored whole
-            store_pair_nt(E.ef + pml_at<R, kEfPml>(p, a * 6 + 0), dw * g1, dw * g2);
-            store_pair_nt(E.ef + pml_at<R, kEfPml>(p, a * 6 + 2), dw * g3, f[9] + hg[0]);
-            store_pair_nt(E.ef + pml_at<R, kEfPml>(p, a * 6 + 4), f[10] + hg[1], f[11] + hg[2]);
+            o[0] = dw * g1, o[1] = dw * g2, o[2] = dw * g3;
         } else {
             // a 3-component node takes the collapsed sums (src/assembleGlobalKU.f90:55-61)
-            store_pair_nt(E.ef + pml_at<R, kEfPml>(p, a * 6 + 0), f[0] + f[1] + f[2] + f[9] + hg[0],
-                          f[3] + f[4] + f[5] + f[10] + hg[1]);
-            store_nt(E.ef + pml_at<R, kEfPml>(p, a * 6 + 2), f[6] + f[7] + f[8] + f[11] + hg[2]);
+            o[0] = f[0] + f[1] + f[2] + f[9] + hg[0];
+            o[1] = f[3] + f[4] + f[5] + f[10] + hg[1];
+            o[2] = f[6] + f[7] + f[8] + f[11] + hg[2];
+        }
+        if constexpr (kTile) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                stage[(a * 3 + k) * kTileElems + tx] = o[k];
+                d[a * 3 + k] = f[9 + k] + hg[k];
+            }
+        } else {
+            store3_nt(E.ef, elem_slot(p, a), o[0], o[1], o[2]);
+            if (mask & (1u << a)) store3_nt(E.ef2, elem_slot(p, a), f[9] + hg[0], f[10] + hg[1], f[11] + hg[2]);
         }
         if constexpr (!kLds && !kKeep) {
 #pragma unroll
             for (int k = 0; k < kNo; k++) opc_[k] = opn_[k];
         }
+    }
+}
+
+// An element of a PML tile with its operators in modal form (kOpsGeom),
+// otherwise as pml_element with kTile.
+template <typename R, int kHG, bool kMass>
+__device__ __forceinline__ void pml_element_modal(const PmlElems<R> &E, const NodeState &N, const StepConsts &C,
+                                                  int64_t p, lds_ptr<R> stage, R d[24])
+{
+#pragma clang fp contract(fast)
+    int nds[8];
+#pragma unroll
+    for (int a = 0; a < 8; a++) nds[a] = load_nt(E.ien + blk_at<8>(p, a));
+    // everything that comes from memory is asked for at once: a tile's waves wait
+    // together, and few of them share a SIMD
+    R xc[kGeoMat + 2], old[21], fv[3][8], fu[3][8], damp[3];
+#pragma unroll
+    for (int i = 0; i < kGeoMat + 2; i++) xc[i] = opb_at<R, kOpG>(E.opb, p, i);
+#pragma unroll
+    for (int i = 0; i < 21; i++) old[i] = load_nt(E.stress + blk_at<21>(p, i));
+#pragma unroll
+    for (int k = 0; k < 3; k++) damp[k] = E.damp[blk_at<3>(p, k)];
+    const unsigned mask = E.mask12[p];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            fv[k][a] = gather_v<R>(N, nds[a], k);
+            if (kHG == 1) fu[k][a] = gather_u<R>(N, nds[a], k);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    const R lam = xc[kGeoMat], miu = xc[kGeoMat + 1];
+    ModalOps<R> G;
+    modal_ops<R>(xc, lam, miu, G);
+    const R rdk = (R)C.rdampk;
+    // modal sums of velocity and of ut = u + rdampk v, relative to the first node
+    R vl[3][3], ul[3][3], uh[3][4], vh[3][4];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+#pragma unroll
+        for (int a = 7; a >= 0; a--) fv[k][a] = fv[k][a] - fv[k][0];
+        split8<R>(fv[k], vl[k], vh[k]);
+        if (kHG == 1) {
+#pragma unroll
+            for (int a = 7; a >= 0; a--) fu[k][a] = fu[k][a] - fu[k][0];
+            split8<R>(fu[k], ul[k], uh[k]);
+#pragma unroll
+            for (int l = 0; l < 3; l++) ul[k][l] = ul[k][l] + rdk * vl[k][l];
+#pragma unroll
+            for (int m = 0; m < 4; m++) uh[k][m] = uh[k][m] + rdk * vh[k][m];
+        }
+    }
+    R D[3][3];  // D[k][i]: gradient of velocity component k along i
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const R g = (G.c[i] * vl[k][0] + G.c[3 + i] * vl[k][1] + G.c[6 + i] * vl[k][2]) * G.q;
+            D[k][i] = g + g * G.dq;  // as in regular_element_modal
+        }
+    const R l2m = lam + (R)2 * miu;
+    const R sr[6] = {D[0][0], D[1][1], D[2][2], D[1][2] + D[2][1], D[0][2] + D[2][0], D[0][1] + D[1][0]};
+    R srt[6];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        R acc = 0;
+#pragma unroll
+        for (int j = 0; j < 3; j++) acc = acc + (i == j ? l2m : lam) * sr[j];
+        srt[i] = acc;
+    }
+#pragma unroll
+    for (int i = 3; i < 6; i++) srt[i] = miu * sr[i];
+    // the 15 split stresses
+    const R rdt = (R)1 / (R)C.dt;
+    const R coef[15] = {l2m, lam, lam, lam, l2m, lam, lam, lam, l2m, miu, miu, miu, miu, miu, miu};
+    const R grad[15] = {D[0][0], D[1][1], D[2][2], D[0][0], D[1][1], D[2][2], D[0][0], D[1][1], D[2][2],
+                        D[1][0], D[0][1], D[2][0], D[0][2], D[2][1], D[1][2]};
+    constexpr int dir[15] = {0, 1, 2, 0, 1, 2, 0, 1, 2, 0, 1, 0, 2, 1, 2};
+    R dmul[3], dden[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        dmul[k] = rdt - damp[k] / (R)2;
+        dden[k] = rdt + damp[k] / (R)2;
+    }
+    R sv[15];
+#pragma unroll
+    for (int c = 0; c < 15; c++) {
+        const R sc = (coef[c] * grad[c] + dmul[dir[c]] * old[c]) / dden[dir[c]];
+        sv[c] = sc;
+        store_nt(E.stress + blk_at<21>(p, c), sc);
+    }
+    const R sum[6] = {sv[0] + sv[1] + sv[2], sv[3] + sv[4] + sv[5], sv[6] + sv[7] + sv[8],
+                      sv[13] + sv[14], sv[11] + sv[12], sv[9] + sv[10]};  // xx, yy, zz, yz, xz, xy
+    // the summed stresses, for the PML nodes' split forces (node_pml_kernel)
+    store_pair(E.ssum + pml_at<R, 6>(p, 0), sum[0], sum[1]);
+    store_pair(E.ssum + pml_at<R, 6>(p, 2), sum[2], sum[5]);
+    store_pair(E.ssum + pml_at<R, 6>(p, 4), sum[4], sum[3]);
+    const int tx = threadIdx.x;
+    const R st[6] = {sum[0], sum[1], sum[2], sum[5], sum[4], sum[3]};
+#pragma unroll
+    for (int c = 0; c < 6; c++) stage[(24 + c) * kTileElems + tx] = st[c];
+    R s0[6], J[9], lin[3][3], hg[3][4];
+#pragma unroll
+    for (int k = 0; k < 6; k++) s0[k] = old[15 + k] + rdk * srt[k];
+#pragma unroll
+    for (int i = 0; i < 9; i++) J[i] = (R)C.w * (R)0.125 * G.c[i];  // det*w*q = w/8
+    constexpr int sym[3][3] = {{0, 5, 4}, {5, 1, 3}, {4, 3, 2}};
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int l = 0; l < 3; l++)
+            lin[k][l] = -(J[3 * l] * s0[sym[k][0]] + J[3 * l + 1] * s0[sym[k][1]] + J[3 * l + 2] * s0[sym[k][2]]);
+    if (kHG == 1) {
+        modal_hourglass<R>(G, ul, uh, lin, hg);
+    } else {
+        R c2 = 0;
+        if (kHG == 2) {
+            const R vp = opb_at<R, kOpG>(E.opb, p, kGeoMat + 2), rho = opb_at<R, kOpG>(E.opb, p, kGeoMat + 3);
+            c2 = (R)0.25 * (R)C.kapa_hg * rho * vp * (R)pow((double)G.det * C.w, 2.0 / 3.0);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int m = 0; m < 4; m++) hg[k][m] = kHG == 2 ? -(c2 * vh[k][m]) : (R)0;
+    }
+    auto mass = [&](int a, int k) -> R {
+        if constexpr (!kMass) return 0;
+        R al = (R)(C.rdampm * node_v<R>(N, nds[a], k));
+        if (k == 2) al = al + (R)C.gterm;
+        return al * E.emass[blk_at<24>(p, a * 3 + k)];
+    };
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        R g[8], f[8];
+        join3<R>(J[k], J[3 + k], J[6 + k], g);
+        join8<R>(lin[k], hg[k], f);
+        // a PML node: det*w*dN_a/dx_k, and force component 10 + k
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            stage[(a * 3 + k) * kTileElems + tx] = g[a];
+            d[a * 3 + k] = f[a] - mass(a, k);
+        }
+    }
+    if (mask != 0xFFu) {
+        // a 3-component node takes the collapsed sums (src/assembleGlobalKU.f90:55-61)
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            R f[8];
+#pragma unroll
+            for (int l = 0; l < 3; l++)
+                lin[k][l] = lin[k][l] - (J[3 * l] * sum[sym[k][0]] + J[3 * l + 1] * sum[sym[k][1]] + J[3 * l + 2] * sum[sym[k][2]]);
+            join8<R>(lin[k], hg[k], f);
+#pragma unroll
+            for (int a = 0; a < 8; a++)
+                if (!(mask & (1u << a))) stage[(a * 3 + k) * kTileElems + tx] = f[a] - mass(a, k);
+        }
+    }
+}
+
+// The end of a PML tile's workgroup, called when the thread's first staged
+// values are written (finish_tile tells the rest): the inner nodes' 9 split
+// components from dw g and the summed stresses, as node_pml_kernel forms them,
+// and the slots of ef; then components 10-12 take the stage.
+template <typename R>
+__device__ __forceinline__ void finish_pml_tile(const PmlElems<R> &E, const NodeState &N, const PmlNodes &P, const Tile &T,
+                                                lds_ptr<R> stage, const R d[24], double dt, int mode, int next_step)
+{
+    const int tid = threadIdx.x, node = T.n0 + tid;
+    const int64_t q = P.n_outer + T.i0 + tid;
+    constexpr int kAhead = 4;
+    const int64_t s0 = (int64_t)T.s0 * 64 + tid;
+    uint4 ent;
+    NodePml S;
+    unsigned src[kAhead];
+    if (tid < T.nn) {
+        ent = E.tile_ent[T.i0 + tid];
+        node_pml_load<R>(N, P, q, node, S);
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; i++)
+        src[i] = tid + i * kTileElems < T.ns ? E.tile_src[s0 + i * kTileElems] : kTileNone;
+    auto send = [&](R *ef) {
+        auto one = [&](unsigned e, int64_t slot) {
+            if (e == kTileNone) return;
+            const unsigned at = (e / kTileElems) * 3 * kTileElems + e % kTileElems;
+            store3_nt<R>(ef, slot, stage[at], stage[at + kTileElems], stage[at + 2 * kTileElems]);
+        };
+#pragma unroll
+        for (int i = 0; i < kAhead; i++) one(src[i], s0 + i * kTileElems);
+        for (int p = tid + kAhead * kTileElems; p < T.ns; p += kTileElems) one(E.tile_src[s0 + p - tid], s0 + p - tid);
+    };
+    // the node's k-th entry in the stage, and its element's lane
+    auto entry = [&](int k, unsigned &at, unsigned &lane) {
+        const uint32_t w = k < 2 ? ent.x : k < 4 ? ent.y : k < 6 ? ent.z : ent.w;
+        const unsigned e = (w >> ((k & 1) * 16)) & 0xFFFFu;
+        lane = e % kTileElems;
+        at = (e / kTileElems) * 3 * kTileElems + lane;
+        return e != kTileNone;
+    };
+    double F[12];
+#pragma unroll
+    for (int k = 0; k < 12; k++) F[k] = 0.0;
+    __syncthreads();
+    send(E.ef);
+    if (tid < T.nn) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            unsigned at, lane;
+            if (!entry(k, at, lane)) continue;
+            R g[3], s[6];
+#pragma unroll
+            for (int i = 0; i < 3; i++) g[i] = stage[at + i * kTileElems];
+#pragma unroll
+            for (int i = 0; i < 6; i++) s[i] = stage[(24 + i) * kTileElems + lane];
+            constexpr int si[9] = {0, 3, 4, 3, 1, 5, 4, 5, 2};  // xx xy xz, xy yy yz, xz yz zz
+#pragma unroll
+            for (int c = 0; c < 9; c++) {
+                const R f = (R)0 - g[c % 3] * s[si[c]];
+                F[c] = F[c] + (double)f;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < T.ne) {
+#pragma unroll
+        for (int i = 0; i < 24; i++) stage[i * kTileElems + tid] = d[i];
+    }
+    __syncthreads();
+    send(E.ef2);
+    if (tid < T.nn) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            unsigned at, lane;
+            if (!entry(k, at, lane)) continue;
+#pragma unroll
+            for (int c = 0; c < 3; c++) F[9 + c] = F[9 + c] + (double)stage[at + c * kTileElems];
+        }
+        node_pml_update<R>(N, P, q, node, S, F, dt, mode, next_step);
+    }
+}
+
+template <typename R, int kHG, bool kMass, int kOps>
+__device__ __forceinline__ void pml_tile_element(const PmlElems<R> &E, const NodeState &N, const StepConsts &C, int64_t p,
+                                                 lds_ptr<R> tables, lds_ptr<R> stage, R d[24])
+{
+    if constexpr (kOps == kOpsGeom) pml_element_modal<R, kHG, kMass>(E, N, C, p, stage, d);
+    else pml_element<R, kHG, kMass, kOps, true>(E, N, C, p, tables, stage, d);
+}
+
+// One workgroup: blockDim.x elements, or (kTile) a tile of elements with its
+// inner nodes.
+//
+// In tiles (elem_regular_kernel tells the reasons) an element's 54 values for
+// its nodes take the stage in two turns, 30 and 24: 30.7 KB in FP32, 61 KB in
+// FP64, which leaves three and two workgroups a CU.  So few waves wait together
+// for memory that everything an element reads is asked for first (FP32 with
+// geometry rows, 1.04 M elements: 177 -> 130 us; two or more nodes in flight
+// in FP64 spill, 48 -> 173 us for 232,000).  Element and PML node kernel of a step:
+// 1.04 M elements FP32 118 + 112 -> 130 + 93 us (the fault kernel runs beside
+// the second), 938,200 with class tables 95 + 84 -> 115 + 65, 466,000 FP64 with
+// stored rows 116 + 76 -> 126 + 48, 232,000 with class tables 47 + 44 -> 48 + 32.
+template <typename R, int kHG, bool kMass, int kOps, bool kTile>
+__global__ void __launch_bounds__(256, (sizeof(R) == 8 ? (kTile ? 2 : 3) : (kOps == kOpsGeom ? EQD_PML_GEO_WAVES : (kTile ? 3 : 4))))
+    elem_pml_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem, int remap)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char eqd_smem[];
+    const unsigned gb = launch_block(remap);
+    const Member<R> &M = Ms[member_of(bmem, gb)];
+    const PmlElems<R> E = M.P;
+    const NodeState N = M.N;
+    const StepConsts C = M.C;
+    const unsigned b = gb - (unsigned)M.blk0[kKPml];
+    lds_ptr<R> tables = (lds_ptr<R>)eqd_smem, stage = tables;
+    if constexpr (kOps == kOpsLds) {
+        // class tables staged in LDS, as in elem_regular_kernel
+        lds_ptr<R> lph = tables + E.n_opc * kOpW;
+        for (int j = threadIdx.x; j < E.n_opc * kOpW; j += blockDim.x) tables[j] = E.optab[j];
+        for (int j = threadIdx.x; j < E.n_phic * 32; j += blockDim.x) lph[j] = E.phitab[j];
+        __syncthreads();
+        stage = lph + E.n_phic * 32;
+    }
+    if constexpr (kTile) {
+        const Tile T = E.tile[b];
+        const int nt = M.clk->nt, mode = M.clk->mode;
+        R d[24];
+        if ((int)threadIdx.x < T.ne)
+            pml_tile_element<R, kHG, kMass, kOps>(E, N, C, T.e0 + (int)threadIdx.x, tables, stage, d);
+        finish_pml_tile<R>(E, N, M.PN, T, stage, d, C.dt, mode, nt + 1);
+    } else {
+        const int64_t p = (int64_t)b * blockDim.x + threadIdx.x;
+        R d[1];
+        if (p < E.n) pml_element<R, kHG, kMass, kOps, false>(E, N, C, p, tables, stage, d);
     }
 }
 
@@ -1594,15 +1973,7 @@ __device__ __forceinline__ void gather3(const NodeState &N, int node, const R *e
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             if (j0 + k < end) {
-                const int64_t idx = e[k] & kEntIdxMask;
-                const int a = (e[k] >> kEntLocalShift) & 7;
-                if (e[k] & kEntPml) {
-                    load_pair(efp + pml_at<R, kEfPml>(idx, a * 6), f[k][0], f[k][1]);
-                    f[k][2] = efp[pml_at<R, kEfPml>(idx, a * 6 + 2)];
-                } else {
-                    load_pair(ef + slot_at<R>(e[k], 0), f[k][0], f[k][1]);
-                    f[k][2] = ef[slot_at<R>(e[k], 2)];
-                }
+                load3(e[k] & kEntPml ? efp : ef, e[k] & kEntSlotMask, f[k][0], f[k][1], f[k][2]);
             }
         }
 #pragma unroll
@@ -1630,15 +2001,7 @@ __device__ __forceinline__ void gather3_ell(const uint32_t *ell, int64_t i, cons
 #pragma unroll
     for (int k = 0; k < kEll3; k++) {
         if (e[k] != kEntNone) {
-            const int64_t idx = e[k] & kEntIdxMask;
-            const int a = (e[k] >> kEntLocalShift) & 7;
-            if (e[k] & kEntPml) {
-                load_pair(efp + pml_at<R, kEfPml>(idx, a * 6), f[k][0], f[k][1]);
-                f[k][2] = efp[pml_at<R, kEfPml>(idx, a * 6 + 2)];
-            } else {
-                load_pair(ef + slot_at<R>(e[k], 0), f[k][0], f[k][1]);
-                f[k][2] = ef[slot_at<R>(e[k], 2)];
-            }
+            load3(e[k] & kEntPml ? efp : ef, e[k] & kEntSlotMask, f[k][0], f[k][1], f[k][2]);
         }
     }
 #pragma unroll
@@ -1679,7 +2042,6 @@ __global__ void __launch_bounds__(256) node3_kernel(const Member<R> *__restrict_
 
 // 12-component (PML) nodes; the gather reads only PML element forces because
 // regular elements never touch a PML node (checked on the host).
-// src/driver.f90:107-141 for the damped split update.
 template <typename R>
 __global__ void __launch_bounds__(256) node_pml_kernel(const Member<R> *__restrict__ Ms,
                                                        const uint16_t *__restrict__ bmem, int remap)
@@ -1687,10 +2049,10 @@ __global__ void __launch_bounds__(256) node_pml_kernel(const Member<R> *__restri
     const unsigned gb = launch_block(remap);
     const Member<R> &M = Ms[member_of(bmem, gb)];
     const int64_t q = (int64_t)(gb - (unsigned)M.blk0[kKNodePml]) * blockDim.x + threadIdx.x;
-    if (q >= M.PN.n) return;
+    if (q >= M.PN.n_outer) return;
     const NodeState N = M.N;
     const PmlNodes P = M.PN;
-    const R *efp = M.P.ef, *ssum = M.P.ssum;
+    const R *efp = M.P.ef, *ef2 = M.P.ef2, *ssum = M.P.ssum;
     const double dt = M.C.dt;
     const Clock ck = *M.clk;
     const int mode = ck.mode, next_step = ck.nt + 1;
@@ -1705,18 +2067,21 @@ __global__ void __launch_bounds__(256) node_pml_kernel(const Member<R> *__restri
         uint32_t e[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) e[k] = j0 + k < end ? N.ent[j0 + k] : 0u;
+        int el[4];
+        if (N.ent_el) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) el[k] = j0 + k < end ? N.ent_el[j0 + k] : 0;
+        }
         R f[4][12];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             if (j0 + k < end) {
-                const int64_t idx = e[k] & kEntIdxMask;
-                const int a = (e[k] >> kEntLocalShift) & 7;
                 // the 9 split components from dw g and the element's summed
                 // stresses, as elem_pml_kernel forms them; 10-12 as stored
+                const int64_t slot = e[k] & kEntSlotMask, idx = N.ent_el ? el[k] : slot_elem(slot);
                 R q1, q2, q3, d1, d2, d3, sxx, syy, szz, sxy, sxz, syz;
-                load_pair(efp + pml_at<R, kEfPml>(idx, a * 6 + 0), q1, q2);
-                load_pair(efp + pml_at<R, kEfPml>(idx, a * 6 + 2), q3, d1);
-                load_pair(efp + pml_at<R, kEfPml>(idx, a * 6 + 4), d2, d3);
+                load3(efp, slot, q1, q2, q3);
+                load3(ef2, slot, d1, d2, d3);
                 load_pair(ssum + pml_at<R, 6>(idx, 0), sxx, syy);
                 load_pair(ssum + pml_at<R, 6>(idx, 2), szz, sxy);
                 load_pair(ssum + pml_at<R, 6>(idx, 4), sxz, syz);
@@ -1742,30 +2107,9 @@ __global__ void __launch_bounds__(256) node_pml_kernel(const Member<R> *__restri
             }
         }
     }
-    const double m = node_mass<R>(N, node);
-    if (mode == 1) {
-#pragma unroll
-        for (int k = 0; k < 12; k++) P.acc[blk_at<12>(q, k)] = F[k] / m;
-        return;
-    }
-    const double d[3] = {pml_damp<R>(P, q, 0), pml_damp<R>(P, q, 1), pml_damp<R>(P, q, 2)};
-    double v[12];
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        const double dv = d[k % 3];
-        v[k] = (F[k] / m + pml_v<R>(P, q, k) * (1.0 / dt - dv / 2.0)) / (1.0 / dt + dv / 2.0);
-    }
-#pragma unroll
-    for (int k = 9; k < 12; k++) v[k] = pml_v<R>(P, q, k) + F[k] / m * dt;
-#pragma unroll
-    for (int k = 0; k < 12; k++) pml_store<R>(P, q, k, v[k]);
-    double vel[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        vel[k] = v[3 * k] + v[3 * k + 1] + v[3 * k + 2] + v[9 + k];
-        node_store<R>(N, node, k, vel[k], node_u<R>(N, node, k) + vel[k] * dt);
-    }
-    flag_nan(N, node, next_step, vel[0], vel[1], vel[2]);
+    NodePml S;
+    node_pml_load<R>(N, P, q, node, S);
+    node_pml_update<R>(N, P, q, node, S, F, dt, mode, next_step);
 }
 
 // Pending update at the start of a run: v += a*dt from the stored F/m
@@ -2431,7 +2775,7 @@ hipError_t launch_elem(const Member<R> *M, const LaunchGrid &g, int q, int dp, i
 }
 
 template <typename R>
-hipError_t launch_pml(const Member<R> *M, const LaunchGrid &g, int hg, int mass, int ops, hipStream_t s,
+hipError_t launch_pml(const Member<R> *M, const LaunchGrid &g, int hg, int mass, int ops, int tiled, hipStream_t s,
                       hipEvent_t t0, hipEvent_t t1)
 {
     if (g.grid == 0) return hipSuccess;
@@ -2439,20 +2783,22 @@ hipError_t launch_pml(const Member<R> *M, const LaunchGrid &g, int hg, int mass,
     if (ops < kOpsRows || ops > kOpsGeom) return hipErrorInvalidValue;
     if (ops == kOpsGeom && sizeof(R) != sizeof(float)) return hipErrorInvalidValue;
     constexpr int kGeoOr = sizeof(R) == sizeof(float) ? kOpsGeom : kOpsCompact;
-    // class tables, or each thread's staged dN/dx (24 values); geometry rows
-    // keep dN/dx in registers
-    const size_t lds = ops == kOpsLds ? g.lds
-                                      : (ops == kOpsGeom ? 0 : (EQD_STAGE_SHP_PML ? (size_t)g.block * 24 * sizeof(R) : 0));
-#define EQD_LAUNCH(HG, MASS)                                                                              \
-    do {                                                                                                  \
-        if (ops == kOpsLds)                                                                               \
-            EQD_GO((elem_pml_kernel<R, HG, MASS, kOpsLds>), g.grid, g.block, lds, s, M, g.bmem, g.remap);     \
-        else if (ops == kOpsGeom)                                                                         \
-            EQD_GO((elem_pml_kernel<R, HG, MASS, kGeoOr>), g.grid, g.block, lds, s, M, g.bmem, g.remap);  \
-        else if (ops == kOpsCompact)                                                                      \
-            EQD_GO((elem_pml_kernel<R, HG, MASS, kOpsCompact>), g.grid, g.block, lds, s, M, g.bmem, g.remap); \
-        else                                                                                              \
-            EQD_GO((elem_pml_kernel<R, HG, MASS, kOpsRows>), g.grid, g.block, lds, s, M, g.bmem, g.remap);    \
+    // class tables and a tile's staged forces; else class tables, or each
+    // thread's staged dN/dx (24 values); geometry rows keep dN/dx in registers
+    const size_t lds = ops == kOpsLds || tiled
+                           ? g.lds
+                           : (ops == kOpsGeom ? 0 : (EQD_STAGE_SHP_PML ? (size_t)g.block * 24 * sizeof(R) : 0));
+#define EQD_LAUNCH_OPS(HG, MASS, OPS)                                                                              \
+    do {                                                                                                           \
+        if (tiled) EQD_GO((elem_pml_kernel<R, HG, MASS, OPS, true>), g.grid, g.block, lds, s, M, g.bmem, g.remap); \
+        else EQD_GO((elem_pml_kernel<R, HG, MASS, OPS, false>), g.grid, g.block, lds, s, M, g.bmem, g.remap);      \
+    } while (0)
+#define EQD_LAUNCH(HG, MASS)                                        \
+    do {                                                            \
+        if (ops == kOpsLds) EQD_LAUNCH_OPS(HG, MASS, kOpsLds);      \
+        else if (ops == kOpsGeom) EQD_LAUNCH_OPS(HG, MASS, kGeoOr); \
+        else if (ops == kOpsCompact) EQD_LAUNCH_OPS(HG, MASS, kOpsCompact); \
+        else EQD_LAUNCH_OPS(HG, MASS, kOpsRows);                    \
     } while (0)
     if (mass) {
         if (hg == 1) EQD_LAUNCH(1, true);
@@ -2464,6 +2810,7 @@ hipError_t launch_pml(const Member<R> *M, const LaunchGrid &g, int hg, int mass,
         else EQD_LAUNCH(0, false);
     }
 #undef EQD_LAUNCH
+#undef EQD_LAUNCH_OPS
     return hipGetLastError();
 }
 
@@ -2536,7 +2883,7 @@ hipError_t launch_step_start(const Member<R> *M, int nmem, hipStream_t s, hipEve
 #define EQD_INSTANTIATE(R)                                                                                     \
     template hipError_t launch_elem<R>(const Member<R> *, const LaunchGrid &, int, int, int, int, int, int, hipStream_t, \
                                        hipEvent_t, hipEvent_t);                                                       \
-    template hipError_t launch_pml<R>(const Member<R> *, const LaunchGrid &, int, int, int, hipStream_t, hipEvent_t,  \
+    template hipError_t launch_pml<R>(const Member<R> *, const LaunchGrid &, int, int, int, int, hipStream_t, hipEvent_t, \
                                       hipEvent_t);                                                                    \
     template hipError_t launch_node3<R>(const Member<R> *, const LaunchGrid &, hipStream_t, hipEvent_t, hipEvent_t);  \
     template hipError_t launch_node_pml<R>(const Member<R> *, const LaunchGrid &, hipStream_t, hipEvent_t,            \

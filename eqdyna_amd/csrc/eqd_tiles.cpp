@@ -1,5 +1,5 @@
-// Tiles of the regular elements: grid positions from the connectivity, a tile
-// shape for the grid's size, and per tile the inner nodes, their force entries
+// Tiles of the elements: grid positions from the connectivity, a tile shape for
+// the grid's size, and per tile the inner nodes, their force entries
 // and the slots of the forces that leave the tile.
 #include "eqd_tiles.h"
 
@@ -14,57 +14,50 @@ namespace {
 
 typedef std::array<int32_t, 3> Pos;
 
-// Integer grid positions of the elements, walking from element to element over
-// shared corners: the neighbour in local direction d of an element is the one
-// whose node 0 is the element's node at the other end of its edge in that
-// direction.  Any positions are valid (they only decide which elements run
-// together); comp numbers the connected pieces.  Wedges (elements with a
-// repeated node), whose edges do not follow the grid, stay out: comp -1.
-void grid_positions(const std::vector<int32_t> &ids, const int32_t *ien, int64_t nn, std::vector<Pos> &pos,
-                    std::vector<int32_t> &comp, int32_t *ncomp)
+// Integer grid positions of all elements, from element to element over shared
+// corners: the neighbour in local direction d of an element is the one whose
+// node 0 is the element's node at the other end of its edge in that direction.
+// Elements are met in their given order, in which one of a grid's neighbours
+// comes before each but the first.  Any positions are valid (they only decide
+// which elements run together); comp numbers the connected pieces as they are
+// met.  Wedges (elements with a repeated node), whose edges do not follow the
+// grid, stay out: comp -1.  Returns the number of pieces.
+int32_t grid_positions(const int32_t *ien, int64_t ne, int64_t nn, std::vector<Pos> &pos, std::vector<int32_t> &comp)
 {
-    const int64_t n = (int64_t)ids.size();
     constexpr int end[3] = {1, 3, 4};  // local node at the far end of node 0's edge in each direction
     std::vector<int32_t> own[4];       // element whose local node 0, 1, 3, 4 is the node
     constexpr int at[4] = {0, 1, 3, 4};
-    std::vector<uint8_t> wedge((size_t)n);
+    pos.assign((size_t)ne, Pos{0, 0, 0});
+    comp.assign((size_t)ne, -2);  // not met yet
 #pragma omp parallel for schedule(static)
-    for (int64_t t = 0; t < n; t++) {
-        const int32_t *nd = ien + (int64_t)ids[t] * 8;
+    for (int64_t e = 0; e < ne; e++) {
+        const int32_t *nd = ien + e * 8;
         for (int a = 0; a < 8; a++)
             for (int b = 0; b < a; b++)
-                if (nd[a] == nd[b]) wedge[t] = 1;
+                if (nd[a] == nd[b]) comp[e] = -1;
     }
 #pragma omp parallel for schedule(static, 1)
     for (int k = 0; k < 4; k++) {
         own[k].assign((size_t)nn, -1);
-        for (int64_t t = 0; t < n; t++)
-            if (!wedge[t]) own[k][ien[(int64_t)ids[t] * 8 + at[k]] - 1] = (int32_t)t;
+        for (int64_t e = 0; e < ne; e++)
+            if (comp[e] != -1) own[k][ien[e * 8 + at[k]] - 1] = (int32_t)e;
     }
-    pos.assign((size_t)n, Pos{0, 0, 0});
-    comp.assign((size_t)n, -1);
-    std::vector<int32_t> stack;
-    *ncomp = 0;
-    for (int64_t s = 0; s < n; s++) {
-        if (wedge[s] || comp[s] >= 0) continue;
-        comp[s] = *ncomp;
-        stack.push_back((int32_t)s);
-        while (!stack.empty()) {
-            const int32_t t = stack.back();
-            stack.pop_back();
-            const int32_t *nd = ien + (int64_t)ids[t] * 8;
-            for (int d = 0; d < 3; d++)
-                for (int back = 0; back < 2; back++) {
-                    const int32_t u = back ? own[d + 1][nd[0] - 1] : own[0][nd[end[d]] - 1];
-                    if (u < 0 || comp[u] >= 0) continue;
-                    comp[u] = *ncomp;
-                    pos[u] = pos[t];
-                    pos[u][d] += back ? -1 : 1;
-                    stack.push_back(u);
-                }
-        }
-        ++*ncomp;
+    int32_t ncomp = 0;
+    for (int64_t e = 0; e < ne; e++) {
+        if (comp[e] == -1) continue;
+        const int32_t *nd = ien + e * 8;
+        for (int d = 0; d < 3 && comp[e] < 0; d++)
+            for (int ahead = 0; ahead < 2; ahead++) {
+                const int32_t u = ahead ? own[0][nd[end[d]] - 1] : own[d + 1][nd[0] - 1];
+                if (u < 0 || comp[u] < 0) continue;
+                comp[e] = comp[u];
+                pos[e] = pos[u];
+                pos[e][d] += ahead ? -1 : 1;
+                break;
+            }
+        if (comp[e] < 0) comp[e] = ncomp++;
     }
+    return ncomp;
 }
 
 // Tiles along each direction for a grid of N elements: the box of at most
@@ -89,203 +82,248 @@ void tile_counts(const int64_t N[3], int64_t cnt[3])
             }
 }
 
-}  // namespace
+struct Grid {
+    std::vector<Pos> pos;
+    std::vector<int32_t> part;  // [ne] 27 * piece + which third in each direction, -1 a wedge
+    int32_t parts;
+    int fast;  // direction in which node numbers run
+};
 
-bool make_tiles(std::vector<int32_t> &ids, const int32_t *ien, int64_t nn, const std::vector<int32_t> &degree,
-                const std::vector<uint8_t> &outer, TileSet &T)
+// Pieces and, in each direction, the thirds below, beside and above the regular
+// elements: the PML elements then fall into layers, edges and corners that
+// are boxes of their own, whatever the layers' thickness.
+bool make_grid(const std::vector<int32_t> &reg, const int32_t *ien, int64_t ne, int64_t nn, Grid &G)
+{
+    const int32_t ncomp = grid_positions(ien, ne, nn, G.pos, G.part);
+    if (ncomp > 1000) return false;
+    std::vector<Pos> lo((size_t)ncomp, Pos{INT32_MAX, INT32_MAX, INT32_MAX}),
+        hi((size_t)ncomp, Pos{INT32_MIN, INT32_MIN, INT32_MIN});
+    for (int32_t e : reg)
+        for (int d = 0; d < 3 && G.part[e] >= 0; d++) {
+            lo[G.part[e]][d] = std::min(lo[G.part[e]][d], G.pos[e][d]);
+            hi[G.part[e]][d] = std::max(hi[G.part[e]][d], G.pos[e][d]);
+        }
+#pragma omp parallel for schedule(static)
+    for (int64_t e = 0; e < ne; e++) {
+        const int32_t c = G.part[e];
+        if (c < 0) continue;
+        int third = 0;
+        for (int d = 0; d < 3; d++) third = third * 3 + (G.pos[e][d] < lo[c][d] ? 0 : G.pos[e][d] > hi[c][d] ? 2 : 1);
+        G.part[e] = c * 27 + third;
+    }
+    G.parts = ncomp * 27;
+    const int32_t *nd = ien + ne / 2 * 8;
+    const int step[3] = {std::abs(nd[1] - nd[0]), std::abs(nd[3] - nd[0]), std::abs(nd[4] - nd[0])};
+    G.fast = 0;
+    for (int d = 1; d < 3; d++)
+        if (step[d] < step[G.fast]) G.fast = d;
+    return true;
+}
+
+// ids tile by tile; false, with ids as they were, when they do not fill their tiles
+bool group(std::vector<int32_t> &ids, const Grid &G, double min_fill, std::vector<Tile> &tile)
 {
     const int64_t n = (int64_t)ids.size();
-    if (n == 0) return false;
-    std::vector<Pos> pos;
-    std::vector<int32_t> comp;
-    int32_t ncomp;
-    grid_positions(ids, ien, nn, pos, comp, &ncomp);
-    std::vector<Pos> lo((size_t)ncomp, Pos{INT32_MAX, INT32_MAX, INT32_MAX}), hi((size_t)ncomp, Pos{INT32_MIN, INT32_MIN, INT32_MIN});
-    for (int64_t t = 0; t < n; t++)
-        for (int d = 0; d < 3 && comp[t] >= 0; d++) {
-            lo[comp[t]][d] = std::min(lo[comp[t]][d], pos[t][d]);
-            hi[comp[t]][d] = std::max(hi[comp[t]][d], pos[t][d]);
+    std::vector<Pos> lo((size_t)G.parts, Pos{INT32_MAX, INT32_MAX, INT32_MAX}),
+        hi((size_t)G.parts, Pos{INT32_MIN, INT32_MIN, INT32_MIN});
+    int64_t nwedge = 0;
+    for (int32_t e : ids) {
+        const int32_t c = G.part[e];
+        if (c < 0) nwedge++;
+        for (int d = 0; d < 3 && c >= 0; d++) {
+            lo[c][d] = std::min(lo[c][d], G.pos[e][d]);
+            hi[c][d] = std::max(hi[c][d], G.pos[e][d]);
         }
-    // the direction in which node numbers run, from a middle element
-    int fast = 0;
-    {
-        const int32_t *nd = ien + (int64_t)ids[n / 2] * 8;
-        const int step[3] = {std::abs(nd[1] - nd[0]), std::abs(nd[3] - nd[0]), std::abs(nd[4] - nd[0])};
-        for (int d = 1; d < 3; d++)
-            if (step[d] < step[fast]) fast = d;
     }
-    const int o1 = (fast + 1) % 3, o2 = (fast + 2) % 3;
-    std::vector<std::array<int64_t, 3>> cnt((size_t)ncomp), len((size_t)ncomp);
-    std::vector<int64_t> base((size_t)ncomp + 1, 0);
-    for (int32_t c = 0; c < ncomp; c++) {
+    const int fast = G.fast, o1 = (fast + 1) % 3, o2 = (fast + 2) % 3;
+    std::vector<std::array<int64_t, 3>> cnt((size_t)G.parts), len((size_t)G.parts);
+    std::vector<int64_t> base((size_t)G.parts + 1, 0);
+    for (int32_t c = 0; c < G.parts; c++) {
+        base[c + 1] = base[c];
+        if (lo[c][0] > hi[c][0]) continue;  // no element of the class
         for (int d = 0; d < 3; d++) len[c][d] = (int64_t)hi[c][d] - lo[c][d] + 1;
         tile_counts(len[c].data(), cnt[c].data());
-        base[c + 1] = base[c] + cnt[c][0] * cnt[c][1] * cnt[c][2];
-        if (base[c + 1] > 4 * n) return false;
+        base[c + 1] += cnt[c][0] * cnt[c][1] * cnt[c][2];
+        if (base[c + 1] > 4 * n + 64) return false;
     }
-    // elements by box, and within a box in rows along the fast direction
-    const int64_t nwedge = std::count(comp.begin(), comp.end(), -1);
-    const int64_t nbox = base[ncomp] + (nwedge + kTileElems - 1) / kTileElems;
+    // elements by box, and within a box in rows along the fast direction;
+    // wedges in their given order, in boxes of their own
+    const int64_t nbox = base[G.parts] + (nwedge + kTileElems - 1) / kTileElems;
     std::vector<int32_t> box((size_t)n);
     std::vector<int64_t> start((size_t)nbox + 1, 0);
-    int64_t w = 0;  // wedges in their given order, in boxes of their own
+    int64_t w = 0;
     for (int64_t t = 0; t < n; t++) {
-        const int32_t c = comp[t];
+        const int32_t c = G.part[ids[t]];
         if (c < 0) {
-            box[t] = (int32_t)(base[ncomp] + w++ / kTileElems);
-            start[box[t] + 1]++;
-            continue;
+            box[t] = (int32_t)(base[G.parts] + w++ / kTileElems);
+        } else {
+            int64_t b[3];
+            for (int d = 0; d < 3; d++) b[d] = (int64_t)(G.pos[ids[t]][d] - lo[c][d]) * cnt[c][d] / len[c][d];
+            box[t] = (int32_t)(base[c] + (b[o2] * cnt[c][o1] + b[o1]) * cnt[c][fast] + b[fast]);
         }
-        int64_t b[3];
-        for (int d = 0; d < 3; d++) b[d] = (int64_t)(pos[t][d] - lo[c][d]) * cnt[c][d] / len[c][d];
-        box[t] = (int32_t)(base[c] + (b[o2] * cnt[c][o1] + b[o1]) * cnt[c][fast] + b[fast]);
         start[box[t] + 1]++;
     }
     int64_t ntile = 0;
     for (int64_t b = 0; b < nbox; b++) ntile += (start[b + 1] + kTileElems - 1) / kTileElems;
     // lanes without an element cost their share of every workgroup
-    if (n < ntile * (kTileElems * 5 / 8)) return false;
+    if ((double)n < min_fill * (double)(ntile * kTileElems)) return false;
     std::partial_sum(start.begin(), start.end(), start.begin());
-    std::vector<int32_t> ord((size_t)n);
+    std::vector<int32_t> out((size_t)n);
     {
         std::vector<int64_t> at(start.begin(), start.end() - 1);
-        for (int64_t t = 0; t < n; t++) ord[at[box[t]]++] = (int32_t)t;
+        for (int64_t t = 0; t < n; t++) out[at[box[t]]++] = ids[t];
     }
 #pragma omp parallel for schedule(dynamic, 64)
     for (int64_t b = 0; b < nbox; b++)
-        std::sort(ord.begin() + start[b], ord.begin() + start[b + 1], [&](int32_t x, int32_t y) {
-            const Pos &p = pos[x], &q = pos[y];
+        std::sort(out.begin() + start[b], out.begin() + start[b + 1], [&](int32_t x, int32_t y) {
+            const Pos &p = G.pos[x], &q = G.pos[y];
             if (p[o2] != q[o2]) return p[o2] < q[o2];
             if (p[o1] != q[o1]) return p[o1] < q[o1];
             if (p[fast] != q[fast]) return p[fast] < q[fast];
             return x < y;
         });
-    T.tile.clear();
     for (int64_t b = 0; b < nbox; b++)
         for (int64_t e = start[b]; e < start[b + 1]; e += kTileElems)
-            T.tile.push_back(Tile{(int32_t)e, (int32_t)std::min<int64_t>(kTileElems, start[b + 1] - e), 0, 0, 0, 0, 0});
-    std::vector<int32_t> out((size_t)n);
-    for (int64_t t = 0; t < n; t++) out[t] = ids[ord[t]];
+            tile.push_back(Tile{(int32_t)e, (int32_t)std::min<int64_t>(kTileElems, start[b + 1] - e), 0, 0, 0, 0, 0});
+    ids.swap(out);
+    return true;
+}
+
+}  // namespace
+
+bool make_tiles(std::vector<int32_t> *const ids[2], const bool want[2], const int32_t *ien, int64_t ne, int64_t nn,
+                const std::vector<int32_t> &degree, const std::vector<uint8_t> &kind, double min_fill, TileSet T[2],
+                NodeOrder &O)
+{
+    if (!want[0] && !want[1]) return false;
+    Grid G;
+    if (!make_grid(*ids[0], ien, ne, nn, G)) return false;
+    for (int c = 0; c < 2; c++)
+        if (want[c] && !ids[c]->empty()) group(*ids[c], G, min_fill, T[c].tile);
+    const int64_t nt0 = (int64_t)T[0].tile.size(), nt = nt0 + (int64_t)T[1].tile.size();
+    if (nt == 0) return false;
+    auto tile = [&](int64_t k) -> Tile & { return k < nt0 ? T[0].tile[k] : T[1].tile[k - nt0]; };
     // The first and last tile that touches a node; nodes in the order of their
     // first tile, a tile's inner nodes first and then its others by last tile,
     // so that a tile's inner nodes, and the nodes that the same tiles share,
     // are neighbours in memory.  Nodes of no tile come first.
-    const int64_t nt = (int64_t)T.tile.size();
     std::vector<int32_t> first((size_t)nn, -1), last((size_t)nn, -1), touch((size_t)nn, 0);
-    for (int64_t k = 0; k < nt; k++)
-        for (int32_t t = T.tile[k].e0; t < T.tile[k].e0 + T.tile[k].ne; t++)
+    for (int64_t k = 0; k < nt; k++) {
+        const Tile &K = tile(k);
+        const std::vector<int32_t> &el = *ids[k < nt0 ? 0 : 1];
+        for (int32_t t = K.e0; t < K.e0 + K.ne; t++)
             for (int a = 0; a < 8; a++) {
-                const int32_t nd = ien[(int64_t)out[t] * 8 + a] - 1;
+                const int32_t nd = ien[(int64_t)el[t] * 8 + a] - 1;
                 if (first[nd] < 0) first[nd] = (int32_t)k;
                 last[nd] = (int32_t)k;
                 touch[nd]++;
             }
+    }
     auto inner = [&](int32_t nd) {
-        return first[nd] >= 0 && first[nd] == last[nd] && touch[nd] == degree[nd] && degree[nd] <= 8 && !outer[nd];
+        return first[nd] >= 0 && first[nd] == last[nd] && touch[nd] == degree[nd] && degree[nd] <= 8 &&
+               kind[nd] == (first[nd] < nt0 ? 1 : 2);
     };
     std::vector<int64_t> nstart((size_t)nt + 2, 0);
     for (int64_t n = 0; n < nn; n++) nstart[first[n] + 2]++;
     std::partial_sum(nstart.begin(), nstart.end(), nstart.begin());
-    T.ref.resize((size_t)nn);
-    T.at.resize((size_t)nn);
+    O.ref.resize((size_t)nn);
+    O.at.resize((size_t)nn);
     {
         std::vector<int64_t> at(nstart.begin(), nstart.end() - 1);
-        for (int64_t n = 0; n < nn; n++) T.ref[at[first[n] + 1]++] = (int32_t)n;
+        for (int64_t n = 0; n < nn; n++) O.ref[at[first[n] + 1]++] = (int32_t)n;
     }
-    T.n_inner = 0;
-    int64_t nin = 0;
-#pragma omp parallel for schedule(dynamic, 64) reduction(+ : nin)
+#pragma omp parallel for schedule(dynamic, 64)
     for (int64_t k = 0; k < nt; k++) {
-        const auto b = T.ref.begin() + nstart[k + 1], e = T.ref.begin() + nstart[k + 2];
+        const auto b = O.ref.begin() + nstart[k + 1], e = O.ref.begin() + nstart[k + 2];
         const auto mid = std::stable_partition(b, e, [&](int32_t n) { return inner(n); });
         std::stable_sort(mid, e, [&](int32_t x, int32_t y) { return last[x] < last[y]; });
-        T.tile[k].n0 = (int32_t)nstart[k + 1];
-        T.tile[k].nn = (int32_t)(mid - b);
-        nin += mid - b;
+        tile(k).n0 = (int32_t)nstart[k + 1];
+        tile(k).nn = (int32_t)(mid - b);
     }
-    T.n_inner = nin;
-    T.inner.assign((size_t)nn, 0);
+    O.inner.assign((size_t)nn, 0);
 #pragma omp parallel for schedule(static)
     for (int64_t i = 0; i < nn; i++) {
-        T.at[T.ref[i]] = (int32_t)i;
-        T.inner[T.ref[i]] = inner(T.ref[i]);
+        O.at[O.ref[i]] = (int32_t)i;
+        O.inner[O.ref[i]] = inner(O.ref[i]);
     }
     // per tile: its (node, element, local node) entries in the order a node
     // sums them; an inner node's become its row of node_ent, the others slots
     // in runs of neighbouring nodes' q-th entries, as the node kernels read them
-    T.slot_of.assign((size_t)n * 8, kEntNone);
     struct Entry {
         int32_t node, elem, q;
         uint16_t src;  // staged force: local node * kTileElems + lane
     };
-    int64_t nodes = 0;
-    for (Tile &K : T.tile) {
-        K.i0 = (int32_t)nodes;
-        nodes += K.nn;
-    }
-    T.node_ent.assign((size_t)nodes * 8, kTileNone);
-    std::vector<std::vector<uint16_t>> tsrc((size_t)nt);
+    for (int c = 0; c < 2; c++) {
+        TileSet &S = T[c];
+        const std::vector<int32_t> &el = *ids[c];
+        const int64_t ntc = (int64_t)S.tile.size();
+        if (ntc == 0) continue;
+        S.slot_of.assign(el.size() * 8, kEntNone);
+        for (Tile &K : S.tile) {
+            K.i0 = (int32_t)S.n_inner;
+            S.n_inner += K.nn;
+        }
+        S.node_ent.assign((size_t)S.n_inner * 8, kTileNone);
+        std::vector<std::vector<uint16_t>> tsrc((size_t)ntc);
 #pragma omp parallel
-    {
-        std::vector<Entry> E, S;
+        {
+            std::vector<Entry> E, B;
 #pragma omp for schedule(dynamic, 16)
-        for (int64_t k = 0; k < nt; k++) {
-            const Tile &K = T.tile[k];
-            E.clear();
-            S.clear();
-            for (int l = 0; l < K.ne; l++) {
-                const int32_t e = out[K.e0 + l];
-                for (int a = 0; a < 8; a++)
-                    E.push_back(Entry{T.at[ien[(int64_t)e * 8 + a] - 1], e, 0, (uint16_t)(a * kTileElems + l)});
-            }
-            std::sort(E.begin(), E.end(), [](const Entry &x, const Entry &y) {
-                if (x.node != y.node) return x.node < y.node;
-                if (x.elem != y.elem) return x.elem < y.elem;
-                return x.src < y.src;
-            });
-            for (size_t i = 0; i < E.size();) {
-                const int32_t nd = E[i].node;
-                for (int32_t q = 0; i < E.size() && E[i].node == nd; i++, q++) {
-                    if (T.inner[T.ref[nd]]) {
-                        T.node_ent[((int64_t)K.i0 + nd - K.n0) * 8 + q] = E[i].src;
-                    } else {
-                        E[i].q = q;
-                        S.push_back(E[i]);
+            for (int64_t k = 0; k < ntc; k++) {
+                const Tile &K = S.tile[k];
+                E.clear();
+                B.clear();
+                for (int l = 0; l < K.ne; l++) {
+                    const int32_t e = el[K.e0 + l];
+                    for (int a = 0; a < 8; a++)
+                        E.push_back(Entry{O.at[ien[(int64_t)e * 8 + a] - 1], e, 0, (uint16_t)(a * kTileElems + l)});
+                }
+                std::sort(E.begin(), E.end(), [](const Entry &x, const Entry &y) {
+                    if (x.node != y.node) return x.node < y.node;
+                    if (x.elem != y.elem) return x.elem < y.elem;
+                    return x.src < y.src;
+                });
+                for (size_t i = 0; i < E.size();) {
+                    const int32_t nd = E[i].node;
+                    for (int32_t q = 0; i < E.size() && E[i].node == nd; i++, q++) {
+                        if (O.inner[O.ref[nd]]) {
+                            S.node_ent[((int64_t)K.i0 + nd - K.n0) * 8 + q] = E[i].src;
+                        } else {
+                            E[i].q = q;
+                            B.push_back(E[i]);
+                        }
                     }
                 }
+                std::sort(B.begin(), B.end(), [&](const Entry &x, const Entry &y) {
+                    const int32_t a = O.ref[x.node], b = O.ref[y.node];
+                    if (first[a] != first[b]) return first[a] < first[b];
+                    if (last[a] != last[b]) return last[a] < last[b];
+                    if (x.q != y.q) return x.q < y.q;
+                    return x.node < y.node;
+                });
+                for (const Entry &x : B) tsrc[k].push_back(x.src);
+                tsrc[k].resize((tsrc[k].size() + 63) / 64 * 64, kTileNone);
             }
-            std::sort(S.begin(), S.end(), [&](const Entry &x, const Entry &y) {
-                const int32_t a = T.ref[x.node], b = T.ref[y.node];
-                if (first[a] != first[b]) return first[a] < first[b];
-                if (last[a] != last[b]) return last[a] < last[b];
-                if (x.q != y.q) return x.q < y.q;
-                return x.node < y.node;
-            });
-            for (const Entry &x : S) tsrc[k].push_back(x.src);
-            tsrc[k].resize((tsrc[k].size() + 63) / 64 * 64, kTileNone);
         }
-    }
-    int64_t slots = 0;
-    for (int64_t k = 0; k < nt; k++) {
-        Tile &K = T.tile[k];
-        K.s0 = (int32_t)(slots / 64);
-        K.ns = (int32_t)tsrc[k].size();
-        slots += K.ns;
-    }
-    if (slots > (int64_t)kEntSlotMask) return false;
-    T.slot_src.resize((size_t)slots);
+        int64_t slots = 0;
+        for (int64_t k = 0; k < ntc; k++) {
+            S.tile[k].s0 = (int32_t)(slots / 64);
+            S.tile[k].ns = (int32_t)tsrc[k].size();
+            slots += S.tile[k].ns;
+        }
+        S.slot_src.resize((size_t)slots);
 #pragma omp parallel for schedule(static)
-    for (int64_t k = 0; k < nt; k++) {
-        const Tile &K = T.tile[k];
-        const int64_t s0 = (int64_t)K.s0 * 64;
-        for (int i = 0; i < K.ns; i++) {
-            const uint16_t src = tsrc[k][i];
-            T.slot_src[s0 + i] = src;
-            if (src != kTileNone)
-                T.slot_of[((int64_t)K.e0 + src % kTileElems) * 8 + src / kTileElems] = (uint32_t)(s0 + i);
+        for (int64_t k = 0; k < ntc; k++) {
+            const Tile &K = S.tile[k];
+            const int64_t s0 = (int64_t)K.s0 * 64;
+            for (int i = 0; i < K.ns; i++) {
+                const uint16_t src = tsrc[k][i];
+                S.slot_src[s0 + i] = src;
+                if (src != kTileNone)
+                    S.slot_of[((int64_t)K.e0 + src % kTileElems) * 8 + src / kTileElems] = (uint32_t)(s0 + i);
+            }
         }
     }
-    ids.swap(out);
     return true;
 }
 

@@ -1,5 +1,5 @@
-// Tiles of the regular elements (host side): compact groups of at most
-// kTileElems elements, one workgroup of elem_regular_kernel each, so that the
+// Tiles of the elements (host side): compact groups of at most kTileElems
+// elements of a class, one workgroup of its element kernel each, so that the
 // workgroup can sum and update the nodes that no other element touches.
 #pragma once
 #include <cstdint>
@@ -18,24 +18,40 @@ namespace eqd {
 // fault, FP32) 214.1 -> 212.
 constexpr int64_t kTileMinElems = 131072;
 
+// The same for the PML elements, whose tiles have three barriers: 127,932
+// (plastic, FP64) neutral, ensembles of 130,000 at most (FP32) 22.1 -> 23.9 ms
+// with tiles, 232,000 (uniform, FP64) 15.03 -> 13.37, 466,000 (rough fault,
+// FP64) 51.2 -> 47.6, 938,200 (layered, FP32) 91.6 -> 89.9, 1.04 M (rough fault,
+// FP32) 200.4 -> 192.3.
+constexpr int64_t kTileMinPml = 196608;
+// Share of the tiles' lanes that must hold an element.
+constexpr double kTileMinFill = 0.625;
+
+// one class's tiles (none: tile is empty)
 struct TileSet {
     std::vector<Tile> tile;
     std::vector<uint16_t> node_ent;  // 8 per inner node, tile by tile: staged forces in ascending element order
                                      // (kTileNone: none)
     std::vector<uint16_t> slot_src;  // staged force that fills each slot (kTileNone: padding)
     std::vector<uint32_t> slot_of;   // [8 n] slot of element t's force on local node a at t * 8 + a (kEntNone: inner)
-    std::vector<uint8_t> inner;      // [nn] 1: the node is an inner node of a tile
-    // order of the nodes on the device: node n of the reference at at[n], ref its inverse
-    std::vector<int32_t> at, ref;
-    int64_t n_inner;
+    int64_t n_inner = 0;
 };
 
-// Order ids (elements of one class, 0-based, ascending) tile by tile and
-// describe the tiles.  ien: 8 one-based nodes per element; degree: element
-// entries of every node over all classes; outer[n] != 0 keeps node n out of
-// the inner nodes.  Returns false, with ids as they were, when the elements do
-// not group into well filled tiles.
-bool make_tiles(std::vector<int32_t> &ids, const int32_t *ien, int64_t nn, const std::vector<int32_t> &degree,
-                const std::vector<uint8_t> &outer, TileSet &T);
+// order of the nodes on the device: node n of the reference at at[n], ref its
+// inverse; inner[n] 1 where the node is an inner node of a tile
+struct NodeOrder {
+    std::vector<int32_t> at, ref;
+    std::vector<uint8_t> inner;
+};
+
+// Order ids[c] (elements of class c, 0 regular, 1 PML; 0-based, ascending)
+// tile by tile for the classes that are wanted and fill their tiles to at least
+// min_fill on average, describe their tiles in T[c] and order the nodes.  ien: 8 one-based
+// nodes per element; degree: element entries of every node; kind[n]: the class
+// whose tiles node n may be an inner node of, plus one (0: none).  Returns
+// whether any class runs in tiles.
+bool make_tiles(std::vector<int32_t> *const ids[2], const bool want[2], const int32_t *ien, int64_t ne, int64_t nn,
+                const std::vector<int32_t> &degree, const std::vector<uint8_t> &kind, double min_fill, TileSet T[2],
+                NodeOrder &O);
 
 }  // namespace eqd

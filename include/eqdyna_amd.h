@@ -170,7 +170,8 @@ int64_t eqd_device_bytes(eqd_handle *h);
  * at most 8 elements; EQD_NODE_ELL=0 keeps the CSR table); "tiles": the
  * regular elements run in this many tiles whose "tile_inner_nodes" nodes the
  * element kernel updates itself, the other forces leaving through
- * "tile_slots" slots (0: no tiles; EQD_ELEMENT_ORDER).
+ * "tile_slots" slots (0: no tiles; EQD_ELEMENT_ORDER); "tiles_pml",
+ * "tile_inner_nodes_pml", "tile_slots_pml": the same of the PML elements.
  * Returns EQD_EINVAL for an unknown key. */
 int eqd_layout_info(eqd_handle *h, const char *key, int64_t *value);
 

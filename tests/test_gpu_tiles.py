@@ -1,5 +1,5 @@
-"""Regular elements in tiles, whose inner nodes the element kernel sums and
-updates itself (the default from 131,072 regular elements on,
+"""Elements in tiles, whose inner nodes the element kernels sum and update
+themselves (the default from 131,072 regular and 196,608 PML elements on,
 EQD_ELEMENT_ORDER=1 on any mesh), against the reference's element order: a
 node sums the same forces in the same order, so every output is the same bit
 for bit."""
@@ -16,7 +16,8 @@ def solver(name, precision, tiles, monkeypatch):
     bundle, sc, _ = load_golden(name)
     s = Solver(bundle, sc, precision)
     info = s.layout_info()
-    assert (info["tiles"] > 0) == tiles and (info["tile_inner_nodes"] > 0) == tiles
+    for k in ("tiles", "tile_inner_nodes", "tiles_pml", "tile_inner_nodes_pml"):
+        assert (info[k] > 0) == tiles, k
     return s, bundle, sc
 
 
