@@ -146,6 +146,49 @@ void free_tables(eqd_engine *e)
     }
 }
 
+// A step in two launches instead of five on two streams: both element classes,
+// then fault pairs and nodes, which are independent of each other.  Each launch
+// then lasts as long as its longest chain of waits, not the sum of them, and
+// the fork and join of the streams, about 10 us a step, fall away.  Step of a
+// slip-weakening box of 2,800 elements (FP64) 44.2 -> 20.5 us, 5,616 (ageing
+// law, FP32) 52.6 -> 28.9, 69,000 (rough fault, FP64) 85 -> 51, 161,000 (dipping
+// fault) 92.6 -> 70.9.  Element classes are merged where neither runs in tiles,
+// up to kMergeElems elements.  Nodes and pairs are merged up to kMergeNodes of
+// them: the pairs' 256 registers leave that launch two waves a SIMD, still ahead
+// with what tiles leave to the nodes of 432,000 elements (118.5 -> 101.9 us) and
+// of 3.1 M (1.3 M nodes and pairs: 386.0 -> 377.4); with the learned guess, whose
+// network takes 24 KB of LDS a workgroup, up to kMergeNodesLearned (200,000
+// elements 88.3 -> 67.2; 1.4 M nodes and pairs 451.0 -> 476.6 us).  Workgroups of
+// 64, so that a small scenario's waves spread over the CUs.  The same bits in
+// either form; EQD_MERGE=0 keeps the launches apart, 1 merges at any size.
+constexpr int64_t kMergeElems = 393216, kMergeNodes = 1500000, kMergeNodesLearned = 262144;
+constexpr int kMergeElemBlock = 64, kMergeNodeBlock = 64;
+
+template <typename R>
+void step_merged(eqd_engine *e)
+{
+    e->merge_elems = e->merge_nodes = false;
+    const char *s = std::getenv("EQD_MERGE");
+    const bool any = s && s[0] == '1';
+    if ((s && s[0] == '0') || e->shaped || e->single_stream) return;
+    int64_t elems = 0, nodes = 0;
+    int esig = -1, fsig = -1;
+    bool eok = true, nok = true;
+    for (const eqd_handle *h : e->hs) {
+        elems += h->n_reg + h->n_pml;
+        nodes += count_of(h, kKNode3) + count_of(h, kKNodePml) + count_of(h, kKFault);
+        size_t lr, lp, lf;
+        const int a = variant<R>(h, kKElem, &lr), b = variant<R>(h, kKPml, &lp), f = variant<R>(h, kKFault, &lf);
+        eok = eok && h->n_reg > 0 && h->n_pml > 0 && !h->n_tile && !h->n_ptile && ((a >> 2) & 3) == 1 &&
+              (a >> 5) == ((b >> 3) & 3) && (esig < 0 || esig == a);
+        esig = a;
+        nok = nok && h->F.nf > 0 && h->PN.n_outer > 0 && count_of(h, kKNode3) > 0 && (fsig < 0 || fsig == f);
+        fsig = f;
+    }
+    e->merge_elems = eok && (any || elems <= kMergeElems);
+    e->merge_nodes = nok && (any || nodes <= (fsig ? kMergeNodesLearned : kMergeNodes));
+}
+
 // launch groups and per-scenario descriptors for the current tune
 template <typename R>
 int build(eqd_engine *e)
@@ -153,12 +196,15 @@ int build(eqd_engine *e)
     drop_graph(e);
     free_tables(e);
     const int n = (int)e->hs.size();
+    step_merged<R>(e);
     std::vector<Member<R>> M(n);
     for (int m = 0; m < n; m++) M[m] = make_member<R>(e, e->hs[m]);
     for (int kind = 0; kind < kKinds; kind++) {
         if (kind == kKClock) continue;
         int tuned = e->tune.block[kind];
         if (kind == kKStation) tuned = 64;
+        if (e->merge_elems && (kind == kKElem || kind == kKPml)) tuned = kMergeElemBlock;
+        if (e->merge_nodes && (kind == kKNode3 || kind == kKNodePml || kind == kKFault)) tuned = kMergeNodeBlock;
         std::map<int, Group> by;
         for (int m = 0; m < n; m++) {
             if (count_of(e->hs[m], kind) == 0) continue;
@@ -184,7 +230,9 @@ int build(eqd_engine *e)
             if (blocks > 0x7fffffff) return fail(e, EQD_EINVAL, "launch %s too large", kKindName[kind]);
             g.g.grid = (unsigned)blocks;
             g.g.block = block;
-            g.g.remap = e->tune.remap[kind];
+            g.g.remap = (e->merge_elems && kind <= kKPml) || (e->merge_nodes && kind >= kKNode3 && kind <= kKFault)
+                            ? 0
+                            : e->tune.remap[kind];
             // without a table every block reads scenario 0: only right when the
             // engine has no other scenario (a group of one scenario m > 0
             // still needs its table)
@@ -285,7 +333,13 @@ int enqueue_step(eqd_engine *e)
         const Stamp p = take_timer(e, kKStation, 1);
         HIPCHK(e, launch_step_start<R>(dM, (int)e->hs.size(), st, p.start(0), p.stop(0)));
     }
-    {
+    // (a step that carries timer events runs one launch per kind)
+    const bool both = e->merge_elems && !e->sample && ge.size() == 1 && e->groups[kKPml].size() == 1;
+    if (both) {
+        const int sig = ge[0].sig;
+        HIPCHK(e, launch_both<R>(dM, ge[0].g, e->groups[kKPml][0].g, sig & 1, (sig >> 1) & 1, (sig >> 4) & 1,
+                                 (sig >> 5) & 3, nstart, st));
+    } else {
         const Stamp p = take_timer(e, kKElem, ge.size());
         for (size_t i = 0; i < ge.size(); i++) {
             const Group &g = ge[i];
@@ -293,7 +347,7 @@ int enqueue_step(eqd_engine *e)
                                      (g.sig >> 5) & 3, i == 0 ? nstart : 0, st, p.start(i), p.stop(i)));
         }
     }
-    {
+    if (!both) {
         const auto &gs = e->groups[kKPml];
         const Stamp p = take_timer(e, kKPml, gs.size());
         for (size_t i = 0; i < gs.size(); i++) {
@@ -301,6 +355,13 @@ int enqueue_step(eqd_engine *e)
             HIPCHK(e, launch_pml<R>(dM, g.g, g.sig & 3, (g.sig >> 2) & 1, (g.sig >> 3) & 3, g.sig >> 5, st, p.start(i),
                                     p.stop(i)));
         }
+    }
+    if (e->merge_nodes && !e->sample && e->groups[kKFault].size() == 1 && e->groups[kKNodePml].size() == 1 &&
+        e->groups[kKNode3].size() == 1) {
+        for (const Group &g : e->groups[kKTp]) HIPCHK(e, launch_thermop<R>(dM, g.g, st));
+        const Group &f = e->groups[kKFault][0];
+        HIPCHK(e, launch_nodes<R>(dM, f.g, e->groups[kKNodePml][0].g, e->groups[kKNode3][0].g, f.sig, st));
+        return EQD_OK;
     }
     // fork: the fault pairs on the second stream, beside the node kernels
     // (EQD_SINGLE_STREAM=1 keeps them on the main stream, in step order)
@@ -585,6 +646,7 @@ int tune_impl(eqd_engine *e, int32_t steps, std::string &report)
     int rc = copy_regions(e, regs, true);
     const int32_t timing = e->timing;
     e->timing = 1;
+    e->shaped = true;
     e->no_harvest = true;
     struct Cand {
         int block, remap;
@@ -744,6 +806,7 @@ int engine_set_launch(eqd_engine *e, int kind, int block, int remap)
     if (remap != 0 && remap != 1) return fail(e, EQD_EINVAL, "remap must be 0 or 1");
     e->tune.block[kind] = block;
     e->tune.remap[kind] = kind == kKFault ? 0 : remap;
+    e->shaped = true;
     e->built = false;
     drop_graph(e);
     return EQD_OK;

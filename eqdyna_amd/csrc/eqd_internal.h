@@ -22,6 +22,12 @@ template <typename R>
 hipError_t launch_pml(const Member<R> *, const LaunchGrid &, int hg, int mass, int ops, int tiled, hipStream_t,
                       hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
 template <typename R>
+hipError_t launch_both(const Member<R> *, const LaunchGrid &reg, const LaunchGrid &pml, int q, int dp, int mass, int ops,
+                       int nstart, hipStream_t);
+template <typename R>
+hipError_t launch_nodes(const Member<R> *, const LaunchGrid &fault, const LaunchGrid &pml, const LaunchGrid &node3,
+                        int learn, hipStream_t);
+template <typename R>
 hipError_t launch_node3(const Member<R> *, const LaunchGrid &, hipStream_t, hipEvent_t t0 = nullptr,
                         hipEvent_t t1 = nullptr);
 template <typename R>
@@ -84,6 +90,8 @@ struct eqd_engine {
     void *d_members = nullptr;  // Member<R>[hs.size()]
     std::vector<eqd::Group> groups[eqd::kKinds];
     eqd::Tune tune{};
+    bool shaped = false;        // launch shapes were chosen by the caller or the tuner
+    bool merge_elems = false, merge_nodes = false;  // step_merged's choice at the last build
     bool built = false;
     int64_t built_version = -1;  // sum of the scenarios' versions at the last build
     bool no_harvest = false;     // set while tuning

@@ -14,6 +14,8 @@
 // operation is the one the reference performs.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
+
 #include "eqd_device.h"
 
 namespace eqd {
@@ -1186,6 +1188,17 @@ __device__ __forceinline__ void finish_tile(const RegElems<R> &E, const NodeStat
     }
 }
 
+// A class's operator tables into LDS (kOpsLds); returns what lies behind them.
+template <typename R, typename E>
+__device__ __forceinline__ lds_ptr<R> stage_tables(const E &X, lds_ptr<R> tables)
+{
+    lds_ptr<R> lph = tables + X.n_opc * kOpW;
+    for (int j = threadIdx.x; j < X.n_opc * kOpW; j += blockDim.x) tables[j] = X.optab[j];
+    for (int j = threadIdx.x; j < X.n_phic * 32; j += blockDim.x) lph[j] = X.phitab[j];
+    __syncthreads();
+    return lph + X.n_phic * 32;
+}
+
 // One workgroup: the step start of a scenario, or a tile of elements with its
 // inner nodes, or (no tiles) blockDim.x elements.
 //
@@ -1222,11 +1235,7 @@ __global__ void __launch_bounds__(256, (kOps == kOpsGeom && !kQ && !kDP && !kMas
     const unsigned b = gb - (unsigned)M.blk0[kKElem];
     lds_ptr<R> tables = (lds_ptr<R>)eqd_smem, stage = tables;
     if constexpr (kOps == kOpsLds) {
-        lds_ptr<R> lph = tables + E.n_opc * kOpW;
-        for (int j = threadIdx.x; j < E.n_opc * kOpW; j += blockDim.x) tables[j] = E.optab[j];
-        for (int j = threadIdx.x; j < E.n_phic * 32; j += blockDim.x) lph[j] = E.phitab[j];
-        __syncthreads();
-        stage = lph + E.n_phic * 32;
+        stage = stage_tables<R>(E, tables);
     }
     if (!E.tile) {
         const int64_t t = (int64_t)b * blockDim.x + threadIdx.x;
@@ -1934,12 +1943,7 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 8 ? (kTile ? 2 : 3) : (kOps
     const unsigned b = gb - (unsigned)M.blk0[kKPml];
     lds_ptr<R> tables = (lds_ptr<R>)eqd_smem, stage = tables;
     if constexpr (kOps == kOpsLds) {
-        // class tables staged in LDS, as in elem_regular_kernel
-        lds_ptr<R> lph = tables + E.n_opc * kOpW;
-        for (int j = threadIdx.x; j < E.n_opc * kOpW; j += blockDim.x) tables[j] = E.optab[j];
-        for (int j = threadIdx.x; j < E.n_phic * 32; j += blockDim.x) lph[j] = E.phitab[j];
-        __syncthreads();
-        stage = lph + E.n_phic * 32;
+        stage = stage_tables<R>(E, tables);
     }
     if constexpr (kTile) {
         const Tile T = E.tile[b];
@@ -1952,6 +1956,37 @@ __global__ void __launch_bounds__(256, (sizeof(R) == 8 ? (kTile ? 2 : 3) : (kOps
         const int64_t p = (int64_t)b * blockDim.x + threadIdx.x;
         R d[1];
         if (p < E.n) pml_element<R, kHG, kMass, kOps, false>(E, N, C, p, tables, stage, d);
+    }
+}
+
+// Both element classes in one launch, for scenarios too small to fill the chip
+// with either (step_merged): blocks past the step starts are nreg blocks of
+// regular elements, then PML elements.
+template <typename R, bool kQ, bool kDP, bool kMass, int kOps>
+__global__ void __launch_bounds__(256)
+    elem_both_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ breg,
+                     const uint16_t *__restrict__ bpml, unsigned nreg, int nstart)
+{
+    const int nskip = step_start_skip(nstart);
+    if ((int)blockIdx.x < nskip) {
+        if ((int)blockIdx.x < nstart) step_start_block<R>(Ms[blockIdx.x]);
+        return;
+    }
+    extern __shared__ __attribute__((aligned(16))) unsigned char eqd_smem[];
+    lds_ptr<R> tables = (lds_ptr<R>)eqd_smem;
+    unsigned gb = blockIdx.x - (unsigned)nskip;
+    if (gb < nreg) {
+        const Member<R> &M = Ms[member_of(breg, gb)];
+        if constexpr (kOps == kOpsLds) (void)stage_tables<R>(M.E, tables);
+        const int64_t t = (int64_t)(gb - (unsigned)M.blk0[kKElem]) * blockDim.x + threadIdx.x;
+        if (t < M.E.n) regular_element<R, kQ, kDP, 1, kMass, kOps>(M.E, M.N, M.C, t, tables, false, tables);
+    } else {
+        gb -= nreg;
+        const Member<R> &M = Ms[member_of(bpml, gb)];
+        if constexpr (kOps == kOpsLds) (void)stage_tables<R>(M.P, tables);
+        const int64_t p = (int64_t)(gb - (unsigned)M.blk0[kKPml]) * blockDim.x + threadIdx.x;
+        R d[1];
+        if (p < M.P.n) pml_element<R, 1, kMass, kOps, false>(M.P, M.N, M.C, p, tables, tables, d);
     }
 }
 
@@ -2017,12 +2052,8 @@ __device__ __forceinline__ void gather3_ell(const uint32_t *ell, int64_t i, cons
 // Node kernel for 3-component nodes that are neither split nodes nor inner
 // nodes of a tile: gather, then node3_update.
 template <typename R>
-__global__ void __launch_bounds__(256) node3_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem,
-                                                    int remap)
+__device__ __forceinline__ void node3_one(const Member<R> &M, int64_t i)
 {
-    const unsigned gb = launch_block(remap);
-    const Member<R> &M = Ms[member_of(bmem, gb)];
-    const int64_t i = (int64_t)(gb - (unsigned)M.blk0[kKNode3]) * blockDim.x + threadIdx.x;
     const Clock ck = *M.clk;
     if (i == 0) M.clk->done = ck.nt;
     if (i >= M.n_node3_free) return;
@@ -2040,15 +2071,20 @@ __global__ void __launch_bounds__(256) node3_kernel(const Member<R> *__restrict_
     node3_update<R>(N, node, S, F, dt, mode, next_step);
 }
 
-// 12-component (PML) nodes; the gather reads only PML element forces because
-// regular elements never touch a PML node (checked on the host).
 template <typename R>
-__global__ void __launch_bounds__(256) node_pml_kernel(const Member<R> *__restrict__ Ms,
-                                                       const uint16_t *__restrict__ bmem, int remap)
+__global__ void __launch_bounds__(256) node3_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bmem,
+                                                    int remap)
 {
     const unsigned gb = launch_block(remap);
     const Member<R> &M = Ms[member_of(bmem, gb)];
-    const int64_t q = (int64_t)(gb - (unsigned)M.blk0[kKNodePml]) * blockDim.x + threadIdx.x;
+    node3_one<R>(M, (int64_t)(gb - (unsigned)M.blk0[kKNode3]) * blockDim.x + threadIdx.x);
+}
+
+// 12-component (PML) nodes; the gather reads only PML element forces because
+// regular elements never touch a PML node (checked on the host).
+template <typename R>
+__device__ __forceinline__ void node_pml_one(const Member<R> &M, int64_t q)
+{
     if (q >= M.PN.n_outer) return;
     const NodeState N = M.N;
     const PmlNodes P = M.PN;
@@ -2110,6 +2146,15 @@ __global__ void __launch_bounds__(256) node_pml_kernel(const Member<R> *__restri
     NodePml S;
     node_pml_load<R>(N, P, q, node, S);
     node_pml_update<R>(N, P, q, node, S, F, dt, mode, next_step);
+}
+
+template <typename R>
+__global__ void __launch_bounds__(256) node_pml_kernel(const Member<R> *__restrict__ Ms,
+                                                       const uint16_t *__restrict__ bmem, int remap)
+{
+    const unsigned gb = launch_block(remap);
+    const Member<R> &M = Ms[member_of(bmem, gb)];
+    node_pml_one<R>(M, (int64_t)(gb - (unsigned)M.blk0[kKNodePml]) * blockDim.x + threadIdx.x);
 }
 
 // Pending update at the start of a run: v += a*dt from the stored F/m
@@ -2250,13 +2295,8 @@ __device__ __forceinline__ double rsf_state(int friclaw, double V2, double state
 // then: lanes past the last pair read pair nf-1 and write only their own
 // padding rows of fric, then leave).
 template <typename R, bool kLearn>
-__global__ void __launch_bounds__(128, EQD_FAULT_WAVES) fault_kernel(const Member<R> *__restrict__ Ms,
-                                                                      const uint16_t *__restrict__ bmem)
+__device__ __forceinline__ void fault_pair(const Member<R> &M, int64_t i0, __bf16 *mlp_lds0, __bf16 *mlp_lds)
 {
-    __shared__ __attribute__((aligned(16))) __bf16 mlp_lds0[kLearn ? 2 * 64 * kLd0 : 8];
-    __shared__ __attribute__((aligned(16))) __bf16 mlp_lds[kLearn ? 2 * 64 * kLd : 8];
-    const unsigned gb = blockIdx.x;
-    const Member<R> &M = Ms[member_of(bmem, gb)];
     const FaultState Fs = M.F;
     const NodeState N = M.N;
     const StepConsts C = M.C;
@@ -2264,7 +2304,6 @@ __global__ void __launch_bounds__(128, EQD_FAULT_WAVES) fault_kernel(const Membe
     const Clock ck = *M.clk;
     const int nt = ck.nt, mode = ck.mode;
     const double time = ck.time;
-    const int64_t i0 = (int64_t)(gb - (unsigned)M.blk0[kKFault]) * blockDim.x + threadIdx.x;
     if (!kLearn && i0 >= Fs.nf) return;
     const bool active = i0 < Fs.nf;
     const int64_t i = active ? i0 : Fs.nf - 1;
@@ -2634,6 +2673,45 @@ __global__ void __launch_bounds__(128, EQD_FAULT_WAVES) fault_kernel(const Membe
     flag_nan(N, nm, nt + 1, vm[0], vm[1], vm[2]);
 }
 
+template <typename R, bool kLearn>
+__global__ void __launch_bounds__(128, EQD_FAULT_WAVES) fault_kernel(const Member<R> *__restrict__ Ms,
+                                                                      const uint16_t *__restrict__ bmem)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 mlp_lds0[kLearn ? 2 * 64 * kLd0 : 8];
+    __shared__ __attribute__((aligned(16))) __bf16 mlp_lds[kLearn ? 2 * 64 * kLd : 8];
+    const unsigned gb = blockIdx.x;
+    const Member<R> &M = Ms[member_of(bmem, gb)];
+    fault_pair<R, kLearn>(M, (int64_t)(gb - (unsigned)M.blk0[kKFault]) * blockDim.x + threadIdx.x, mlp_lds0, mlp_lds);
+}
+
+// The fault pairs, the PML nodes and the 3-component nodes in one launch, for
+// scenarios whose nodes all have a wave's place at once (step_merged): blocks
+// of pairs (the longest) first, then nfault .. of PML nodes, then npml .. of
+// the others.
+template <typename R, bool kLearn>
+__global__ void __launch_bounds__(128, EQD_FAULT_WAVES)
+    nodes_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bfault, const uint16_t *__restrict__ bpml,
+                 const uint16_t *__restrict__ bnode3, unsigned nfault, unsigned npml)
+{
+    __shared__ __attribute__((aligned(16))) __bf16 mlp_lds0[kLearn ? 2 * 64 * kLd0 : 8];
+    __shared__ __attribute__((aligned(16))) __bf16 mlp_lds[kLearn ? 2 * 64 * kLd : 8];
+    unsigned gb = blockIdx.x;
+    auto item = [&](const Member<R> &M, int kind) -> int64_t {
+        return (int64_t)(gb - (unsigned)M.blk0[kind]) * blockDim.x + threadIdx.x;
+    };
+    if (gb < nfault) {
+        const Member<R> &M = Ms[member_of(bfault, gb)];
+        fault_pair<R, kLearn>(M, item(M, kKFault), mlp_lds0, mlp_lds);
+    } else if ((gb -= nfault) < npml) {
+        const Member<R> &M = Ms[member_of(bpml, gb)];
+        node_pml_one<R>(M, item(M, kKNodePml));
+    } else {
+        gb -= npml;
+        const Member<R> &M = Ms[member_of(bnode3, gb)];
+        node3_one<R>(M, item(M, kKNode3));
+    }
+}
+
 // The start of a step as a launch of its own, one block per scenario (used
 // when a step has no regular-element launch to carry it).
 template <typename R>
@@ -2814,6 +2892,52 @@ hipError_t launch_pml(const Member<R> *M, const LaunchGrid &g, int hg, int mass,
     return hipGetLastError();
 }
 
+// Both element classes (stiffness hourglass, operators from the same place) in
+// one launch.
+template <typename R>
+hipError_t launch_both(const Member<R> *M, const LaunchGrid &gr, const LaunchGrid &gp, int q, int dp, int mass, int ops,
+                       int nstart, hipStream_t s)
+{
+    if (gr.block != gp.block || gr.block < 64 || gr.block > 256 || gr.block % 64 || gr.remap || gp.remap || nstart < 0)
+        return hipErrorInvalidValue;
+    const unsigned grid = gr.grid + gp.grid + (unsigned)step_start_skip(nstart);
+    constexpr int kGeoOr = sizeof(R) == sizeof(float) ? kOpsGeom : kOpsCompact;
+    if (ops < kOpsRows || ops > kOpsGeom || (ops == kOpsGeom && sizeof(R) != sizeof(float))) return hipErrorInvalidValue;
+    // class tables, or each PML thread's staged dN/dx (launch_pml)
+    const size_t lds = ops == kOpsLds ? std::max(gr.lds, gp.lds)
+                                      : (ops == kOpsGeom ? 0 : (EQD_STAGE_SHP_PML ? (size_t)gp.block * 24 * sizeof(R) : 0));
+#define EQD_BOTH(Q, DP, MASS, OPS) \
+    elem_both_kernel<R, Q, DP, MASS, OPS><<<grid, gr.block, lds, s>>>(M, gr.bmem, gp.bmem, gr.grid, nstart)
+#define EQD_BOTH_OPS(Q, DP, MASS)                                    \
+    do {                                                             \
+        if (ops == kOpsLds) EQD_BOTH(Q, DP, MASS, kOpsLds);          \
+        else if (ops == kOpsGeom) EQD_BOTH(Q, DP, MASS, kGeoOr);     \
+        else if (ops == kOpsCompact) EQD_BOTH(Q, DP, MASS, kOpsCompact); \
+        else EQD_BOTH(Q, DP, MASS, kOpsRows);                        \
+    } while (0)
+    if (q && mass) EQD_BOTH_OPS(true, false, true);
+    else if (q) EQD_BOTH_OPS(true, false, false);
+    else if (dp) EQD_BOTH_OPS(false, true, true);
+    else if (mass) EQD_BOTH_OPS(false, false, true);
+    else EQD_BOTH_OPS(false, false, false);
+#undef EQD_BOTH_OPS
+#undef EQD_BOTH
+    return hipGetLastError();
+}
+
+// Fault pairs and nodes in one launch.
+template <typename R>
+hipError_t launch_nodes(const Member<R> *M, const LaunchGrid &gf, const LaunchGrid &gp, const LaunchGrid &g3, int learn,
+                        hipStream_t s)
+{
+    if ((gf.block != 64 && gf.block != 128) || gp.block != gf.block || g3.block != gf.block || gp.remap || g3.remap)
+        return hipErrorInvalidValue;
+    const unsigned grid = gf.grid + gp.grid + g3.grid;
+    if (learn) nodes_kernel<R, true><<<grid, gf.block, 0, s>>>(M, gf.bmem, gp.bmem, g3.bmem, gf.grid, gp.grid);
+    else nodes_kernel<R, false><<<grid, gf.block, 0, s>>>(M, gf.bmem, gp.bmem, g3.bmem, gf.grid, gp.grid);
+    return hipGetLastError();
+}
+
 template <typename R>
 hipError_t launch_node3(const Member<R> *M, const LaunchGrid &g, hipStream_t s, hipEvent_t t0, hipEvent_t t1)
 {
@@ -2885,6 +3009,10 @@ hipError_t launch_step_start(const Member<R> *M, int nmem, hipStream_t s, hipEve
                                        hipEvent_t, hipEvent_t);                                                       \
     template hipError_t launch_pml<R>(const Member<R> *, const LaunchGrid &, int, int, int, int, hipStream_t, hipEvent_t, \
                                       hipEvent_t);                                                                    \
+    template hipError_t launch_both<R>(const Member<R> *, const LaunchGrid &, const LaunchGrid &, int, int, int, int,  \
+                                       int, hipStream_t);                                                             \
+    template hipError_t launch_nodes<R>(const Member<R> *, const LaunchGrid &, const LaunchGrid &, const LaunchGrid &, \
+                                        int, hipStream_t);                                                            \
     template hipError_t launch_node3<R>(const Member<R> *, const LaunchGrid &, hipStream_t, hipEvent_t, hipEvent_t);  \
     template hipError_t launch_node_pml<R>(const Member<R> *, const LaunchGrid &, hipStream_t, hipEvent_t,            \
                                            hipEvent_t);                                                               \

@@ -11,13 +11,13 @@ namespace eqd {
 
 // Regular elements from which on a scenario runs in tiles.  Below about three
 // tiles per CU a launch is one chain of waits, which the barrier and the
-// nodes' loads lengthen: chunks of steps of 90,192 elements (dipping fault,
-// FP64) 10.07 -> 10.84 ms with tiles; 167,808 (plastic) 11.38 -> 10.54,
-// 200,000 (uniform, FP64) 14.94 -> 15.05, 686,000 (rough fault, FP64)
-// 55.4 -> 51.2, 2.17 M (layered with Q, FP32) 96.7 -> 91.9, 2.42 M (rough
-// fault, FP32) 214.1 -> 212.
-constexpr int64_t kTileMinElems = 131072;
-
+// nodes' loads lengthen, and elements without tiles share a launch with the
+// PML elements.  Step without tiles and with them: 148,000 elements (rough
+// fault, FP64) 112.2 and 121.9 us, FP32 74.0 and 75.6; 167,808 (plastic) 102.1
+// and 86.8, 200,000 (uniform, FP64) 115.9 and 101.2; chunks of 150 to 400 steps
+// of 686,000 (rough fault, FP64) 55.4 and 51.2 ms, 2.17 M (layered with Q, FP32)
+// 96.7 and 91.9.
+constexpr int64_t kTileMinElems = 163840;
 // The same for the PML elements, whose tiles have three barriers: 127,932
 // (plastic, FP64) neutral, ensembles of 130,000 at most (FP32) 22.1 -> 23.9 ms
 // with tiles, 232,000 (uniform, FP64) 15.03 -> 13.37, 466,000 (rough fault,

@@ -252,3 +252,50 @@ def test_element_order_does_not_change_results(name, monkeypatch):
     monkeypatch.setenv("EQD_ELEMENT_ORDER", "1")
     got = eager_run(name, "fp64", [nstep])
     assert_same(got, ref, f"{name} brick order")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,precision", [("box_sw", "fp64"), ("box_rsf4", "fp32"), ("box_q", "fp32"),
+                                            ("box_plastic", "fp64"), ("box_dip", "fp64"), ("box_rough", "fp32"),
+                                            ("box_tp", "fp64"), ("box_hg2", "fp64")])
+def test_merged_launches_match_launches_apart(name, precision, monkeypatch):
+    # both element classes in one launch, fault pairs and nodes in another
+    # (the default for small scenarios), against one launch per kind on two
+    # streams: every launch does the same work per element, node and pair; with
+    # timer events on every third step both forms alternate within a run
+    bundle, sc, _ = load_golden(name)
+    n = int(sc["nstep"])
+    guess = (learned.load()[0], 6, 0.5) if name in ("box_rsf4", "box_rough") else None
+    res = []
+    for merge, timing in (("0", 0), ("1", 0), ("1", 3)):
+        print(f"case {name} {precision} merge {merge} timing {timing}", flush=True)
+        monkeypatch.setenv("EQD_MERGE", merge)
+        s = Solver(bundle, sc, precision)
+        if guess:
+            s.set_guess(*guess)
+        s.set_timing(timing)
+        s.run(n // 3)
+        s.run(n - n // 3)
+        res.append(dict(outputs(s), stations=s.get("OffFaultStGramSCEC")))
+        s.close()
+    assert_same(res[1], res[0], f"{name} {precision} merged")
+    assert_same(res[2], res[0], f"{name} {precision} merged, sampled timing")
+
+
+@pytest.mark.gpu
+def test_merged_ensemble_replay(monkeypatch):
+    # slip weakening alone shares one kernel variant of each kind
+    names = ["box_sw", "box_c5sw", "box_layered"]
+    out = {}
+    for merge in ("0", "1"):
+        monkeypatch.setenv("EQD_MERGE", merge)
+        members = [Solver(*load_golden(n)[:2], "fp32") for n in names]
+        e = Ensemble(members)
+        for _ in range(3):  # replays of the captured step
+            e.run(6)
+        out[merge] = [outputs(m) for m in members]
+        e.close()
+        for m in members:
+            m.close()
+    for n, a, b in zip(names, out["1"], out["0"]):
+        assert_same(a, b, f"member {n} merged")

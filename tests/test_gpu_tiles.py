@@ -1,5 +1,5 @@
 """Elements in tiles, whose inner nodes the element kernels sum and update
-themselves (the default from 131,072 regular and 196,608 PML elements on,
+themselves (the default from 163,840 regular and 196,608 PML elements on,
 EQD_ELEMENT_ORDER=1 on any mesh), against the reference's element order: a
 node sums the same forces in the same order, so every output is the same bit
 for bit."""
