@@ -70,6 +70,12 @@ struct Group {
     uint16_t *d_bmem = nullptr;  // block-to-scenario table, owned (null when the engine has one scenario)
 };
 
+// captured steps
+struct StepGraph {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+};
+
 }  // namespace eqd
 
 struct eqd_handle;
@@ -95,9 +101,8 @@ struct eqd_engine {
     bool built = false;
     int64_t built_version = -1;  // sum of the scenarios' versions at the last build
     bool no_harvest = false;     // set while tuning
-    bool graph_on = false;  // replay one captured step instead of launching every step
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    bool graph_on = false;  // replay captured steps instead of launching every step
+    eqd::StepGraph one, many;  // a step, and several
     int32_t timing = 0;   // per-kernel event timing: 0 off, k: every k-th step of a run
     bool sample = false;  // the step being enqueued carries timer events
     std::map<std::string, eqd::KTimer> timers;
