@@ -98,6 +98,7 @@ template <typename T, typename S>
 static std::vector<T> to_blocks(const std::vector<S> &cm, int64_t n, int w)
 {
     std::vector<T> b((size_t)((n + 63) / 64 * 64 * w), T(0));
+#pragma omp parallel for schedule(static)
     for (int64_t t = 0; t < n; t++)
         for (int k = 0; k < w; k++) b[(size_t)(((t >> 6) * w + k) * 64 + (t & 63))] = (T)cm[(size_t)k * n + t];
     return b;
@@ -739,6 +740,7 @@ int eqd_commit(eqd_handle *h)
     auto node_blocks = [&](auto zero, const auto &cm) {
         using T = decltype(zero);
         std::vector<T> b((size_t)blocked_count(nn, 3), zero);
+#pragma omp parallel for schedule(static)
         for (int64_t n = 0; n < nn; n++)
             for (int k = 0; k < 3; k++) b[blocked_index(at(n), k, 3)] = (T)cm[(size_t)k * nn + n];
         return b;
@@ -1064,6 +1066,7 @@ int eqd_commit(eqd_handle *h)
             // NodeState); split nodes keep FP64 copies in the fault's arrays
             std::vector<float> hi(3 * nn), m32(nn);
             std::vector<uint16_t> lo(3 * nn);
+#pragma omp parallel for schedule(static)
             for (int64_t j = 0; j < 3 * nn; j++) {
                 hi[j] = (float)disp[j];
                 lo[j] = bf16_bits((float)(disp[j] - (double)hi[j]));

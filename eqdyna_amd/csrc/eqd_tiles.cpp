@@ -208,15 +208,24 @@ bool make_tiles(std::vector<int32_t> *const ids[2], const bool want[2], const in
     // so that a tile's inner nodes, and the nodes that the same tiles share,
     // are neighbours in memory.  Nodes of no tile come first.
     std::vector<int32_t> first((size_t)nn, -1), last((size_t)nn, -1), touch((size_t)nn, 0);
+    auto lower = [](int32_t &x, int32_t v) {
+        int32_t c = __atomic_load_n(&x, __ATOMIC_RELAXED);
+        while ((c < 0 || v < c) && !__atomic_compare_exchange_n(&x, &c, v, true, __ATOMIC_RELAXED, __ATOMIC_RELAXED)) {}
+    };
+    auto raise = [](int32_t &x, int32_t v) {
+        int32_t c = __atomic_load_n(&x, __ATOMIC_RELAXED);
+        while (v > c && !__atomic_compare_exchange_n(&x, &c, v, true, __ATOMIC_RELAXED, __ATOMIC_RELAXED)) {}
+    };
+#pragma omp parallel for schedule(dynamic, 64)
     for (int64_t k = 0; k < nt; k++) {
         const Tile &K = tile(k);
         const std::vector<int32_t> &el = *ids[k < nt0 ? 0 : 1];
         for (int32_t t = K.e0; t < K.e0 + K.ne; t++)
             for (int a = 0; a < 8; a++) {
                 const int32_t nd = ien[(int64_t)el[t] * 8 + a] - 1;
-                if (first[nd] < 0) first[nd] = (int32_t)k;
-                last[nd] = (int32_t)k;
-                touch[nd]++;
+                lower(first[nd], (int32_t)k);
+                raise(last[nd], (int32_t)k);
+                __atomic_fetch_add(&touch[nd], 1, __ATOMIC_RELAXED);
             }
     }
     auto inner = [&](int32_t nd) {
@@ -249,10 +258,10 @@ bool make_tiles(std::vector<int32_t> *const ids[2], const bool want[2], const in
     // per tile: its (node, element, local node) entries in the order a node
     // sums them; an inner node's become its row of node_ent, the others slots
     // in runs of neighbouring nodes' q-th entries, as the node kernels read them
-    struct Entry {
-        int32_t node, elem, q;
-        uint16_t src;  // staged force: local node * kTileElems + lane
-    };
+    // (an entry as one number: node, the element's rank in its tile, local node, lane)
+    auto node_of = [](uint64_t e) { return (int32_t)(e >> 24); };
+    auto src_of = [](uint64_t e) { return (uint16_t)((e >> 8 & 7) * kTileElems + (e & 255)); };
+    static_assert(kTileElems == 256, "lane and rank are 8 bits");
     for (int c = 0; c < 2; c++) {
         TileSet &S = T[c];
         const std::vector<int32_t> &el = *ids[c];
@@ -267,41 +276,49 @@ bool make_tiles(std::vector<int32_t> *const ids[2], const bool want[2], const in
         std::vector<std::vector<uint16_t>> tsrc((size_t)ntc);
 #pragma omp parallel
         {
-            std::vector<Entry> E, B;
+            std::vector<uint64_t> E;
+            std::vector<std::pair<int32_t, uint16_t>> B;  // q and source of a run's entries
+            std::vector<int32_t> byid;
 #pragma omp for schedule(dynamic, 16)
             for (int64_t k = 0; k < ntc; k++) {
                 const Tile &K = S.tile[k];
+                byid.assign(el.begin() + K.e0, el.begin() + K.e0 + K.ne);
+                std::sort(byid.begin(), byid.end());
                 E.clear();
-                B.clear();
                 for (int l = 0; l < K.ne; l++) {
                     const int32_t e = el[K.e0 + l];
+                    const uint64_t rank = std::lower_bound(byid.begin(), byid.end(), e) - byid.begin();
                     for (int a = 0; a < 8; a++)
-                        E.push_back(Entry{O.at[ien[(int64_t)e * 8 + a] - 1], e, 0, (uint16_t)(a * kTileElems + l)});
+                        E.push_back((uint64_t)O.at[ien[(int64_t)e * 8 + a] - 1] << 24 | rank << 16 | (uint64_t)a << 8 | l);
                 }
-                std::sort(E.begin(), E.end(), [](const Entry &x, const Entry &y) {
-                    if (x.node != y.node) return x.node < y.node;
-                    if (x.elem != y.elem) return x.elem < y.elem;
-                    return x.src < y.src;
-                });
-                for (size_t i = 0; i < E.size();) {
-                    const int32_t nd = E[i].node;
-                    for (int32_t q = 0; i < E.size() && E[i].node == nd; i++, q++) {
-                        if (O.inner[O.ref[nd]]) {
-                            S.node_ent[((int64_t)K.i0 + nd - K.n0) * 8 + q] = E[i].src;
-                        } else {
-                            E[i].q = q;
-                            B.push_back(E[i]);
+                std::sort(E.begin(), E.end());
+                // the other nodes in runs that the same tiles share: such nodes follow
+                // one another
+                auto flush = [&] {
+                    for (int32_t q = 0; !B.empty(); q++) {
+                        size_t left = 0;
+                        for (const auto &x : B) {
+                            if (x.first == q) tsrc[k].push_back(x.second);
+                            else B[left++] = x;
                         }
+                        B.resize(left);
+                    }
+                };
+                int32_t f = -1, g = -1;
+                for (size_t i = 0; i < E.size();) {
+                    const int32_t nd = node_of(E[i]), rn = O.ref[nd];
+                    const bool in = O.inner[rn] != 0;
+                    if (!in && (first[rn] != f || last[rn] != g)) {
+                        flush();
+                        f = first[rn];
+                        g = last[rn];
+                    }
+                    for (int32_t q = 0; i < E.size() && node_of(E[i]) == nd; i++, q++) {
+                        if (in) S.node_ent[((int64_t)K.i0 + nd - K.n0) * 8 + q] = src_of(E[i]);
+                        else B.push_back({q, src_of(E[i])});
                     }
                 }
-                std::sort(B.begin(), B.end(), [&](const Entry &x, const Entry &y) {
-                    const int32_t a = O.ref[x.node], b = O.ref[y.node];
-                    if (first[a] != first[b]) return first[a] < first[b];
-                    if (last[a] != last[b]) return last[a] < last[b];
-                    if (x.q != y.q) return x.q < y.q;
-                    return x.node < y.node;
-                });
-                for (const Entry &x : B) tsrc[k].push_back(x.src);
+                flush();
                 tsrc[k].resize((tsrc[k].size() + 63) / 64 * 64, kTileNone);
             }
         }
