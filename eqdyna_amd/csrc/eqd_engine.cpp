@@ -113,9 +113,13 @@ int variant(const eqd_handle *h, int kind, size_t *lds)
         return q | dp << 1 | hg << 2 | mass << 4 | ops << 5;
     }
     if (kind == kKPml) {
-        *lds = class_lds(pmls<R>(h), sizeof(R));
-        const int ops = ops_of(pmls<R>(h), *lds);
-        if (h->n_ptile) *lds += kPmlStage * kTileElems * sizeof(R);
+        // class tables stay in memory where they and a tile's stage (61,440 bytes
+        // in FP64) do not fit a workgroup's 64 KiB together
+        const size_t stage = h->n_ptile ? kPmlStage * kTileElems * sizeof(R) : 0;
+        size_t tables = class_lds(pmls<R>(h), sizeof(R));
+        if (tables + stage > 65536) tables = 0;
+        const int ops = ops_of(pmls<R>(h), tables);
+        *lds = tables + stage;
         return hg | mass << 2 | ops << 3 | (h->n_ptile ? 1 : 0) << 5;
     }
     if (kind == kKFault) return h->learn ? 1 : 0;

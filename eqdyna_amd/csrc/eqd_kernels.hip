@@ -1310,9 +1310,10 @@ __device__ __forceinline__ void node_pml_update(const NodeState &N, const PmlNod
 // accumulates the velocity gradients and hourglass mode amplitudes; pass 2
 // forms each node's 12 (or collapsed 3) force slots, hourglass included, and
 // writes every slot once.
-// At least 3 waves per SIMD in FP64 (4 in FP32): caps the FP64 per-element
-// variant at 168 VGPRs without spills (it would take 176, leaving 2 waves);
-// measured 0.324 -> 0.307 ms on the rough-fault box.
+// Without tiles at least 3 waves per SIMD in FP64 (4 in FP32): caps the FP64
+// per-element variant at 168 VGPRs without spills (it would take 176, leaving 2
+// waves); measured 0.324 -> 0.307 ms on the rough-fault box.
+//
 // kTile: the forces are staged in LDS (component c of local node a of lane l at
 // (a*3+c)*kTileElems + l, the six summed stresses behind them) and components
 // 10-12 of the nodes returned in d, to be staged once the others are used.
