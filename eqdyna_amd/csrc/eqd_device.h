@@ -160,7 +160,8 @@ __host__ __device__ __forceinline__ R phi_compact(const R *c, int m, int a, R s0
 }
 
 // One tile: elements [e0, e0 + ne) of a class, one workgroup.  Its
-// inner nodes, the ones that no element outside the tile touches, are nodes
+// inner nodes, of those that no element outside the tile touches at most one
+// per thread (kTileElems), are nodes
 // [n0, n0 + nn) with 8 entries each at tile_ent + i0, and the forces on its
 // other nodes leave through slots [64 s0, 64 s0 + ns) of ef in the order of
 // tile_src.  An entry names a force staged in LDS: local node * kTileElems +

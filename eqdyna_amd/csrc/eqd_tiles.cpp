@@ -228,7 +228,7 @@ bool make_tiles(std::vector<int32_t> *const ids[2], const bool want[2], const in
                 __atomic_fetch_add(&touch[nd], 1, __ATOMIC_RELAXED);
             }
     }
-    auto inner = [&](int32_t nd) {
+    auto own = [&](int32_t nd) {
         return first[nd] >= 0 && first[nd] == last[nd] && touch[nd] == degree[nd] && degree[nd] <= 8 &&
                kind[nd] == (first[nd] < nt0 ? 1 : 2);
     };
@@ -244,17 +244,22 @@ bool make_tiles(std::vector<int32_t> *const ids[2], const bool want[2], const in
 #pragma omp parallel for schedule(dynamic, 64)
     for (int64_t k = 0; k < nt; k++) {
         const auto b = O.ref.begin() + nstart[k + 1], e = O.ref.begin() + nstart[k + 2];
-        const auto mid = std::stable_partition(b, e, [&](int32_t n) { return inner(n); });
+        // A workgroup updates one node a thread.  Tiles among other elements own
+        // fewer nodes than elements, but one at free faces on opposite sides (a
+        // slab of any extent, or a mesh of one tile) owns up to
+        // (x + 1)(y + 1)(z + 1): those past the workgroup stay with the node kernels.
+        auto mid = std::stable_partition(b, e, [&](int32_t n) { return own(n); });
+        if (mid - b > kTileElems) mid = b + kTileElems;
         std::stable_sort(mid, e, [&](int32_t x, int32_t y) { return last[x] < last[y]; });
         tile(k).n0 = (int32_t)nstart[k + 1];
         tile(k).nn = (int32_t)(mid - b);
     }
     O.inner.assign((size_t)nn, 0);
 #pragma omp parallel for schedule(static)
-    for (int64_t i = 0; i < nn; i++) {
-        O.at[O.ref[i]] = (int32_t)i;
-        O.inner[O.ref[i]] = inner(O.ref[i]);
-    }
+    for (int64_t i = 0; i < nn; i++) O.at[O.ref[i]] = (int32_t)i;
+#pragma omp parallel for schedule(static)
+    for (int64_t k = 0; k < nt; k++)
+        for (int32_t i = tile(k).n0; i < tile(k).n0 + tile(k).nn; i++) O.inner[O.ref[i]] = 1;
     // per tile: its (node, element, local node) entries in the order a node
     // sums them; an inner node's become its row of node_ent, the others slots
     // in runs of neighbouring nodes' q-th entries, as the node kernels read them
