@@ -1713,13 +1713,11 @@ __device__ __forceinline__ void pml_element_modal(const PmlElems<R> &E, const No
         for (int a = 7; a >= 0; a--) fv[k][a] = fv[k][a] - fv[k][0];
         split8<R>(fv[k], vl[k], vh[k]);
         if (kHG == 1) {
+            // ut in FP64, rounded once, as pml_element forms it
 #pragma unroll
-            for (int a = 7; a >= 0; a--) fu[k][a] = fu[k][a] - fu[k][0];
+            for (int a = 7; a >= 0; a--)
+                fu[k][a] = (R)((double)(fu[k][a] - fu[k][0]) + C.rdampk * (double)fv[k][a]);
             split8<R>(fu[k], ul[k], uh[k]);
-#pragma unroll
-            for (int l = 0; l < 3; l++) ul[k][l] = ul[k][l] + rdk * vl[k][l];
-#pragma unroll
-            for (int m = 0; m < 4; m++) uh[k][m] = uh[k][m] + rdk * vh[k][m];
         }
     }
     R D[3][3];  // D[k][i]: gradient of velocity component k along i
