@@ -206,6 +206,7 @@ int build(eqd_engine *e)
     for (int m = 0; m < n; m++) M[m] = make_member<R>(e, e->hs[m]);
     for (int kind = 0; kind < kKinds; kind++) {
         if (kind == kKClock) continue;
+        if (kind == kKRecord && e->no_harvest) continue;  // make_member gives its kernel no recorder
         int tuned = e->tune.block[kind];
         if (kind == kKStation) tuned = 64;
         if (e->merge_elems && (kind == kKElem || kind == kKPml)) tuned = kMergeElemBlock;
@@ -713,8 +714,10 @@ int tune_impl(eqd_engine *e, int32_t steps, std::string &report)
     e->timing = timing;
     const int rc2 = copy_regions(e, regs, false);
     for (Region &x : regs) (void)hipFree(x.backup);
-    if (rc) return rc;
-    if (rc2) return rc2;
+    if (rc || rc2) {
+        e->built = false;  // the tables are the trial steps'
+        return rc ? rc : rc2;
+    }
     for (auto &kv : e->timers) {
         kv.second.total_ms = 0;
         kv.second.launches = 0;

@@ -174,3 +174,23 @@ def test_records_match_oracle_at_record_steps(name):
     es = np.abs(got_s - ref_s).max() / max(np.abs(ref_s).max(), 1e-300)
     print(f"[{name}] {len(steps)} records vs oracle: velocity {ev:.2e}, slip rate {es:.2e}", flush=True)
     assert ev <= TOL_FP64 and es <= TOL_FP64
+
+
+@pytest.mark.gpu
+def test_tuning_with_a_recorder():
+    # the tuner's trial steps launch no record kernel, and the records after
+    # tuning are those of an untuned run
+    bundle, sc, _ = load_golden("box_sw")
+    nodes = surface_nodes(bundle)
+    got = []
+    for tune in (False, True):
+        s = Solver(bundle, sc)
+        s.record(nodes, every=10, capacity=8)
+        s.run(15)
+        if tune:
+            s.tune(2)
+        s.run(20)
+        got.append(s.record_get(8))
+        s.close()
+    assert len(got[0][0]) == 4
+    assert np.array_equal(got[1][0], got[0][0]) and np.array_equal(got[1][1], got[0][1])
