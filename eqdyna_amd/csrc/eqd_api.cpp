@@ -749,7 +749,8 @@ int eqd_commit(eqd_handle *h)
     std::sort(n3free.begin(), n3free.end());
     std::sort(n3all.begin(), n3all.end());
     const int64_t nr = (int64_t)h->reg_ids.size(), np = (int64_t)h->pml_ids.size();
-    if (8 * (nr + 64) >= (int64_t)kEntSlotMask || 8 * (np + 64) >= (int64_t)kEntSlotMask) return fail(h, EQD_EINVAL, "too many elements in one class");
+    // (no tiles: slots of whole blocks of 64 elements)
+    if (!slots_fit(nr, 8) || !slots_fit(np, 8)) return fail(h, EQD_EINVAL, "too many elements in one class");
     h->n_reg = (int32_t)nr;
     h->n_pml = (int32_t)np;
     const bool fp32 = s.precision == EQD_PREC_FP32;

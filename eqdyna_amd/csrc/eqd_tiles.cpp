@@ -167,6 +167,7 @@ bool group(std::vector<int32_t> &ids, const Grid &G, double min_fill, std::vecto
     for (int64_t b = 0; b < nbox; b++) ntile += (start[b + 1] + kTileElems - 1) / kTileElems;
     // lanes without an element cost their share of every workgroup
     if ((double)n < min_fill * (double)(ntile * kTileElems)) return false;
+    if (!slots_fit(n, ntile)) return false;
     std::partial_sum(start.begin(), start.end(), start.begin());
     std::vector<int32_t> out((size_t)n);
     {

@@ -27,6 +27,11 @@ constexpr int64_t kTileMinPml = 196608;
 // Share of the tiles' lanes that must hold an element.
 constexpr double kTileMinFill = 0.625;
 
+// whether any slot of n elements in ntile tiles has a number that an entry of the
+// gather tables can hold: at most 8 slots an element, and each tile's are rounded up
+// to 64
+inline bool slots_fit(int64_t n, int64_t ntile) { return 8 * n + 64 * ntile < (int64_t)kEntSlotMask; }
+
 // one class's tiles (none: tile is empty)
 struct TileSet {
     std::vector<Tile> tile;

@@ -25,6 +25,7 @@ def lib(tmp_path_factory):
                     "-x", "hip", os.path.join(HERE, "tiles_host.cpp"), "-shared", "-o", out], check=True)
     L = C.CDLL(out)
     L.tiles_make.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int, C.c_int, C.c_double]
+    L.tiles_slots_fit.argtypes = [C.c_int64, C.c_int64]
     L.tiles_get.argtypes = [C.c_int, C.c_char_p, C.POINTER(C.c_int64)]
     L.tiles_get.restype = C.c_void_p
     return L
@@ -143,3 +144,13 @@ def test_a_class_that_does_not_fill_its_tiles_keeps_its_order(lib):
     check(lib, ien, nn, cls, kind)  # (ids of the other class: ascending, as they were)
     assert make(lib, ien, nn, cls, kind, (0, 1), 0.625) == 0
     assert np.array_equal(get(lib, 1, "ids", np.int32), np.flatnonzero(cls == 1))
+
+
+def test_slot_numbers_fit_a_table_entry(lib):
+    # an entry has 31 bits for the slot, one value of which means none; tiles
+    # that hold few elements each take 64 slots for one, more than the elements do
+    limit = 2**31 - 1
+    for n, ntile in ((1, 1), (100_000_000, 1_000_000), (33_554_431, 0), (2**25, 2**25), (2**24, 2**25), (2**28, 8),
+                     (2**28 - 9, 8), (2**28 - 65, 8)):
+        assert lib.tiles_slots_fit(n, ntile) == (8 * n + 64 * ntile < limit)
+    assert not lib.tiles_slots_fit(2**25, 2**25) and lib.tiles_slots_fit(2**25, 2**17)

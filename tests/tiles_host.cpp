@@ -30,6 +30,8 @@ int tiles_make(const int32_t *ien, const uint8_t *cls, int64_t ne, int64_t nn, c
                            g_order);
 }
 
+int tiles_slots_fit(int64_t n, int64_t ntile) { return eqd::slots_fit(n, ntile); }
+
 // an array of class c (or of the node order) and its number of values
 const void *tiles_get(int c, const char *what, int64_t *count)
 {
