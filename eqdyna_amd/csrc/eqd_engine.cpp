@@ -79,6 +79,19 @@ int64_t count_of(const eqd_handle *h, int kind)
     }
 }
 
+// every scenario that has the kind runs it in tiles: its launches are workgroups of
+// kTileElems whatever block size was asked for
+bool all_tiles(const eqd_engine *e, int kind)
+{
+    bool any = false;
+    for (const eqd_handle *h : e->hs) {
+        if (count_of(h, kind) == 0) continue;
+        any = true;
+        if (!(kind == kKElem ? h->n_tile : kind == kKPml ? h->n_ptile : 0)) return false;
+    }
+    return any;
+}
+
 // class tables of an element kind in LDS: both tables present and at most 16 KiB
 template <typename X>
 size_t class_lds(const X &E, size_t rsize)
@@ -681,7 +694,8 @@ int tune_impl(eqd_engine *e, int32_t steps, std::string &report)
             for (int b : {64, 128}) cands.push_back({b, 0, 0.0});
         } else {
             for (int b : {64, 128, 256})
-                for (int r : {0, 1}) cands.push_back({b, r, 0.0});
+                for (int r : {0, 1})
+                    if (b == kTileElems || !all_tiles(e, kind)) cands.push_back({b, r, 0.0});
         }
         for (Cand &c : cands) {
             e->tune.block[kind] = c.block;
@@ -906,7 +920,7 @@ int eqd_get_launch(eqd_handle *h, int32_t kind, int32_t *block, int32_t *remap)
     if (!h || !block || !remap) return EQD_EINVAL;
     if (!h->committed) return fail(h, EQD_ESTATE, "eqd_get_launch before eqd_commit");
     if (kind < 0 || kind > kKFault) return fail(h, EQD_EINVAL, "launch kind %d outside 0..4", kind);
-    *block = h->eng->tune.block[kind];
+    *block = all_tiles(h->eng, kind) ? kTileElems : h->eng->tune.block[kind];
     *remap = h->eng->tune.remap[kind];
     return EQD_OK;
 }

@@ -299,3 +299,30 @@ def test_merged_ensemble_replay(monkeypatch):
             m.close()
     for n, a, b in zip(names, out["1"], out["0"]):
         assert_same(a, b, f"member {n} merged")
+
+
+@pytest.mark.gpu
+def test_launch_shape_of_elements_in_tiles(monkeypatch):
+    # a tile is a workgroup of 256 whatever block size is asked for, and that is
+    # what is reported and tried; the node kinds take any
+    bundle, sc, _ = load_golden("box_rsf4")
+    n = 12
+    out = []
+    for order in ("0", "1"):
+        monkeypatch.setenv("EQD_ELEMENT_ORDER", order)
+        s = Solver(bundle, sc)
+        for kind in ("element", "element_pml", "node"):
+            s.set_launch(kind, 64, 1)
+        got = s.get_launch()
+        block = 64 if order == "0" else 256
+        assert got["element"] == (block, 1) and got["element_pml"] == (block, 1) and got["node"] == (64, 1)
+        s.run(n)
+        rep = s.tune(2)
+        for kind in ("element", "element_pml"):
+            shapes = [tuple(c[:2]) for c in rep[kind]["candidates"]]
+            assert shapes == [(b, r) for b in ((64, 128, 256) if order == "0" else (256,)) for r in (0, 1)]
+            assert (rep[kind]["block"], rep[kind]["remap"]) == s.get_launch()[kind]
+        s.run(n)
+        out.append(outputs(s))
+        s.close()
+    assert_same(out[1], out[0], "tiles with launch shapes set and tuned")
