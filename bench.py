@@ -14,7 +14,8 @@ Other workloads (c1, c2, c3) time one run in the --precision given; c5 is
 the batched ensemble (64 seeded scenarios of uneven size, FP32 bulk / FP64
 fault, advanced together as one graph-captured step per time step).
 Before the timed steps the launch-shape tuner (eqd_tune) picks block sizes
-and XCD remapping per kernel on the workload itself (--tune 0 skips it).
+and XCD remapping per kernel, or launches that kinds share, on the workload
+itself (--tune 0 skips it).
 
 A "step" is one explicit time step (src/driver.f90:9-34) over the whole mesh,
 with the mesh resident in HBM.  Prints one JSON line:
@@ -99,6 +100,11 @@ def load_traffic(workload: str, precision: str, kernel: str):
         return None, None
 
 
+def shapes_text(tuned: dict) -> str:
+    return ", ".join(f"{k} block {v['block']} remap {v['remap']} ({v['ms']:.4f} ms)" +
+                     (", in a shared launch" if v["merged"] else "") for k, v in tuned.items())
+
+
 def run_one(bundle, sc, precision: str, warmup: int, steps: int, guess=None, tune: int = 0, timing_every: int = 10):
     """One timed run: warm-up steps, the tuner (state restored), then `steps`
     timed, with per-kernel events on every `timing_every`-th of them."""
@@ -114,8 +120,7 @@ def run_one(bundle, sc, precision: str, warmup: int, steps: int, guess=None, tun
     tuned = None
     if tune > 0 and steps > tune + 1:
         tuned = s.tune(tune)
-        log(f"  tuner: " + ", ".join(f"{k} block {v['block']} remap {v['remap']} ({v['ms']:.4f} ms)"
-                                     for k, v in tuned.items()))
+        log(f"  tuner: " + shapes_text(tuned))
     s.set_timing(timing_every)
     s.run(min(warmup, 1))  # the launch tables for the chosen shapes are built here, not in the timed steps
     t0 = time.perf_counter()
@@ -123,22 +128,26 @@ def run_one(bundle, sc, precision: str, warmup: int, steps: int, guess=None, tun
     wall = time.perf_counter() - t0
     ktimes = {k: s.kernel_time(k) for k in ("element", "element_pml", "fault", "node", "node_pml", "station")}
     r = {"wall": wall, "ktimes": ktimes, "layout": layout, "nt": s.clock()[0], "newton": s.newton_stats(),
-         "fnft": s.get("fnft"), "fric": s.get("fric"), "launch": s.get_launch()}
+         "fnft": s.get("fnft"), "fric": s.get("fric"),
+         "launch": {k: {"block": b, "remap": m, "merged": bool(tuned and k in tuned and tuned[k]["merged"])}
+                    for k, (b, m) in s.get_launch().items()}, "tuned": tuned is not None}
     s.close()
     for k, (ms, n) in ktimes.items():
         log(f"  kernel {k}: {ms:.4f} ms avg over {n} launches")
     return r
 
 
-def run_graph(bundle, sc, precision: str, warmup: int, steps: int, guess=None, launch=None) -> float:
-    """The same run with every step replayed from one captured HIP graph (no
-    per-kernel events); returns its wall time."""
+def run_graph(bundle, sc, precision: str, warmup: int, steps: int, like: dict, guess=None) -> float:
+    """The run `like` (run_one) with every step replayed from one captured HIP
+    graph (no per-kernel events); returns its wall time."""
     from eqdyna_amd.solver import Solver
     s = Solver(bundle, sc, precision, device=0, nstep=warmup + steps)
     if guess is not None:
         s.set_guess(guess, GUESS["k_fallback"], GUESS["gate"])
-    for k, (b, r) in (launch or {}).items():
-        s.set_launch(k, b, r)
+    # (the tuner's shapes, unless it kept the shared launches a scenario starts with)
+    if like["tuned"] and not any(v["merged"] for v in like["launch"].values()):
+        for k, v in like["launch"].items():
+            s.set_launch(k, v["block"], v["remap"])
     s.set_graph(True)
     s.run(warmup)  # captures and instantiates the step graph outside the timed region
     t0 = time.perf_counter()
@@ -428,15 +437,15 @@ def main() -> int:
     if "fp64_value" in extra:
         extra["ratio_fp32_learned_vs_fp64"] = round(value / extra["fp64_value"], 4)
     if args.graph and args.workload == "c4":
-        w64 = run_graph(bundle, sc, "fp64", args.warmup, steps, launch=ref["launch"])
-        w32 = run_graph(bundle, sc, "fp32", args.warmup, steps, guess=params, launch=run["launch"])
+        w64 = run_graph(bundle, sc, "fp64", args.warmup, steps, ref)
+        w32 = run_graph(bundle, sc, "fp32", args.warmup, steps, run, guess=params)
         g64, g32 = 3.0 * nn * steps / w64 / 1e6, 3.0 * nn * steps / w32 / 1e6
         log(f"graph replay: fp64 {g64:.1f}, fp32+learned {g32:.1f} Mdof-steps/s")
         extra["graph_replay"] = {"fp64_value": round(g64, 2), "fp32_learned_value": round(g32, 2),
                                  "ratio": round(g32 / g64, 4),
                                  "note": "same steps replayed from one captured step; no per-kernel events"}
     elif args.graph:
-        wg = run_graph(bundle, sc, precision, args.warmup, steps, launch=run["launch"])
+        wg = run_graph(bundle, sc, precision, args.warmup, steps, run)
         g = 3.0 * nn * steps / wg / 1e6
         log(f"graph replay: {precision} {g:.1f} Mdof-steps/s")
         extra["graph_replay"] = {"value": round(g, 2), "ms_per_step": round(wg / steps * 1e3, 4),
@@ -479,7 +488,7 @@ def main() -> int:
                    "regular_elements": n_regular, "fault_pairs": int(sc["nftnd"]), "precision": precision,
                    "steps_run": run["nt"],
                    "layout": run["layout"],
-                   "launch_shapes": {k: {"block": b, "remap": r} for k, (b, r) in run["launch"].items()}, **extra},
+                   "launch_shapes": run["launch"], **extra},
         "roofline": roof, "cpu_baseline": cpu,
     }
     print(json.dumps(out), flush=True)
@@ -571,8 +580,7 @@ def bench_c5(args) -> int:
     if args.tune > 0:
         t = time.perf_counter()
         tuned = ens.tune(args.tune)
-        log(f"  tuner ({time.perf_counter() - t:.1f} s): " +
-            ", ".join(f"{k} block {v['block']} remap {v['remap']} ({v['ms']:.4f} ms)" for k, v in tuned.items()))
+        log(f"  tuner ({time.perf_counter() - t:.1f} s): " + shapes_text(tuned))
     t0 = time.perf_counter()
     ens.run(steps)  # graph replay; returns after the stream has drained
     wall = time.perf_counter() - t0

@@ -13,6 +13,7 @@
 // remapping per kind) are chosen by a tuner that times candidates on the
 // scenarios themselves and restores their state afterwards.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -178,7 +179,9 @@ void free_tables(eqd_engine *e)
 // network takes 24 KB of LDS a workgroup, up to kMergeNodesLearned (200,000
 // elements 88.3 -> 67.2; 1.4 M nodes and pairs 451.0 -> 476.6 us).  Workgroups of
 // 64, so that a small scenario's waves spread over the CUs.  The same bits in
-// either form; EQD_MERGE=0 keeps the launches apart, 1 merges at any size.
+// either form; EQD_MERGE=0 keeps the launches apart, 1 merges at any size; shapes
+// set by the caller keep them apart, and the tuner times both forms (a tuned box of
+// 2,800 elements would otherwise go back from 20 to 44 us a step).
 constexpr int64_t kMergeElems = 393216, kMergeNodes = 1500000, kMergeNodesLearned = 262144;
 constexpr int kMergeElemBlock = 64, kMergeNodeBlock = 64;
 
@@ -674,6 +677,7 @@ int tune_impl(eqd_engine *e, int32_t steps, std::string &report)
         }
     int rc = copy_regions(e, regs, true);
     const int32_t timing = e->timing;
+    const bool shaped = e->shaped;
     e->timing = 1;
     e->shaped = true;
     e->no_harvest = true;
@@ -681,9 +685,13 @@ int tune_impl(eqd_engine *e, int32_t steps, std::string &report)
         int block, remap;
         double ms;
     };
-    report = "{";
+    struct Choice {
+        int kind;
+        Cand best;
+        std::vector<Cand> cands;
+    };
+    std::vector<Choice> choices;
     const int kinds[] = {kKElem, kKPml, kKNode3, kKNodePml, kKFault};
-    bool first = true;
     for (int kind : kinds) {
         if (rc) break;
         bool any = false;
@@ -712,18 +720,47 @@ int tune_impl(eqd_engine *e, int32_t steps, std::string &report)
             if (c.ms < best->ms) best = &c;
         e->tune.block[kind] = best->block;
         e->tune.remap[kind] = best->remap;
-        char buf[160];
-        snprintf(buf, sizeof(buf), "%s\"%s\": {\"block\": %d, \"remap\": %d, \"ms\": %.5f, \"candidates\": [", first ? "" : ", ",
-                 kKindName[kind], best->block, best->remap, best->ms);
+        choices.push_back({kind, *best, cands});
+    }
+    // Shared launches, where the scenario runs them unasked, against the chosen
+    // shapes: whole steps as a run takes them (launched or replayed, no events),
+    // the better of three runs of each, since the two share no launch to time.
+    e->timing = 0;
+    e->shaped = false;
+    step_merged<R>(e);
+    e->shaped = true;
+    if (!rc && (e->merge_elems || e->merge_nodes)) {
+        double us[2];
+        for (int form = 0; form < 2 && !rc; form++) {
+            e->shaped = form == 0;
+            if ((rc = build<R>(e)) || (rc = copy_regions(e, regs, false)) || (rc = run<R>(e, steps, false))) break;
+            us[form] = 1e300;
+            for (int k = 0; k < 3 && !rc; k++) {
+                if ((rc = copy_regions(e, regs, false))) break;
+                const auto t0 = std::chrono::steady_clock::now();
+                rc = run<R>(e, steps, false);
+                us[form] = std::min(us[form],
+                                    std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count());
+            }
+        }
+        e->shaped = rc || us[0] < us[1];
+    }
+    report = "{";
+    for (const Choice &c : choices) {
+        const bool shared = !e->shaped && (c.kind <= kKPml ? e->merge_elems : e->merge_nodes);
+        char buf[200];
+        snprintf(buf, sizeof(buf), "%s\"%s\": {\"block\": %d, \"remap\": %d, \"ms\": %.5f, \"merged\": %s, \"candidates\": [",
+                 c.kind == choices[0].kind ? "" : ", ", kKindName[c.kind], c.best.block, c.best.remap, c.best.ms,
+                 shared ? "true" : "false");
         report += buf;
-        for (size_t i = 0; i < cands.size(); i++) {
-            snprintf(buf, sizeof(buf), "%s[%d, %d, %.5f]", i ? ", " : "", cands[i].block, cands[i].remap, cands[i].ms);
+        for (size_t i = 0; i < c.cands.size(); i++) {
+            snprintf(buf, sizeof(buf), "%s[%d, %d, %.5f]", i ? ", " : "", c.cands[i].block, c.cands[i].remap, c.cands[i].ms);
             report += buf;
         }
         report += "]}";
-        first = false;
     }
     report += "}";
+    if (rc) e->shaped = shaped;
     e->no_harvest = false;
     e->timing = timing;
     const int rc2 = copy_regions(e, regs, false);

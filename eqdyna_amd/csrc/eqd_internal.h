@@ -96,7 +96,7 @@ struct eqd_engine {
     void *d_members = nullptr;  // Member<R>[hs.size()]
     std::vector<eqd::Group> groups[eqd::kKinds];
     eqd::Tune tune{};
-    bool shaped = false;        // launch shapes were chosen by the caller or the tuner
+    bool shaped = false;        // one launch per kind: shapes set by the caller, or found faster by the tuner
     bool merge_elems = false, merge_nodes = false;  // step_merged's choice at the last build
     bool built = false;
     int64_t built_version = -1;  // sum of the scenarios' versions at the last build

@@ -335,17 +335,21 @@ int eqd_precompute(const eqd_precompute_args *a, int32_t *bad_elem, double *devi
 
 /* Block size (64, 128 or 256; fault pairs 64 or 128) and XCD remapping (1:
  * each of the 8 XCDs takes one contiguous range of the launch) of one kind.
- * Elements in tiles (eqd_layout_info) always run in blocks of 256, a tile
- * each: eqd_get_launch then gives 256, whatever was set. */
+ * Setting one gives every kind a launch of its own.  Elements in tiles
+ * (eqd_layout_info) always run in blocks of 256, a tile each: eqd_get_launch
+ * then gives 256, whatever was set. */
 int eqd_set_launch(eqd_handle *h, int32_t kind, int32_t block, int32_t remap);
 int eqd_get_launch(eqd_handle *h, int32_t kind, int32_t *block, int32_t *remap);
 
 /* Autotuner: times every launch shape of each kind (elements in tiles: the two
  * with blocks of 256) on the handle's own scenario (1 + steps steps per
  * candidate, state saved before and restored after, so the scenario does not
- * advance; needs nt + 1 + steps <= nstep), keeps the fastest, and writes a JSON
- * report (per kind: the choice, its milliseconds per launch and all candidates)
- * into report[report_cap]. */
+ * advance; needs nt + 1 + steps <= nstep) and keeps the fastest.  A scenario
+ * small enough to share launches between kinds until shapes are set or tuned
+ * (elements of both classes; fault pairs and nodes) keeps those where whole
+ * steps are faster with them.  Writes a JSON report (per kind: the choice, its
+ * milliseconds per launch, whether it runs in a shared launch instead, and all
+ * candidates) into report[report_cap]. */
 int eqd_tune(eqd_handle *h, int32_t steps, char *report, int64_t report_cap);
 
 /* on = 1: eqd_run captures one step as a HIP graph (once) and replays it;

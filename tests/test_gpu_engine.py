@@ -326,3 +326,31 @@ def test_launch_shape_of_elements_in_tiles(monkeypatch):
         out.append(outputs(s))
         s.close()
     assert_same(out[1], out[0], "tiles with launch shapes set and tuned")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ensemble", [False, True])
+def test_tuner_weighs_shared_launches(ensemble, monkeypatch):
+    # a small scenario runs two launches a step unless it is told otherwise
+    # (about half the time of one launch per kind): tuning keeps that, a launch
+    # shape set by the caller and EQD_MERGE=0 do not, and the results are the same
+    bundle, sc, _ = load_golden("box_sw")
+    n = 40
+    ref = eager_run("box_sw", "fp64", [n])
+    for merge in ("", "0"):
+        if merge:
+            monkeypatch.setenv("EQD_MERGE", merge)
+        members = [Solver(bundle, sc) for _ in range(2 if ensemble else 1)]
+        top = Ensemble(members) if ensemble else members[0]
+        rep = top.tune(4)
+        print(f"merge '{merge}' ensemble {ensemble}: {rep}", flush=True)
+        assert all(v["merged"] == (merge == "") for v in rep.values())
+        top.run(n // 2)
+        if not ensemble:
+            top.set_launch("node", 128, 0)
+        top.run(n - n // 2)
+        if ensemble:
+            top.close()
+        for s in members:
+            assert_same(outputs(s), ref, f"tuned, merge '{merge}'")
+            s.close()
