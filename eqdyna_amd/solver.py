@@ -188,11 +188,13 @@ class Solver:
             raise EqdError(rc, "eqd_create rejected the scalars")
         self.h = h
         try:
+            held = []  # eqd_commit reads the arrays: copies live until then
             for name in INPUTS:
                 if name not in bundle:
                     continue
                 fid, dt = FIELDS[name]
                 a = np.ascontiguousarray(bundle[name], dtype="<" + dt)
+                held.append(a)
                 self._check(self.L.eqd_set(self.h, fid, a.ctypes.data, a.size))
             if timing:
                 self._check(self.L.eqd_set_timing(self.h, 1))
