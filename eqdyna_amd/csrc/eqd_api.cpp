@@ -600,6 +600,10 @@ int eqd_commit(eqd_handle *h)
     h->pml_node_index.assign(nn, -1);
     std::vector<double> vel(3 * nn, 0.0), disp(3 * nn, 0.0), acc(3 * nn, 0.0);
     std::vector<double> pdamp, pv12, pacc;
+    const size_t n12 = (size_t)std::count(ndof, ndof + nn, 12);  // fixed nodes among them
+    pdamp.reserve(3 * n12);
+    pv12.reserve(12 * n12);
+    pacc.reserve(12 * n12);
     for (int64_t n = 0; n < nn; n++) {
         for (int k = 0; k < 3; k++) {
             vel[k * nn + n] = vel0 ? vel0[n * 3 + k] : 0.0;
@@ -652,6 +656,7 @@ int eqd_commit(eqd_handle *h)
     // per-PML-node arrays to component-major (then to blocks at upload)
     auto tr = [](const std::vector<double> &a, int64_t cnt, int w) {
         std::vector<double> b(a.size());
+#pragma omp parallel for schedule(static)
         for (int64_t q = 0; q < cnt; q++)
             for (int k = 0; k < w; k++) b[k * cnt + q] = a[q * w + k];
         return b;
@@ -719,7 +724,8 @@ int eqd_commit(eqd_handle *h)
                 if (h->pml_node_index[n] >= 0 && order.inner[n] == in) q.push_back(h->pml_node_index[n]);
         auto &id = h->pml_node_ids;
         auto take = [&](auto &v, int w) {  // component-major
-            auto old = v;
+            const auto old = v;
+#pragma omp parallel for collapse(2) schedule(static)
             for (int k = 0; k < w; k++)
                 for (int64_t i = 0; i < npn; i++) v[k * npn + i] = old[k * npn + q[i]];
         };
@@ -745,9 +751,23 @@ int eqd_commit(eqd_handle *h)
             for (int k = 0; k < 3; k++) b[blocked_index(at(n), k, 3)] = (T)cm[(size_t)k * nn + n];
         return b;
     };
-    std::vector<int32_t> n3free = in_place(h->node3_free), n3all = in_place(h->node3_all);
-    std::sort(n3free.begin(), n3free.end());
-    std::sort(n3all.begin(), n3all.end());
+    // the 3-component nodes in device order (given in the reference's)
+    std::vector<int32_t> n3free, n3all;
+    if (h->at.empty()) {
+        n3free = h->node3_free;
+        n3all = h->node3_all;
+    } else {
+        std::vector<uint8_t> three(nn, 0);
+        for (int32_t n : h->node3_all) three[n] = 1;
+        for (int32_t n : h->node3_free) three[n] = 2;
+        n3free.reserve(h->node3_free.size());
+        n3all.reserve(h->node3_all.size());
+        for (int64_t i = 0; i < nn; i++) {
+            const uint8_t t = three[order.ref[i]];
+            if (t) n3all.push_back((int32_t)i);
+            if (t == 2) n3free.push_back((int32_t)i);
+        }
+    }
     const int64_t nr = (int64_t)h->reg_ids.size(), np = (int64_t)h->pml_ids.size();
     // (no tiles: slots of whole blocks of 64 elements)
     if (!slots_fit(nr, 8) || !slots_fit(np, 8)) return fail(h, EQD_EINVAL, "too many elements in one class");
@@ -765,21 +785,22 @@ int eqd_commit(eqd_handle *h)
     for (int32_t e : h->reg_ids)
         if (etype[e] == 11 || etype[e] == 12) reg_wedges = true;
 
+    // the element masses are read by the inertia and gravity terms alone
+    const bool mass_term = s.rdampm != 0.0 || s.C_elastic == 0;
+
     // regular class SoA
     {
         std::vector<int32_t> r_ien(8 * nr);
         std::vector<double> r_shp(24 * nr), r_det(nr), r_lam(nr), r_mu(nr), r_vp(nr), r_rho(nr), r_st(nst * nr),
-            r_ss(6 * nr), r_phi(32 * nr), r_em(24 * nr), r_porep(nr), r_pstrain(nr);
+            r_ss(6 * nr), r_phi(32 * nr), r_em(mass_term ? 24 * nr : 0), r_porep(nr), r_pstrain(nr);
         std::vector<uint8_t> r_q(s.C_Q == 1 ? nr : 0);
         int qbad = 0;
 #pragma omp parallel for schedule(static) reduction(max : qbad)
         for (int64_t t = 0; t < nr; t++) {
             const int64_t e = h->reg_ids[t];
             for (int a = 0; a < 8; a++) r_ien[a * nr + t] = at(ien[e * 8 + a] - 1);
-            for (int i = 0; i < 24; i++) {
-                r_shp[i * nr + t] = shp[e * 24 + i];
-                r_em[i * nr + t] = emass[e * 24 + i];
-            }
+            for (int i = 0; i < 24; i++) r_shp[i * nr + t] = shp[e * 24 + i];
+            for (int i = 0; i < 24 && mass_term; i++) r_em[i * nr + t] = emass[e * 24 + i];
             r_det[t] = det[e];
             r_vp[t] = mat[0 * ne + e];
             r_rho[t] = mat[2 * ne + e];
@@ -872,7 +893,7 @@ int eqd_commit(eqd_handle *h)
                     return geometry_row<R>(xl, r_lam[t], r_mu[t], r_vp[t], r_rho[t], s.w, sh, r_det[t], s6, ph, row);
                 })))
                 return r2;
-            if (s.rdampm != 0.0 || s.C_elastic == 0) {
+            if (mass_term) {
                 if ((r2 = up(&E.emass, r_em, 24))) return r2;
             }
             R *p;
@@ -898,7 +919,7 @@ int eqd_commit(eqd_handle *h)
     {
         std::vector<int32_t> p_ien(8 * np);
         std::vector<double> p_shp(24 * np), p_det(np), p_lam(np), p_mu(np), p_vp(np), p_rho(np), p_st(21 * np),
-            p_ss(6 * np), p_phi(32 * np), p_em(24 * np), p_damp(3 * np);
+            p_ss(6 * np), p_phi(32 * np), p_em(mass_term ? 24 * np : 0), p_damp(3 * np);
         std::vector<uint8_t> p_mask(np);
 #pragma omp parallel for schedule(static)
         for (int64_t p = 0; p < np; p++) {
@@ -916,10 +937,8 @@ int eqd_commit(eqd_handle *h)
             double d[3];
             pml_elem_damping(s, xc, d);
             for (int i = 0; i < 3; i++) p_damp[i * np + p] = d[i];
-            for (int i = 0; i < 24; i++) {
-                p_shp[i * np + p] = shp[e * 24 + i];
-                p_em[i * np + p] = emass[e * 24 + i];
-            }
+            for (int i = 0; i < 24; i++) p_shp[i * np + p] = shp[e * 24 + i];
+            for (int i = 0; i < 24 && mass_term; i++) p_em[i * np + p] = emass[e * 24 + i];
             p_det[p] = det[e];
             p_vp[p] = mat[0 * ne + e];
             p_rho[p] = mat[2 * ne + e];
@@ -974,7 +993,7 @@ int eqd_commit(eqd_handle *h)
                     return geometry_row<R>(xl, p_lam[p], p_mu[p], p_vp[p], p_rho[p], s.w, sh, p_det[p], s6, ph, row);
                 })))
                 return r2;
-            if (s.rdampm != 0.0 || s.C_elastic == 0) {
+            if (mass_term) {
                 if ((r2 = up(&P.emass, p_em, 24))) return r2;
             }
             R *q;
