@@ -512,7 +512,8 @@ __device__ __forceinline__ double exact_u(const Member<R> &M, int node, int k)
 // displacement or velocity of every off-fault station row.  Every thread
 // reads the old clock before the barrier and thread 0 writes the new one
 // after it.  Later kernels of the step read the advanced clock from device
-// memory; the element kernels do not read it.
+// memory.  The regular elements, whose launch these blocks share, read only
+// what they do not write: in tiles Clock::done and run_end, else nothing.
 template <typename R>
 __device__ __forceinline__ void step_start_block(const Member<R> &M)
 {
@@ -677,12 +678,6 @@ __device__ __forceinline__ void node3_update(const NodeState &N, int node, const
 template <typename R>
 using lds_ptr = __attribute__((address_space(3))) R *;
 
-// kOps: where the operators come from (kOpsRows, kOpsLds, kOpsCompact).  With
-// kOpsLds both class tables are staged in LDS (dynamic shared memory of
-// (n_opc * kOpW + n_phic * 32) values) at block start, so the operator reads
-// of the element loop are LDS reads; with kOpsCompact Phi is rebuilt per node
-// (phi_compact) from 16 values read once per element; with kOpsGeom all
-// operators are rebuilt from the element's corner coordinates (geo_ops).
 // Stress update of a regular element from its strain rate (and, with Q, its
 // strain): Hooke's law, the Q memory variables, the Drucker-Prager return
 // (src/calcElemKU.f90:36-167).  srt: the stress rate; stress: the new stress,
@@ -872,8 +867,15 @@ __device__ __forceinline__ void regular_element_modal(const RegElems<R> &E, cons
     }
 }
 
-// stage: the tile's force buffer in LDS (component c of local node a of lane l
-// at (a*3+c)*kTileElems + l), or null to store the forces to their slots.
+// One regular element.
+// kOps: where the operators come from (kOpsRows, kOpsLds, kOpsCompact).  With
+// kOpsLds both class tables are staged in LDS (dynamic shared memory of
+// (n_opc * kOpW + n_phic * 32) values) at block start, so the operator reads
+// of the element loop are LDS reads; with kOpsCompact Phi is rebuilt per node
+// (phi_compact) from 16 values read once per element; with kOpsGeom all
+// operators are rebuilt from the element's corner coordinates (geo_ops).
+// staged: the forces go to the tile's buffer in LDS, stage (component c of local
+// node a of lane l at (a*3+c)*kTileElems + l), otherwise to their slots.
 template <typename R, bool kQ, bool kDP, int kHG, bool kMass, int kOps>
 __device__ __forceinline__ void regular_element(const RegElems<R> &E, const NodeState &N, const StepConsts &C, int64_t t,
                                                 lds_ptr<R> tables, bool staged, lds_ptr<R> stage)
@@ -2065,7 +2067,6 @@ __device__ __forceinline__ void node3_one(const Member<R> &M, int64_t i)
     const double dt = M.C.dt;
     const int mode = ck.mode, next_step = ck.nt + 1;
     const int node = M.node3_free[i];
-    const int64_t nn = N.nn;
     Node3 S;
     if constexpr (kAhead) node3_load<R>(N, node, S);
     double F[3];
@@ -2097,7 +2098,6 @@ __device__ __forceinline__ void node_pml_one(const Member<R> &M, int64_t q)
     const Clock ck = *M.clk;
     const int mode = ck.mode, next_step = ck.nt + 1;
     const int node = P.node[q];
-    const int64_t nn = N.nn;
     NodePml S;
     if constexpr (kAhead) node_pml_load<R>(N, P, q, node, S);
     double F[12];
@@ -2689,10 +2689,13 @@ __global__ void __launch_bounds__(128, EQD_FAULT_WAVES) fault_kernel(const Membe
     fault_pair<R, kLearn>(M, (int64_t)(gb - (unsigned)M.blk0[kKFault]) * blockDim.x + threadIdx.x, mlp_lds0, mlp_lds);
 }
 
-// The fault pairs, the PML nodes and the 3-component nodes in one launch, for
-// scenarios whose nodes all have a wave's place at once (step_merged): blocks
-// of pairs (the longest) first, then nfault .. of PML nodes, then npml .. of
-// the others.
+// The fault pairs, the PML nodes and the 3-component nodes in one launch, up to
+// the sizes of step_merged (kMergeNodes, kMergeNodesLearned): blocks of pairs
+// (the longest) first, then nfault .. of PML nodes, then npml .. of the others.
+// The pairs' 256 registers leave all of them two waves a SIMD.  Measured at both
+// ends: 2,800 elements in two launches a step instead of five 44.2 -> 20.5 us,
+// 1.3 M nodes and pairs 386.0 -> 377.4; with the learned guess 200,000 elements
+// 88.3 -> 67.2, and at 1.4 M nodes and pairs, past its line, 451.0 -> 476.6.
 template <typename R, bool kLearn>
 __global__ void __launch_bounds__(128, EQD_FAULT_WAVES)
     nodes_kernel(const Member<R> *__restrict__ Ms, const uint16_t *__restrict__ bfault, const uint16_t *__restrict__ bpml,

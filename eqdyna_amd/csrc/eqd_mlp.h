@@ -95,8 +95,8 @@ __device__ __forceinline__ void zero_acc(f32x16 acc[2][2])
 __device__ __forceinline__ int acc_row(int mt, int i) { return mt * 32 + 8 * (i >> 2) + 4 * ((threadIdx.x & 63) >> 5) + (i & 3); }
 __device__ __forceinline__ int acc_col(int nt) { return nt * 32 + (threadIdx.x & 31); }
 
-// out[m][n] = bf16(gelu(acc + bias[n])); when zsave is given it receives gelu'(z) (float, stride 64)
-__device__ __forceinline__ void epilogue_gelu(const f32x16 acc[2][2], const float *bias, __bf16 *out, float *gsave)
+// out[m][n] = bf16(gelu(acc + bias[n]))
+__device__ __forceinline__ void epilogue_gelu(const f32x16 acc[2][2], const float *bias, __bf16 *out)
 {
 #pragma unroll
     for (int mt = 0; mt < 2; mt++)
@@ -109,7 +109,6 @@ __device__ __forceinline__ void epilogue_gelu(const f32x16 acc[2][2], const floa
                 const int m = acc_row(mt, i);
                 const float z = acc[mt][nt][i] + b;
                 out[m * kLd + n] = to_bf16(gelu(z));
-                if (gsave) gsave[m * 64 + n] = gelu_grad(z);
             }
         }
 }
@@ -137,17 +136,17 @@ __device__ __forceinline__ float mlp_wave_forward(const MlpNet &M, const float x
     f32x16 acc[2][2];
     zero_acc(acc);
     wave_mm(buf0, kLd0, M.w1, kMlpK1, kMlpK1, acc);
-    epilogue_gelu(acc, M.b1, buf, nullptr);
+    epilogue_gelu(acc, M.b1, buf);
     __syncthreads();
     zero_acc(acc);
     wave_mm(buf, kLd, M.w2, 64, 64, acc);
     __syncthreads();
-    epilogue_gelu(acc, M.b2, buf, nullptr);
+    epilogue_gelu(acc, M.b2, buf);
     __syncthreads();
     zero_acc(acc);
     wave_mm(buf, kLd, M.w3, 64, 64, acc);
     __syncthreads();
-    epilogue_gelu(acc, M.b3, buf, nullptr);
+    epilogue_gelu(acc, M.b3, buf);
     __syncthreads();
     float y = M.b4[0];
     for (int n = 0; n < 64; n++) y = y + from_bf16(buf[l * kLd + n]) * M.w4r[n];
