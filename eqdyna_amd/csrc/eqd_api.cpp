@@ -9,6 +9,7 @@
 #include <cstring>
 #include <algorithm>
 #include <map>
+#include <memory>
 #include <string>
 #include <type_traits>
 #include <unordered_map>
@@ -83,8 +84,25 @@ static int dalloc(eqd_handle *h, T **p, int64_t count)
     return 0;
 }
 
+// Host arrays of the commit that are written in full, by all threads, straight
+// after they are made: their pages are then touched by the threads that fill
+// them, not first zeroed by one (3.46 M elements: 2.8 GB of them).
 template <typename T>
-static int dupload(eqd_handle *h, T **p, const std::vector<T> &v)
+struct NoInit : std::allocator<T> {
+    template <typename U>
+    struct rebind {
+        typedef NoInit<U> other;
+    };
+    template <typename U>
+    void construct(U *p) noexcept { ::new ((void *)p) U; }
+    template <typename U, typename... A>
+    void construct(U *p, A &&...a) { ::new ((void *)p) U(std::forward<A>(a)...); }
+};
+template <typename T>
+using Raw = std::vector<T, NoInit<T>>;
+
+template <typename T, typename A>
+static int dupload(eqd_handle *h, T **p, const std::vector<T, A> &v)
 {
     int rc = dalloc(h, p, (int64_t)v.size());
     if (rc) return rc;
@@ -94,13 +112,15 @@ static int dupload(eqd_handle *h, T **p, const std::vector<T> &v)
 
 // Component-major [w][n] values to the kernels' AoSoA blocks (blk_at<w>),
 // zero padded to whole blocks of 64 items.
-template <typename T, typename S>
-static std::vector<T> to_blocks(const std::vector<S> &cm, int64_t n, int w)
+template <typename T, typename S, typename A>
+static Raw<T> to_blocks(const std::vector<S, A> &cm, int64_t n, int w)
 {
-    std::vector<T> b((size_t)((n + 63) / 64 * 64 * w), T(0));
+    const int64_t padded = (n + 63) / 64 * 64;
+    Raw<T> b((size_t)(padded * w));
 #pragma omp parallel for schedule(static)
-    for (int64_t t = 0; t < n; t++)
-        for (int k = 0; k < w; k++) b[(size_t)(((t >> 6) * w + k) * 64 + (t & 63))] = (T)cm[(size_t)k * n + t];
+    for (int64_t t = 0; t < padded; t++)
+        for (int k = 0; k < w; k++)
+            b[(size_t)(((t >> 6) * w + k) * 64 + (t & 63))] = t < n ? (T)cm[(size_t)k * n + t] : T(0);
     return b;
 }
 static inline int64_t blocked_count(int64_t n, int w) { return (n + 63) / 64 * 64 * w; }
@@ -340,10 +360,10 @@ static bool geometry_row(const double xl[3][8], double lam, double mu, double vp
 // (kOpsGeom): 25 values per element instead of 51.
 template <typename R, typename E, typename OpRow, typename GeomRow>
 static int upload_operators(eqd_handle *h, E &X, int64_t n, bool no_classes, OpRow oprow,
-                            const std::vector<double> &shp, const std::vector<double> &phi, int64_t *n_op_classes,
+                            const Raw<double> &shp, const Raw<double> &phi, int64_t *n_op_classes,
                             int64_t *n_phi_classes, int32_t *compact, bool allow_geom, GeomRow geomrow)
 {
-    std::vector<R> cmp;
+    Raw<R> cmp;
     int ok = 1;
     const char *fe = std::getenv("EQD_FULL_PHI");
     if (!(fe && fe[0] == '1') && n > 0) {
@@ -395,12 +415,12 @@ static int upload_operators(eqd_handle *h, E &X, int64_t n, bool no_classes, OpR
     const int64_t nb = (n + 63) / 64;
     X.opb_geom = 0;
     if (allow_geom && ok) {
-        std::vector<R> g((size_t)(nb * 64 * kOpG), (R)0);
+        Raw<R> g((size_t)(nb * 64 * kOpG));
         int gok = 1;
 #pragma omp parallel for schedule(static) reduction(min : gok)
-        for (int64_t t = 0; t < n; t++) {
-            R row[kOpG];
-            if (!geomrow(t, row)) {
+        for (int64_t t = 0; t < nb * 64; t++) {
+            R row[kOpG] = {};  // zeros in the last block's padding
+            if (t < n && !geomrow(t, row)) {
                 gok = 0;
                 continue;
             }
@@ -421,14 +441,14 @@ static int upload_operators(eqd_handle *h, E &X, int64_t n, bool no_classes, OpR
         }
     }
     const int W = ok ? kOpBc : kOpB;
-    std::vector<R> b((size_t)(nb * 64 * W), (R)0);
+    Raw<R> b((size_t)(nb * 64 * W));
 #pragma omp parallel for schedule(static)
-    for (int64_t t = 0; t < n; t++) {
-        R row[kOpB];
-        oprow(t, row);
-        if (ok) {
+    for (int64_t t = 0; t < nb * 64; t++) {
+        R row[kOpB] = {};
+        if (t < n) oprow(t, row);
+        if (t < n && ok) {
             for (int i = 0; i < 16; i++) row[kOpW + i] = cmp[(size_t)t * 16 + i];
-        } else {
+        } else if (t < n) {
             phirow(t, row + kOpW);
         }
         R *dst = b.data() + (t / 64) * W * 64 + (t % 64);
@@ -600,10 +620,6 @@ int eqd_commit(eqd_handle *h)
     h->pml_node_index.assign(nn, -1);
     std::vector<double> vel(3 * nn, 0.0), disp(3 * nn, 0.0), acc(3 * nn, 0.0);
     std::vector<double> pdamp, pv12, pacc;
-    const size_t n12 = (size_t)std::count(ndof, ndof + nn, 12);  // fixed nodes among them
-    pdamp.reserve(3 * n12);
-    pv12.reserve(12 * n12);
-    pacc.reserve(12 * n12);
     for (int64_t n = 0; n < nn; n++) {
         for (int k = 0; k < 3; k++) {
             vel[k * nn + n] = vel0 ? vel0[n * 3 + k] : 0.0;
@@ -790,9 +806,9 @@ int eqd_commit(eqd_handle *h)
 
     // regular class SoA
     {
-        std::vector<int32_t> r_ien(8 * nr);
-        std::vector<double> r_shp(24 * nr), r_det(nr), r_lam(nr), r_mu(nr), r_vp(nr), r_rho(nr), r_st(nst * nr),
-            r_ss(6 * nr), r_phi(32 * nr), r_em(mass_term ? 24 * nr : 0), r_porep(nr), r_pstrain(nr);
+        Raw<int32_t> r_ien(8 * nr);
+        Raw<double> r_shp(24 * nr), r_det(nr), r_lam(nr), r_mu(nr), r_vp(nr), r_rho(nr), r_st(nst * nr), r_ss(6 * nr),
+            r_phi(32 * nr), r_em(mass_term ? 24 * nr : 0), r_porep(nr), r_pstrain(nr);
         std::vector<uint8_t> r_q(s.C_Q == 1 ? nr : 0);
         int qbad = 0;
 #pragma omp parallel for schedule(static) reduction(max : qbad)
@@ -862,7 +878,7 @@ int eqd_commit(eqd_handle *h)
         if ((rc = dupload(h, &d_pstrain, r_pstrain))) return rc;
         auto fill = [&](auto &E) -> int {
             using R = std::remove_pointer_t<decltype(E.ef)>;
-            auto up = [&](const R **dst, const std::vector<double> &src, int w) -> int {
+            auto up = [&](const R **dst, const Raw<double> &src, int w) -> int {
                 R *p;
                 int r2 = dupload(h, &p, to_blocks<R>(src, nr, w));
                 *dst = p;
@@ -917,9 +933,9 @@ int eqd_commit(eqd_handle *h)
     }
     // PML class SoA
     {
-        std::vector<int32_t> p_ien(8 * np);
-        std::vector<double> p_shp(24 * np), p_det(np), p_lam(np), p_mu(np), p_vp(np), p_rho(np), p_st(21 * np),
-            p_ss(6 * np), p_phi(32 * np), p_em(mass_term ? 24 * np : 0), p_damp(3 * np);
+        Raw<int32_t> p_ien(8 * np);
+        Raw<double> p_shp(24 * np), p_det(np), p_lam(np), p_mu(np), p_vp(np), p_rho(np), p_st(21 * np), p_ss(6 * np),
+            p_phi(32 * np), p_em(mass_term ? 24 * np : 0), p_damp(3 * np);
         std::vector<uint8_t> p_mask(np);
 #pragma omp parallel for schedule(static)
         for (int64_t p = 0; p < np; p++) {
@@ -956,7 +972,7 @@ int eqd_commit(eqd_handle *h)
         if ((rc = dupload(h, &pm, p_mask))) return rc;
         auto fillp = [&](auto &P) -> int {
             using R = std::remove_pointer_t<decltype(P.ef)>;
-            auto up = [&](const R **dst, const std::vector<double> &src, int w) -> int {
+            auto up = [&](const R **dst, const Raw<double> &src, int w) -> int {
                 R *q;
                 int r2 = dupload(h, &q, to_blocks<R>(src, np, w));
                 *dst = q;
