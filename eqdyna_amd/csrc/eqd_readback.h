@@ -19,8 +19,8 @@ namespace eqd {
 constexpr size_t kStageSlot = (size_t)8 << 20;
 constexpr int kStageSlots = 2, kStageLeases = 4;
 
-// Users of the staging slots (handles, start-up calls): the slots are given
-// back when the last user goes.
+// Users of the staging slots (handles, start-up calls): the slots, and the
+// threads that empty them, are given back when the last user goes.
 void stage_retain();
 void stage_release();
 

@@ -4,11 +4,16 @@
 #include "eqd_readback.h"
 
 #include <omp.h>
+#include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
+#include <new>
+#include <thread>
+#include <vector>
 
 namespace eqd {
 namespace {
@@ -69,8 +74,110 @@ __global__ void __launch_bounds__(256) pack_fric_kernel(const double *__restrict
 
 // ---------------- staging slots
 
+// From a slot into the caller's memory, which is often not yet backed by
+// pages: a few threads share the page faults (83 MB into new memory: 19 ms
+// with one thread, 5.4 with four, 3.5 with eight, 2.5 with sixteen).  They
+// belong to the lease and sleep between calls.  An OpenMP team spins on for
+// 200 ms after its last loop and slows what the caller does next (the inputs
+// and the commit of the next scenario, 161,500 elements: 202 -> 229 ms); threads
+// made in each call cost it 0.05 to 0.14 ms, waking these 0.02 (8 MB: 0.36, 0.25;
+// an OpenMP team still spinning 0.23).
+class Crew {
+   public:
+    Crew() : pid_(getpid())
+    {
+        try {
+            for (int k = std::min(8, omp_get_max_threads()) - 1; k > 0; k--) helpers_.emplace_back([this] { help(); });
+        } catch (...) {  // as many as there are
+        }
+    }
+    ~Crew()
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            stop_ = true;
+        }
+        wake_.notify_all();
+        for (std::thread &t : helpers_) t.join();
+    }
+    bool here() const { return pid_ == getpid(); }  // not in a child of the process that made it
+    // a call begins: the helpers wake while its first slot is being filled
+    void begin()
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            active_.store(true, std::memory_order_relaxed);
+        }
+        wake_.notify_all();
+    }
+    void end() { active_.store(false, std::memory_order_relaxed); }
+    // The caller copies too and waits for pieces, not for helpers: one that
+    // wakes late, or not at all, costs nothing.
+    void copy(char *dst, const char *src, size_t bytes)
+    {
+        if (bytes <= kCrewMin) {
+            memcpy(dst, src, bytes);
+            return;
+        }
+        const uint64_t pieces = (bytes + kPiece - 1) / kPiece, job = ++jobs_ << 32;
+        dst_ = dst;
+        src_ = src;
+        bytes_ = bytes;
+        done_.store(0, std::memory_order_relaxed);
+        next_.store(job, std::memory_order_release);
+        limit_.store(job | pieces, std::memory_order_release);
+        while (piece()) {}
+        for (int k = 0; done_.load(std::memory_order_acquire) != pieces; k++)
+            if (k >= 100) std::this_thread::yield();
+    }
+    static constexpr size_t kPiece = (size_t)1 << 20, kCrewMin = 2 * kPiece;
+
+   private:
+    const pid_t pid_;
+    std::mutex mu_;
+    std::condition_variable wake_;
+    bool stop_ = false;
+    std::atomic<bool> active_{false};
+    // the job's number above, the next piece or the number of pieces below
+    std::atomic<uint64_t> next_{0}, limit_{0}, done_{0};
+    uint64_t jobs_ = 0;
+    char *dst_ = nullptr;
+    const char *src_ = nullptr;
+    size_t bytes_ = 0;
+    std::vector<std::thread> helpers_;
+
+    // Copy one piece; false when there is none.  A piece that was taken is of the
+    // current job, since a job ends only when all its pieces are copied.
+    bool piece()
+    {
+        uint64_t at = next_.load(std::memory_order_acquire);
+        for (;;) {
+            const uint64_t end = limit_.load(std::memory_order_acquire);
+            if (at >> 32 != end >> 32 || at >= end) return false;
+            if (next_.compare_exchange_weak(at, at + 1, std::memory_order_acq_rel, std::memory_order_acquire)) break;
+        }
+        const size_t b = (size_t)(at & 0xFFFFFFFFu) * kPiece;
+        memcpy(dst_ + b, src_ + b, std::min(kPiece, bytes_ - b));
+        done_.fetch_add(1, std::memory_order_release);
+        return true;
+    }
+    void help()
+    {
+        for (;;) {
+            for (int k = 0; active_.load(std::memory_order_relaxed); k++) {
+                if (piece()) k = 0;
+                else if (k >= 100) std::this_thread::yield();
+            }
+            std::unique_lock<std::mutex> lk(mu_);
+            wake_.wait(lk, [this] { return stop_ || active_.load(std::memory_order_relaxed); });
+            if (stop_) return;
+        }
+    }
+};
+
 struct Lease {
     void *slot[kStageSlots] = {};
+    Crew *crew = nullptr;
     bool busy = false;
 };
 
@@ -101,6 +208,8 @@ void drop(Lease &l)
         if (p) (void)hipHostFree(p);
         p = nullptr;
     }
+    if (l.crew && l.crew->here()) delete l.crew;
+    l.crew = nullptr;
 }
 
 void give(Lease *l)
@@ -109,25 +218,6 @@ void give(Lease *l)
     l->busy = false;
     if (g_users == 0) drop(*l);
     g_free.notify_one();
-}
-
-// from the slot into the caller's memory, which is often not yet backed by
-// pages: a few threads share the page faults (83 MB into new memory: 19 ms
-// with one thread, 5.4 with four, 3.5 with eight, 2.5 with sixteen)
-void empty_slot(char *dst, const char *src, size_t bytes)
-{
-    constexpr size_t kPiece = (size_t)1 << 20;
-    if (bytes <= 2 * kPiece) {
-        memcpy(dst, src, bytes);
-        return;
-    }
-    const int64_t pieces = (int64_t)((bytes + kPiece - 1) / kPiece);
-    const int threads = std::min<int>(8, omp_get_max_threads());
-#pragma omp parallel for schedule(static) num_threads(threads)
-    for (int64_t p = 0; p < pieces; p++) {
-        const size_t b = (size_t)p * kPiece;
-        memcpy(dst + b, src + b, std::min(kPiece, bytes - b));
-    }
 }
 
 }  // namespace
@@ -152,6 +242,10 @@ hipError_t stage_out(void *out, size_t bytes, size_t unit, hipStream_t s, const 
     if (unit == 0 || unit > kStageSlot) return hipErrorInvalidValue;
     const size_t step = kStageSlot / unit * unit;
     Lease *l = take();
+    if (bytes > Crew::kCrewMin) {
+        if (!l->crew) l->crew = new (std::nothrow) Crew();
+        if (l->crew) l->crew->begin();
+    }
     hipEvent_t ev[kStageSlots] = {};
     hipError_t rc = hipSuccess;
     auto start = [&](size_t first) {  // fill the slot of the piece at `first`
@@ -169,8 +263,12 @@ hipError_t stage_out(void *out, size_t bytes, size_t unit, hipStream_t s, const 
         if (b + step < bytes) start(b + step);
         const hipError_t w = bytes > step ? hipEventSynchronize(ev[k]) : hipStreamSynchronize(s);
         if (rc == hipSuccess) rc = w;
-        if (rc == hipSuccess) empty_slot((char *)out + b, (const char *)l->slot[k], std::min(step, bytes - b));
+        if (rc != hipSuccess) break;
+        char *dst = (char *)out + b;
+        if (l->crew) l->crew->copy(dst, (const char *)l->slot[k], std::min(step, bytes - b));
+        else memcpy(dst, l->slot[k], std::min(step, bytes - b));
     }
+    if (l->crew) l->crew->end();
     if (rc != hipSuccess) (void)hipStreamSynchronize(s);  // nothing writes a slot that is given back
     for (hipEvent_t e : ev)
         if (e) (void)hipEventDestroy(e);

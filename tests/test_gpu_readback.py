@@ -55,3 +55,21 @@ def test_readback_is_the_committed_state(nx, ny, nz, pieces, precision):
     assert np.array_equal(got["dispArr"], disp)
     assert np.array_equal(got["fric"], b["fric"])
     assert np.array_equal(got["fnft"], b["fnft"])
+
+
+@pytest.mark.gpu
+def test_no_thread_is_busy_after_a_readback():
+    # the threads that empty the staging slots end with the call: what the
+    # caller does next has the cores to itself
+    import time
+    b, sc = scenario(69, 30, 75, seed=1)
+    s = Solver(b, sc, "fp32")
+    time.sleep(0.5)  # (the commit's own threads come to rest)
+    for k in ("velArr", "dispArr"):
+        s.get(k)
+    cpu = time.process_time()
+    time.sleep(0.1)
+    cpu = time.process_time() - cpu
+    s.close()
+    print(f"CPU time within 0.1 s after reading back: {cpu:.3f} s", flush=True)
+    assert cpu <= 0.05  # half a core; a spinning team takes 0.7
