@@ -173,7 +173,7 @@ void free_tables(eqd_engine *e)
 // law, FP32) 52.6 -> 28.9, 69,000 (rough fault, FP64) 85 -> 51, 161,000 (dipping
 // fault) 92.6 -> 70.9.  Element classes are merged where neither runs in tiles,
 // up to kMergeElems elements.  Nodes and pairs are merged up to kMergeNodes of
-// them: the pairs' 256 registers leave that launch two waves a SIMD, still ahead
+// them: the pairs' 204 registers leave that launch two waves a SIMD, still ahead
 // with what tiles leave to the nodes of 432,000 elements (118.5 -> 101.9 us) and
 // of 3.1 M (1.3 M nodes and pairs: 386.0 -> 377.4); with the learned guess, whose
 // network takes 24 KB of LDS a workgroup, up to kMergeNodesLearned (200,000

@@ -665,12 +665,13 @@ __device__ __forceinline__ void node3_update(const NodeState &N, int node, const
 #ifndef EQD_PML_GEO_WAVES
 #define EQD_PML_GEO_WAVES 3
 #endif
-// Waves per SIMD the fault kernel is bounded to (1: unbounded, 256 VGPRs).
-// Bounded to 2 (28-68 bytes per lane spilled) it measured the same on the
-// 64-scenario ensemble (12.90 against 12.88 ms per step, ~9,650 fault waves)
-// and on the rough-fault box (0.552 against 0.550 ms): the pairs' kernel runs
-// beside the node kernels and fills the slots they leave, so its occupancy is
-// not what bounds the step.
+// Waves per SIMD the fault kernel is bounded to (1: unbounded, 204 VGPRs and two
+// waves; with the learned guess 256 and 82 accumulation registers, one).  While
+// it took 256 registers without the guess too, a bound of 2 (28-68 bytes per lane
+// spilled) measured the same on the 64-scenario ensemble (12.90 against 12.88 ms
+// per step, ~9,650 fault waves) and on the rough-fault box (0.552 against 0.550
+// ms): the pairs' kernel runs beside the node kernels and fills the slots they
+// leave, so its occupancy is not what bounds the step.
 #ifndef EQD_FAULT_WAVES
 #define EQD_FAULT_WAVES 1
 #endif
@@ -2692,8 +2693,8 @@ __global__ void __launch_bounds__(128, EQD_FAULT_WAVES) fault_kernel(const Membe
 // The fault pairs, the PML nodes and the 3-component nodes in one launch, up to
 // the sizes of step_merged (kMergeNodes, kMergeNodesLearned): blocks of pairs
 // (the longest) first, then nfault .. of PML nodes, then npml .. of the others.
-// The pairs' 256 registers leave all of them two waves a SIMD.  Measured at both
-// ends: 2,800 elements in two launches a step instead of five 44.2 -> 20.5 us,
+// The pairs' 204 registers leave all of them two waves a SIMD, the learned
+// guess's 338 one.  Measured at both ends: 2,800 elements in two launches a step instead of five 44.2 -> 20.5 us,
 // 1.3 M nodes and pairs 386.0 -> 377.4; with the learned guess 200,000 elements
 // 88.3 -> 67.2, and at 1.4 M nodes and pairs, past its line, 451.0 -> 476.6.
 template <typename R, bool kLearn>

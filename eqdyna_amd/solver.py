@@ -358,7 +358,7 @@ class Solver:
         return json.loads(buf.value.decode())
 
     def set_graph(self, on: bool) -> None:
-        """True: capture one step as a HIP graph and replay it in run(); False
+        """True: capture steps as HIP graphs and replay them in run(); False
         (the default): launch every step."""
         self._check(self.L.eqd_set_graph(self.h, 1 if on else 0))
 

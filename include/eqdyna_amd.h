@@ -352,10 +352,10 @@ int eqd_get_launch(eqd_handle *h, int32_t kind, int32_t *block, int32_t *remap);
  * candidates) into report[report_cap]. */
 int eqd_tune(eqd_handle *h, int32_t steps, char *report, int64_t report_cap);
 
-/* on = 1: eqd_run captures one step as a HIP graph (once) and replays it;
- * on = 0 (the default): eqd_run launches every step's kernels, which measured
- * faster on this ROCm for one scenario (432,000 hexahedra: 0.094 against
- * 0.105 ms per FP32 step; 3.46 M hexahedra: 0.491 against 0.502 ms).
+/* on = 1: eqd_run captures steps as HIP graphs (one, and sixteen in a row, once)
+ * and replays them; on = 0 (the default): eqd_run launches every step's
+ * kernels.  The two are close for one scenario (432,000 hexahedra: 0.083
+ * launched and 0.081 replayed ms per FP32 step; 3.46 M: 0.441 and 0.444).
  * Per-kernel timing (eqd_set_timing) runs steps uncaptured.
  * Replayed and launched steps compute the same bits. */
 int eqd_set_graph(eqd_handle *h, int32_t on);
